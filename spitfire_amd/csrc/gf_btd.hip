@@ -15,35 +15,18 @@
 //
 // The batched flamelet solver uses a throughput form of the same recurrence (btd_inv_*): each chain is
 // eliminated from both ends at once (twisted factorisation, halving the serial chain), every Schur-updated
-// diagonal block is inverted in registers by Gauss-Jordan elimination with partial pivoting (gf_twist_impl.h)
+// diagonal block is inverted by blocked Gauss-Jordan elimination with partial pivoting on the matrix cores (gf_twist.hip)
 // and stored as its inverse, so no L blocks are stored and both sweeps of a solve are matrix-vector products.
 #include "gf_internal.h"
 #include "../../include/griffon_amd.h"
 #include "gf_wave.h"
-#include "gf_twist.h"
 
-#include <atomic>
-#include <type_traits>
-#include <utility>
 
 namespace gfa {
 
 namespace {
 
 using wave::lane_value;
-
-// Compute units of the current device, looked up once per device.
-int compute_units() {
-  static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cache[dev].load(std::memory_order_relaxed);
-  if (n <= 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cache[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
 
 constexpr int BW = 64;
 constexpr int BT_THREADS = 256;
@@ -408,32 +391,6 @@ int launch_btd_solve_t(int nsys, const int *nblocks, int bs, const double *value
 }
 
 template <typename T>
-using TwistFactorFn = void (*)(int, const int *, const double *, const long *, T *, const long *, bool,
-                               hipStream_t);
-
-template <typename T, int... I>
-constexpr TwistFactorFn<T> twist_factor_table_entry(int bs, std::integer_sequence<int, I...>) {
-  constexpr TwistFactorFn<T> tab[] = {&launch_twist_factor<T, I + 1>...};
-  return tab[bs - 1];
-}
-
-template <typename T>
-int launch_btd_inv_factor(int nsys, const int *nblocks, int bs, const double *values, const long *voff, T *dinv,
-                          const long *doff, hipStream_t st) {
-  if (nsys <= 0) return GF_OK;
-  if (bs < 1 || bs > 64) return fail(GF_ERR_UNSUPPORTED, "block size must be in 1..64");
-  // Two waves per chain shorten every pivot step, but their barriers cost issue slots: measured on 53x53
-  // blocks, the split kernel wins up to 512 systems (chains of 62..254 blocks: 7.5 against 11.2 ms) and loses
-  // from 1024 systems on (single blocks: 0.105 against 0.057 ms; chains: 13.2 against 11.9 ms), i.e. once
-  // the systems alone give every SIMD (four per compute unit) a chain.
-  const bool split = nsys < 4 * compute_units();
-  twist_factor_table_entry<T>(bs, std::make_integer_sequence<int, 64>{})(nsys, nblocks, values, voff, dinv, doff,
-                                                                          split, st);
-  if (hipGetLastError() != hipSuccess) return fail(GF_ERR_HIP, "btd inverse factor launch failed");
-  return GF_OK;
-}
-
-template <typename T>
 int launch_btd_inv_solve(int nsys, const int *nblocks, int bs, const double *values, const long *voff,
                          const T *dinv, const long *doff, const double *rhs, double *x, const long *xoff,
                          hipStream_t st) {
@@ -445,10 +402,6 @@ int launch_btd_inv_solve(int nsys, const int *nblocks, int bs, const double *val
   return GF_OK;
 }
 
-template int launch_btd_inv_factor<double>(int, const int *, int, const double *, const long *, double *, const long *,
-                                           hipStream_t);
-template int launch_btd_inv_factor<float>(int, const int *, int, const double *, const long *, float *, const long *,
-                                          hipStream_t);
 template int launch_btd_inv_solve<double>(int, const int *, int, const double *, const long *, const double *,
                                           const long *, const double *, double *, const long *, hipStream_t);
 template int launch_btd_inv_solve<float>(int, const int *, int, const double *, const long *, const float *,

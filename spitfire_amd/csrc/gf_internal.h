@@ -281,6 +281,10 @@ int launch_btd_factor_t(int nsys, const int *nblocks, int bs, double *values, co
 template <typename T>
 int launch_btd_inv_factor(int nsys, const int *nblocks, int bs, const double *values, const long *voff, T *dinv,
                           const long *doff, hipStream_t st);
+constexpr int kSmallFactor = 11;  // largest block of the one-wave-per-chain factor (gf_twist_small.hip)
+template <typename T>
+int launch_btd_inv_factor_small(int nsys, const int *nblocks, int bs, const double *values, const long *voff, T *dinv,
+                                const long *doff, hipStream_t st);
 template <typename T>
 int launch_btd_inv_solve(int nsys, const int *nblocks, int bs, const double *values, const long *voff,
                          const T *dinv, const long *doff, const double *rhs, double *x, const long *xoff,

@@ -1,0 +1,76 @@
+"""The batched inverse factor at the edges of its tiles, panels and workgroup pairs (GPU)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _recurrence(V, lo, up):
+    """inverse diagonal blocks of the elimination from both ends towards the middle block, in FP64 (NumPy)"""
+    n = len(V)
+    m = (n - 1) // 2
+    inv = [None] * n
+    for i in list(range(m)) + list(range(n - 1, m, -1)) + [m]:
+        M = V[i].copy()
+        if 0 < i <= m:
+            M -= lo[i - 1][:, None] * inv[i - 1] * up[i - 1][None, :]
+        if m <= i < n - 1:
+            M -= up[i][:, None] * inv[i + 1] * lo[i][None, :]
+        inv[i] = np.linalg.inv(M)
+    return inv
+
+
+def _factor(sizes, bs, values, precision):
+    import torch
+    from spitfire_amd import _native
+    dev = torch.device('cuda:0')
+    nb = np.asarray(sizes)
+    voff = np.cumsum([0] + [v.size for v in values])[:-1].astype(np.int64)
+    doff = np.cumsum(np.r_[0, nb * bs * bs])[:-1].astype(np.int64)
+    V = torch.tensor(np.concatenate(values), device=dev)
+    D = torch.zeros(int((nb * bs * bs).sum()), device=dev,
+                    dtype=torch.float64 if precision == 64 else torch.float32)
+    t = [torch.tensor(a, device=dev) for a in (nb.astype(np.int32), voff, doff)]
+    _native.check(_native.lib().gf_batch_btddod_inverse_factorize(
+        len(sizes), t[0].data_ptr(), bs, V.data_ptr(), t[1].data_ptr(), D.data_ptr(), t[2].data_ptr(), precision,
+        torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    d = D.cpu().numpy().astype(np.float64)
+    return [d[doff[s]:doff[s] + nb[s] * bs * bs].reshape(nb[s], bs, bs).transpose(0, 2, 1) for s in range(len(sizes))]
+
+
+@pytest.mark.parametrize('precision', [64, 32])
+@pytest.mark.parametrize('bs', [7, 8, 9, 15, 16, 17, 32, 33, 47, 48, 49, 56, 57, 63, 64])
+def test_inverse_factor_tile_edges(bs, precision):
+    """Block sizes around the panels of 8 and tiles of 16; 515 systems, so that one-block systems share workgroups
+    (two that are 256 apart), some with a longer system in the partner's place and the last ones without a
+    partner. Rows are scaled and permuted so that every pivot exchanges rows. Tolerance: growth of at most 4 (diagonal
+    weights) times N eps cond, cond <= 100 for these blocks after row scaling."""
+    rng = np.random.default_rng(bs)
+    sizes = [1] * 515
+    sizes[3], sizes[260], sizes[270], sizes[514] = 2, 3, 4, 5
+    values, parts = [], []
+    for n in sizes:
+        V = rng.standard_normal((n, bs, bs)) + (4. + 2. * np.sqrt(bs)) * np.eye(bs)
+        V = V[:, rng.permutation(bs)] * 10. ** rng.uniform(-1., 1., (n, bs, 1))
+        lo, up = 0.1 * rng.standard_normal((n - 1, bs)), 0.1 * rng.standard_normal((n - 1, bs))
+        parts.append((V, lo, up))
+        values.append(np.concatenate([V.transpose(0, 2, 1).ravel(), lo.ravel(), up.ravel()]))
+    got = _factor(sizes, bs, values, precision)
+    tol = 4. * bs * 100. * (2.2e-16 if precision == 64 else 6.0e-8)
+    for s in list(range(0, 515, 37)) + [3, 4, 259, 260, 14, 270, 256, 513, 514]:
+        for a, b in zip(got[s], _recurrence(*parts[s])):
+            assert np.max(np.abs(a - b)) <= tol * np.max(np.abs(b))
+
+
+@pytest.mark.parametrize('bs', [10, 53])
+def test_inverse_factor_of_singular_and_nonfinite_blocks(bs):
+    """A zero block and a block with a NaN give no finite inverse, and leave the other systems alone."""
+    rng = np.random.default_rng(1)
+    blocks = [rng.standard_normal((1, bs, bs)) + 20. * np.eye(bs) for _ in range(4)]
+    blocks[1] = np.zeros((1, bs, bs))
+    blocks[2][0, bs // 2, 1] = np.nan
+    got = _factor([1] * 4, bs, [b.transpose(0, 2, 1).ravel() for b in blocks], 64)
+    assert not np.isfinite(got[1]).any() and not np.isfinite(got[2]).all()
+    for s in (0, 3):
+        assert np.max(np.abs(got[s][0] @ blocks[s][0] - np.eye(bs))) <= 1e-12
