@@ -241,12 +241,6 @@ int gf_batch_btddod_inverse_solve(int nsys, const int *nblocks, int bs, const do
                                   const void *dinv, const long *doff, int precision, const double *rhs, double *x,
                                   const long *xoff, void *stream);
 
-/* Inverses of nblk independent dense blocks (no counterpart in the reference; the Newton and adjoint matrices of a
- * reactor batch): column-major n x n blocks one after another in values (left unmodified) and inv, 1 <= n <= 64,
- * Gauss-Jordan elimination with partial pivoting in FP64. Device pointers, stream-ordered. A solve is
- * gf_batch_btddod_inverse_solve with one block per system. */
-int gf_batch_block_inverse(int nblk, int n, const double *values, double *inv, void *stream);
-
 /* ---------------- many steady flamelets at once, device-resident ------------------------------------ */
 /* A batch of adiabatic flamelets sharing one mechanism and pressure, solved together on the GPU by the
  * reference's steady solvers: Newton's method (Flamelet.steady_solve_newton, flamelet.py:1352-1485) and

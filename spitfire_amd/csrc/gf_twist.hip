@@ -9,33 +9,36 @@
 // is the reference's forward block Thomas recurrence (btddod_matrix_kernels.cpp:19-80); the bottom half running
 // at the same time halves the serial chain.
 //
-// Inverse of one block: blocked in-place Gauss-Jordan elimination with partial (row) pivoting, eight pivot columns
-// (a panel) at a time, on the matrix cores. What bounds it is the serial chain of pivots, so the work between two
+// Inverse of one block: in-place Gauss-Jordan elimination with partial (row) pivoting, eight pivot columns (a panel) at a
+// time, on the matrix cores. What bounds it is the serial chain of pivots, so the work between two
 // pivots is kept small: one wave factors a panel with lane = row and the panel's eight columns in registers (a
-// pivot is a wave-wide search, a reciprocal and seven fused multiply-adds), and the rank-8 update of every
-// other column is two 16x16x4 MFMAs per 16x16 tile, spread over the chain's NT = ceil(N / 16) waves.
+// pivot is a wave-wide search, a reciprocal and at most seven fused multiply-adds), and the rank-8 update of the
+// columns is two 16x16x4 MFMAs per 16x16 tile, spread over the chain's NT = ceil(N / 16) tile waves.
 //   - Rows are never interchanged: the pivot of column k is the unused row p with the largest |entry|, and the
-//     exchange is done in place at (p, k); the permutation is undone when the inverse is written to LDS, from where
-//     the next Schur update and the store read it in order.
+//     exchange is done in place at (p, k); the order of rows and columns that this leaves is carried to the next block.
 //   - Row scaling is deferred: row r is sig_r times its stored values, sig_p = 1/d from the step that pivots it. One
 //     pivot (row p, column k, stored value d) is
-//         rows r != p:  g_r = x_r[k] / d,  x_r[c] -= g_r x_p[c] (c != k),  x_r[k] = -g_r
+//         rows r != p:  g_r = -x_r[k] / d,  x_r[c] += g_r x_p[c] (c != k),  x_r[k] = g_r
 //         row p:        x_p[k] = 1,  sig_p = 1 / d
-//   - A panel of pivots (p_j, k_j) changes every other column c by x[c] += H x_P[c], x_P the old pivot rows and H_rj the
-//     panel's own new entry x_r[k_j], less one at r = p_j (both are -A_rK A_PK^{-1} there, up to the deferred scale). The
-//     wave that factors the panel keeps its columns less that one (so that H does not lose its last digits to it) and hands
-//     back nothing else.
-// What bounds it: a panel's eight pivots take about 2,800 cycles of its wave (50 instructions a pivot at one per four
-// cycles and more, the lane shifts, scalar broadcasts and the reciprocal one after another), the hand-over to the tile
-// waves, their first two MFMAs and the way back 1,100, a block's exchange and Schur update 4,000; FP64 MFMAs run on
-// the vector FP64 units, so they do not overlap with a panel on the same SIMD. Before, every pivot was broadcast row
-// by row through scalar registers to one or two waves, with a barrier a pivot. Measured before and after (53x53, us):
+//   - A panel of pivots (p_j, k_j) adds g_rj u_j[c], j = 0 .. 7 to column c of row r, where u_j is row p_j as it is when it is
+//     pivoted: u_j[c] = x_pj[c] + g_{pj,0} u_0[c] + .. + g_{pj,j-1} u_{j-1}[c]. The panel's own columns are columns like the
+//     others, starting from g_rj (1 at row p_j), with u_i = 0 up to their own pivot.
+//   - An MFMA accumulates its four products in ascending order with one rounding each, and u_j is formed in the same
+//     order, so every entry passes through the same fused multiply-adds as in an elimination pivot by pivot: the
+//     inverses are bitwise those of gf_twist_small.hip, whatever the panel and tile sizes.
+// What bounds it: a panel's eight pivots take about 3,400 cycles of its wave (the lane shifts of the search, the scalar
+// broadcasts and the division one after another), forming the u_j, the first two MFMAs and the two hand-overs 1,900, the
+// change to the next block 2,000. FP64 MFMAs run on the vector FP64 units, so they do not overlap with a panel on the same
+// SIMD. Before, every pivot was broadcast row by row through scalar registers to one or two waves, with a barrier a
+// pivot. Measured before and after (53x53, us):
 //   systems                     FP64             FP32
-//   one chain of 126 blocks     2,248 -> 1,026   1,663 ->   732
-//   256 chains of 62..254       4,807 -> 2,090   3,547 -> 1,508
-//   512 chains                  6,455 -> 4,050   4,546 -> 2,911
-//   1,024 chains               11,555 -> 7,071   8,106 -> 5,117
-//   1,024 / 4,000 blocks       53 / 238 -> 46 / 172   45 / 155 -> 37 / 144
+//   one chain of 126 blocks     2,248 -> 1,140   1,663 ->   854
+//   256 chains of 62..254       4,807 -> 2,386   3,547 -> 1,818
+//   512 chains                  6,455 -> 4,580   4,546 -> 3,520
+//   1,024 chains               11,555 -> 8,046   8,106 -> 6,184
+//   1,024 / 4,000 blocks       53 / 238 -> 50 / 199   45 / 155 -> 42 / 173
+// (The panel's multipliers instead of the u_j, H = -A_rK A_PK^{-1}, save the substitution, 1,026 us for the chain, but round
+// differently.)
 #include "gf_internal.h"
 #include "gf_wave.h"
 #include "../../include/griffon_amd.h"
@@ -56,142 +59,231 @@ __device__ __forceinline__ Vec4<float> mfma4(float a, float b, Vec4<float> c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Pivot search. The key of an unused row orders like |f|, up to the low bits of the mantissa that the lane number
-// replaces (14 fraction bits are compared in FP64, 17 in FP32): a pivot within 1e-4 of the largest bounds the growth as
-// well as the largest does, and one scan of 32-bit keys finds it without a second search among equal high words.
-__device__ __forceinline__ unsigned magnitude(double f) { return (unsigned)__double2hiint(f) & 0x7fffffffu; }
-__device__ __forceinline__ unsigned magnitude(float f) { return (unsigned)__float_as_int(f) & 0x7fffffffu; }
-template <typename T>
-__device__ __forceinline__ unsigned pivot_key(T f, bool used, int lane) {
-  return used ? 0u : (magnitude(f) & ~63u) | (unsigned)(63 - lane);
-}
-// step k = 0 .. 5 of the wave-wide maximum of the keys, complete in lane 63 after step 5
+// Pivot search: the first unused row with the largest |f|, on the bit patterns. A row's key is the word of its entry that
+// holds the exponent under its mask, which is 0 once the row is used.
+__device__ __forceinline__ unsigned key_of(double f, unsigned mask) { return (unsigned)__double2hiint(f) & mask; }
+__device__ __forceinline__ unsigned key_of(float f, unsigned mask) { return (unsigned)__float_as_int(f) & mask; }
+// step k = 0 .. 5 of the wave-wide maximum, complete in lane 63 after step 5
 template <int K>
 __device__ __forceinline__ unsigned max_step(unsigned v) {
   constexpr int ctrl[6] = {0x111, 0x112, 0x114, 0x118, 0x142, 0x143};  // row_shr 1, 2, 4, 8, row_bcast 15, 31
   constexpr int rows[6] = {0xF, 0xF, 0xF, 0xF, 0xA, 0xC};
   return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl[K], rows[K], 0xF, false));
 }
-__device__ __forceinline__ int pivot_of(unsigned scanned) {
-  return 63 - (int)((unsigned)__builtin_amdgcn_readlane((int)scanned, 63) & 63u);
+template <typename T>
+__device__ __forceinline__ int pivot_of(unsigned scanned, unsigned key, T f, unsigned mask) {
+  const unsigned top = (unsigned)__builtin_amdgcn_readlane((int)scanned, 63);
+  unsigned long long hit = __ballot(key == top);
+  if constexpr (sizeof(T) == 8) {
+    if (hit & (hit - 1)) {  // rare: the low words decide (or all are zero, and used rows have that key as well)
+      const bool in = (key == top) & (mask != 0u);
+      const unsigned lo = in ? (unsigned)__double2loint(f) : 0u;
+      const unsigned most = wave::dpp_wave_max_u32(lo);
+      hit = __ballot(in & (lo == most));
+    }
+  } else {
+    if (top == 0u) hit = __ballot(mask != 0u);
+  }
+  return __builtin_ctzll(hit);
 }
 
-// 1 / x in steps that are spread between other work: the hardware reciprocal, two Newton steps (FP64), and zeros,
-// infinities and NaN as a division gives them. About half the dependent chain of the division.
+// 1 / x as a division gives it, in steps that are spread between other work.
 struct Recip64 {
-  double x, r, e;
+  double x, n, m, r, e;
+  bool flag;
   template <int K>
   __device__ __forceinline__ void step() {
-    if constexpr (K == 0) r = __builtin_amdgcn_rcp(x);
-    else if constexpr (K == 1 || K == 3) e = fma(-x, r, 1.);
-    else if constexpr (K == 2 || K == 4) r = fma(r, e, r);
-    else r = __builtin_amdgcn_div_fixup(r, x, 1.);
+    if constexpr (K == 0) {
+      bool unused;
+      n = __builtin_amdgcn_div_scale(1., x, false, &unused);
+      m = __builtin_amdgcn_div_scale(1., x, true, &flag);
+      r = __builtin_amdgcn_rcp(n);
+    } else if constexpr (K == 1 || K == 3) e = fma(-n, r, 1.);
+    else if constexpr (K == 2) r = fma(r, e, r);
+    else if constexpr (K == 4) {
+      r = fma(r, e, r);
+      e = m * r;
+    } else if constexpr (K == 5) m = fma(-n, e, m);
+    else r = __builtin_amdgcn_div_fixup(__builtin_amdgcn_div_fmas(m, r, e, flag), x, 1.);
   }
 };
 struct Recip32 {
-  float x, r;
+  float x, n, m, r, e, q;
+  bool flag;
   template <int K>
   __device__ __forceinline__ void step() {
-    if constexpr (K == 0) r = 1.f / x;
+    if constexpr (K == 0) {
+      bool unused;
+      n = __builtin_amdgcn_div_scalef(1.f, x, false, &unused);
+      m = __builtin_amdgcn_div_scalef(1.f, x, true, &flag);
+      r = __builtin_amdgcn_rcpf(n);
+    } else if constexpr (K == 1) e = fmaf(-n, r, 1.f);
+    else if constexpr (K == 2) {
+      r = fmaf(e, r, r);
+      q = m * r;
+    } else if constexpr (K == 3) e = fmaf(-n, q, m);
+    else if constexpr (K == 4) q = fmaf(e, r, q);
+    else if constexpr (K == 5) e = fmaf(-n, q, m);
+    else r = __builtin_amdgcn_div_fixupf(__builtin_amdgcn_div_fmasf(e, r, q, flag), x, 1.f);
   }
 };
-__device__ __forceinline__ Recip64 recip_of(double x) { return Recip64{x, 0., 0.}; }
-__device__ __forceinline__ Recip32 recip_of(float x) { return Recip32{x, 0.f}; }
+__device__ __forceinline__ Recip64 recip_of(double x) { return Recip64{x}; }
+__device__ __forceinline__ Recip32 recip_of(float x) { return Recip32{x}; }
 
 // One chain's LDS. Rows and columns are padded to Np = 8 ceil(N / 8) by an identity, so that every panel is full: the
-// padding's pivots are its own ones. M holds the block before each panel's update, a row as [lane group][tile][register]
-// (the pivot rows are read from it), and between two blocks the inverse, column-major with stride IS.
+// padding's pivots are its own ones. Two more arrays are in dynamic LDS: M, the block before each panel's update, a row as
+// [lane group][tile][register] (the pivot rows are read from it), and V, the values of the chain's next block, column-major
+// with one row and one column of zeros, which stand for the padding.
 template <typename T, int NT>
 struct ChainLds {
   static constexpr int R = 16 * NT;
-  static constexpr int GS = 4 * NT + 2;  // stride of a lane group, and MS of a row: they spread the banks
+  static constexpr int GS = 4 * NT;      // stride of a lane group, and MS of a row, which spreads the banks
   static constexpr int MS = 4 * GS + 2;
-  static constexpr int IS = R + 2;
-  static constexpr int PS = 10;  // stride of a row of P: spreads the rows over the banks
-  alignas(16) T P[R][PS];  // the panel's columns before its elimination, then H: [row][column]
-  T sig[R];         // scale of each row: the reciprocal of its pivot
-  double cs[4][4 * NT + 1];  // column scales of the next Schur update, column 16 t + 4 k + g at [g][4 t + k]
-  int rowj[R];      // which of the panel's pivots a row is, -1 if none
-  int prow[R];      // pivot row of each column
-  static __host__ __device__ constexpr int words(int np) {  // of M: np rows and one that takes the rows beyond
-    return (np + 1) * MS > R * IS ? (np + 1) * MS : R * IS;
-  }
+  static constexpr int PS = 10;  // stride of a row of P and G: spreads the rows over the banks
+  static constexpr int CS = 4 * NT + 2;
+  alignas(16) T P[R][PS];  // the panel's columns before its elimination: [row][column]
+  alignas(16) T G[R][PS];  // multipliers of the panel's pivots: [row][pivot]
+  double cs[4][CS];        // column scales of the next Schur update, column 16 t + 4 k + g at [g][4 t + k]
+  double rs[R];            // its row scales
+  T sig[R];                // scale of each row: the reciprocal of its pivot
+  alignas(16) int prow[R];  // pivot row of each column
+  int rowid[R];            // the row and the column of the inverse that a row and a column hold, N for padding
+  alignas(16) int colid[4][CS + 2];
+  static __host__ __device__ constexpr int m_words(int np) { return (np + 1) * MS; }  // a row more, for those beyond
+  static __host__ __device__ constexpr int v_words(int n) { return (n + 1) * n + 1; }
 };
 
-// The wave that factors a chain's panels, lane = row. Per panel: eight pivots, each found among the unused rows,
-//   h_r = -x_r[k] / d (0 at the pivot row),  x_r[c] += h_r x_p[c] for the panel's other columns,  H_r[k] = h_r.
-// Only the panel's columns are touched here. A single wave issues at most one instruction every four cycles and the
+// The wave that factors a chain's panels, lane = row. Per panel: eight pivots, each found among the unused rows, the
+// multipliers g_r = -x_r[k] / d (0 at the pivot row), and x_r[c] += g_r x_p[c] for the panel's later columns c. Only these
+// are touched here. A single wave issues at most one instruction every four cycles and the
 // search of the next pivot is a chain of dependent lane shifts, so a step updates the next pivot's column first
-// and then does one lane shift, one step of the next reciprocal and one of the six other columns at a time, in an
+// and then does one lane shift, one step of the next reciprocal and one of the other columns at a time, in an
 // order that the compiler's scheduler (which otherwise runs the chains one after the other) has to keep.
+// The padding is not pivoted. Returns the pivot column of the lane's row.
+template <bool PART, typename T>
+__device__ __forceinline__ void panel_pivots(T (&f)[8], T (&g)[8], unsigned &mask, T &sig, int &rj, int left, int lane) {
+  unsigned key = key_of(f[0], mask), most = key;
+  auto rc = recip_of(f[0]);
+  most = max_step<0>(most); rc.template step<0>();
+  most = max_step<1>(most); rc.template step<1>();
+  most = max_step<2>(most); rc.template step<2>();
+  most = max_step<3>(most); rc.template step<3>();
+  most = max_step<4>(most); rc.template step<4>();
+  most = max_step<5>(most); rc.template step<5>();
+  rc.template step<6>();
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    if (PART && j > 0 && left <= j) {
+      g[j] = T(0);
+      continue;
+    }
+    const int p = pivot_of(most, key, f[j], mask);  // left - j unused rows remain
+    const bool isp = lane == p;
+    T h = f[j] * -lane_value(rc.r, p);
+    asm("" : "+v"(h));  // (a select, not a branch around the product)
+    h = isp ? T(-0.) : h;
+    g[j] = h;
+    auto update = [&](int c) {
+      if (c < 8) f[c] = fma(h, lane_value(f[c], p), f[c]);
+    };
+    mask = isp ? 0u : mask;
+    rj = isp ? j : rj;
+    sig = isp ? rc.r : sig;
+    if (j < 7) {
+      update(j + 1);
+      most = key = key_of(f[(j + 1) & 7], mask);
+      rc = recip_of(f[(j + 1) & 7]);
+      rc.template step<0>();
+      __builtin_amdgcn_sched_barrier(0);
+      most = max_step<0>(most); rc.template step<1>(); update(j + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      most = max_step<1>(most); rc.template step<2>(); update(j + 3);
+      __builtin_amdgcn_sched_barrier(0);
+      most = max_step<2>(most); rc.template step<3>(); update(j + 4);
+      __builtin_amdgcn_sched_barrier(0);
+      most = max_step<3>(most); rc.template step<4>(); update(j + 5);
+      __builtin_amdgcn_sched_barrier(0);
+      most = max_step<4>(most); rc.template step<5>(); update(j + 6);
+      __builtin_amdgcn_sched_barrier(0);
+      most = max_step<5>(most); rc.template step<6>(); update(j + 7);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
 template <typename T, int NT>
-__device__ __forceinline__ void factor_panels(ChainLds<T, NT> &s, int Np, int lane) {
+__device__ __forceinline__ int factor_panels(ChainLds<T, NT> &s, int N, int Np, int lane) {
   const int row = NT == 4 || lane < 16 * NT ? lane : 0;
-  bool used = lane >= Np;
+  unsigned mask = lane < N ? 0x7fffffffu : 0u;
   T sig = T(1);
+  int kap = lane;
   for (int base = 0; base < Np; base += 8) {
     __syncthreads();
-    T f[8];
+    T f[8], g[8];
     typedef T V2 __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int j = 0; j < 8; j += 2) {
-      const V2 g = *reinterpret_cast<const V2 *>(&s.P[row][j]);
-      f[j] = g[0];
-      f[j + 1] = g[1];
+      const V2 v = *reinterpret_cast<const V2 *>(&s.P[row][j]);
+      f[j] = v[0];
+      f[j + 1] = v[1];
     }
     int rj = -1;
-    unsigned key = pivot_key(f[0], used, lane);
-    auto rc = recip_of(f[0]);
-    key = max_step<0>(key); rc.template step<0>();
-    key = max_step<1>(key); rc.template step<1>();
-    key = max_step<2>(key); rc.template step<2>();
-    key = max_step<3>(key); rc.template step<3>();
-    key = max_step<4>(key); rc.template step<4>();
-    key = max_step<5>(key); rc.template step<5>();
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int p = pivot_of(key);  // Np - base - j unused rows remain
-      const T ip = lane_value(rc.r, p);
-      const bool isp = lane == p;
-      const T h = isp ? T(0) : -(f[j] * ip);
-      auto update = [&](int c) { f[c & 7] = fma(h, lane_value(f[c & 7], p), f[c & 7]); };
-      used = used || isp;
-      rj = isp ? j : rj;
-      sig = isp ? ip : sig;
-      if (j < 7) {
-        update(j + 1);
-        key = pivot_key(f[(j + 1) & 7], used, lane);
-        rc = recip_of(f[(j + 1) & 7]);
-        rc.template step<0>();
-        __builtin_amdgcn_sched_barrier(0);
-        key = max_step<0>(key); rc.template step<1>(); update(j + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        key = max_step<1>(key); rc.template step<2>(); update(j + 3);
-        __builtin_amdgcn_sched_barrier(0);
-        key = max_step<2>(key); rc.template step<3>(); update(j + 4);
-        __builtin_amdgcn_sched_barrier(0);
-        key = max_step<3>(key); rc.template step<4>(); update(j + 5);
-        __builtin_amdgcn_sched_barrier(0);
-        key = max_step<4>(key); rc.template step<5>(); update(j + 6);
-        __builtin_amdgcn_sched_barrier(0);
-        key = max_step<5>(key); update(j + 7);
-        f[j] = h;
-        __builtin_amdgcn_sched_barrier(0);
-      } else {
-#pragma unroll
-        for (int c = 0; c < 7; ++c) update(c);
-        f[7] = h;
-      }
-    }
+    if (base + 8 <= N) panel_pivots<false>(f, g, mask, sig, rj, 8, lane);
+    else panel_pivots<true>(f, g, mask, sig, rj, N - base, lane);
     if (NT == 4 || lane < 16 * NT) {
 #pragma unroll
-      for (int j = 0; j < 8; j += 2) *reinterpret_cast<V2 *>(&s.P[lane][j]) = V2{f[j], f[j + 1]};
-      s.rowj[lane] = rj;
+      for (int j = 0; j < 8; j += 2) *reinterpret_cast<V2 *>(&s.G[lane][j]) = V2{g[j], g[j + 1]};
       if (base + 8 == Np) s.sig[lane] = sig;
       if (rj >= 0) s.prow[base + rj] = lane;
     }
     __syncthreads();
+    kap = rj >= 0 ? base + rj : kap;
   }
+  return kap;
+}
+
+// a[i] of lane group k becomes a[k] of lane group i: the four registers' 16-lane rows transposed
+__device__ __forceinline__ void swap_halves(int &a, int &b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+__device__ __forceinline__ void swap_rows(int &a, int &b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+template <typename T>
+__device__ __forceinline__ void transpose4(T &a, T &b, T &c, T &d) {
+  constexpr int W = sizeof(T) / 4;
+  typedef int Words __attribute__((ext_vector_type(W)));
+  int v[4][W];
+  auto get = [&](int i, T x) {
+    if constexpr (W == 1) v[i][0] = __builtin_bit_cast(int, x);
+    else {
+      const Words q = __builtin_bit_cast(Words, x);
+      v[i][0] = q[0];
+      v[i][W - 1] = q[W - 1];
+    }
+  };
+  auto put = [&](int i) {
+    if constexpr (W == 1) return __builtin_bit_cast(T, v[i][0]);
+    else return __builtin_bit_cast(T, Words{v[i][0], v[i][W - 1]});
+  };
+  get(0, a); get(1, b); get(2, c); get(3, d);
+#pragma unroll
+  for (int k = 0; k < W; ++k) {
+    swap_halves(v[0][k], v[2][k]);
+    swap_halves(v[1][k], v[3][k]);
+    swap_rows(v[0][k], v[1][k]);
+    swap_rows(v[2][k], v[3][k]);
+  }
+  a = put(0); b = put(1); c = put(2); d = put(3);
+}
+// the value of lane L of each 16-lane row, in all lanes of that row
+template <int L, typename T>
+__device__ __forceinline__ T row_lane(T v) {
+  return __builtin_amdgcn_mov_dpp(v, 0x150 + L, 0xF, 0xF, true);
 }
 
 // A block row as its NT tile waves hold it: wave w has rows 16 w .. 16 w + 15 of every column. The tile of columns
@@ -201,139 +293,142 @@ template <typename T, int NT>
 struct Tiles {
   using S = ChainLds<T, NT>;
   Vec4<T> x[NT];
+  T a[2][4];  // left operands by tile: pivots 0 .. 3 and 4 .. 7 of a panel
+  T b0, b1;
 
-  // In-place elimination of all columns: afterwards element (row, column) times s.sig[row] is element (kap,
-  // s.prow[column]) of the inverse; returns kap, the pivot column of the lane's row. `idle(k)` runs while panel k = 0 or 1
-  // is factored. Of a panel's update only the tile that holds the next panel is waited for; the other tiles'
-  // MFMAs (operands a0, a1, b0, b1) and the copy to M are issued while the next panel is factored.
-  template <class F>
-  __device__ __forceinline__ int eliminate(S &s, T *M, int Np, int w, int lane, F idle) {
-    const int r16 = lane & 15, grp = lane >> 4, row = 16 * w + r16;
+  // Left operands of all tiles for the panel at `base` (lane group g: the rows of pivots g and 4 + g, as each is when it
+  // is pivoted), with lane = column of the NT tiles.
+  __device__ __forceinline__ void pivot_rows(const S &s, const T *M, int base, int N, int lane) {
+    const int n = lane & 15;
+    // lane n of each 16 holds the n-th multiplier of the pivot rows 1 .. 5, and of the rows 6 and 7
+    const int ja = n < 1 ? 1 : n < 3 ? 2 : n < 6 ? 3 : n < 10 ? 4 : 5, jb = n < 6 ? 6 : 7;
+    const int pa = s.prow[base + ja], pb = s.prow[base + jb];
+    typedef int I4 __attribute__((ext_vector_type(4)));
+    const I4 p0 = *reinterpret_cast<const I4 *>(&s.prow[base]), p1 = *reinterpret_cast<const I4 *>(&s.prow[base + 4]);
     // row i of the left operand is column 4 q + g of the tile, i = 4 q + g in an FP64 accumulator, 4 g + q in FP32
     constexpr bool f64 = sizeof(T) == 8;
-    const T *src = M + (f64 ? (r16 & 3) : (r16 >> 2)) * S::GS + (f64 ? (r16 >> 2) : (r16 & 3));
+    const int g = f64 ? (n & 3) : (n >> 2), k = f64 ? (n >> 2) : (n & 3);
+    // column c of the panel starts from its multipliers at pivot c
+    int c = (lane & 48) + 4 * k + g - base;
+    c = (unsigned)c < 8u ? c : -1;
+    asm volatile("" : "+v"(c));  // opaque: its comparisons are not kept (and spilled) over the blocks for each panel
+    const T *src = c >= 0 ? &s.G[0][c] : M + g * S::GS + 4 * min(lane >> 4, NT - 1) + k;
+    const int stride = c >= 0 ? S::PS : S::MS;
+    const T la = s.G[pa][n - ja * (ja - 1) / 2], lb = s.G[pb][n < 6 ? n : n - 6];
+    T u[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) u[j] = src[(j < 4 ? p0[j & 3] : p1[j & 3]) * stride];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) u[j] = c < j ? u[j] : T(0);
+#define GF_ROW(J, I, L, AT) u[J] = fma(row_lane<AT>(L), u[I], u[J]);
+    GF_ROW(1, 0, la, 0)
+    GF_ROW(2, 0, la, 1) GF_ROW(2, 1, la, 2)
+    GF_ROW(3, 0, la, 3) GF_ROW(3, 1, la, 4) GF_ROW(3, 2, la, 5)
+    GF_ROW(4, 0, la, 6) GF_ROW(4, 1, la, 7) GF_ROW(4, 2, la, 8) GF_ROW(4, 3, la, 9)
+    GF_ROW(5, 0, la, 10) GF_ROW(5, 1, la, 11) GF_ROW(5, 2, la, 12) GF_ROW(5, 3, la, 13) GF_ROW(5, 4, la, 14)
+    GF_ROW(6, 0, lb, 0) GF_ROW(6, 1, lb, 1) GF_ROW(6, 2, lb, 2) GF_ROW(6, 3, lb, 3) GF_ROW(6, 4, lb, 4) GF_ROW(6, 5, lb, 5)
+    GF_ROW(7, 0, lb, 6) GF_ROW(7, 1, lb, 7) GF_ROW(7, 2, lb, 8) GF_ROW(7, 3, lb, 9) GF_ROW(7, 4, lb, 10)
+    GF_ROW(7, 5, lb, 11) GF_ROW(7, 6, lb, 12)
+#undef GF_ROW
+    if (base + 8 > N) {
+#pragma unroll
+      for (int j = 1; j < 8; ++j) u[j] = base + j < N ? u[j] : T(0);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      transpose4(u[4 * h], u[4 * h + 1], u[4 * h + 2], u[4 * h + 3]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) a[h][t] = u[4 * h + t];
+    }
+  }
+
+  __device__ __forceinline__ void update(int t) { x[t] = mfma4(a[1][t], b1, mfma4(a[0][t], b0, x[t])); }
+
+  // what is left of a panel's update: every tile but the one that was waited for
+  __device__ __forceinline__ void pending(int done) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      if (t != done) update(t);
+  }
+
+  // In-place elimination of all columns. On entry tile 0 is complete, and `enter` completes the other ones
+  // while the first panel is factored; on return tile 0 is complete up to its rows' scale s.sig, and pending(0) does the
+  // others. `idle` runs while the second panel is factored (the first, if there is one tile only). Of a panel's update only
+  // the tile that holds the next panel is waited for; the other tiles' MFMAs and the copy to M are issued while the
+  // next panel is factored.
+  template <class Enter, class Idle>
+  __device__ __forceinline__ void eliminate(S &s, T *M, int N, int Np, int w, int lane, Enter enter, Idle idle) {
+    const int r16 = lane & 15, grp = lane >> 4, row = 16 * w + r16;
     T *dst = M + min(row, Np) * S::MS + grp * S::GS;
-    int kap = row;
-    T a0[NT], a1[NT], b0 = T(0), b1 = T(0), pn0 = T(0), pn1 = T(0);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) a0[t] = a1[t] = T(0);
-    auto update = [&](int t) { x[t] = mfma4(a1[t], b1, mfma4(a0[t], b0, x[t])); };
-    auto pending = [&](bool wrapped) {
-#pragma unroll
-      for (int t = 1; t < NT; ++t) update(t);
-      if (NT > 1 && wrapped) {
-        x[NT - 1][2] = pn0;
-        x[NT - 1][3] = pn1;
-      }
-    };
-    auto rotate = [&] {  // the next column tile moves to register tile 0 (back in place after NT of these)
-      const Vec4<T> x0 = x[0];
-      const T c0 = a0[0], c1 = a1[0];
-#pragma unroll
-      for (int t = 0; t + 1 < NT; ++t) {
-        x[t] = x[t + 1];
-        a0[t] = a0[t + 1];
-        a1[t] = a1[t + 1];
-      }
-      x[NT - 1] = x0;
-      a0[NT - 1] = c0;
-      a1[NT - 1] = c1;
-    };
     s.P[row][grp] = x[0][0];
     s.P[row][4 + grp] = x[0][1];
-    for (int ct = 0; ct < NT; ++ct) {
+#pragma unroll
+    for (int ct = 0; ct < NT; ++ct)
 #pragma unroll
       for (int q = 0; q < 4; q += 2) {
         const int base = 16 * ct + 4 * q;
-        if (base < Np) {
+        if (ct + 1 < NT || base < Np) {
           __syncthreads();
-          if (q > 0 || ct > 0) pending(q == 0);
+          if (q == 0 && ct == 0) enter();
+          else pending(ct);
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
             typedef T V2 __attribute__((ext_vector_type(2)));
             *reinterpret_cast<V2 *>(dst + 4 * t) = V2{x[t][0], x[t][1]};
             *reinterpret_cast<V2 *>(dst + 4 * t + 2) = V2{x[t][2], x[t][3]};
           }
-          if (ct == 0) idle(q / 2);
+          if (ct == 0 && q == (NT == 1 ? 0 : 2)) idle();
           __syncthreads();
-          const int p0 = s.prow[base + grp], p1 = s.prow[base + 4 + grp], rj = s.rowj[row];
-          b0 = s.P[row][grp];
-          b1 = s.P[row][4 + grp];
-          pn0 = b0 + (rj == grp ? T(1) : T(0));
-          pn1 = b1 + (rj == 4 + grp ? T(1) : T(0));
-          kap = rj >= 0 ? base + rj : kap;
-          const T *s0 = src + p0 * S::MS, *s1 = src + p1 * S::MS;
-          constexpr int tn = (NT > 1) ? 1 : 0;
-          const int first = q == 2 ? tn : 0;  // the tile of the next panel
-          a0[first] = s0[4 * first];
-          a1[first] = s1[4 * first];
-          update(first);
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-            if (t != first) {
-              a0[t] = s0[4 * t];
-              a1[t] = s1[4 * t];
-            }
-          if (first == 0) {
-            x[0][q] = pn0;
-            x[0][q + 1] = pn1;
+          b0 = s.G[row][grp];
+          b1 = s.G[row][4 + grp];
+          x[ct][q] = s.prow[base + grp] == row ? T(1) : b0;
+          x[ct][q + 1] = s.prow[base + 4 + grp] == row ? T(1) : b1;
+          pivot_rows(s, M, base, N, lane);
+          const bool last = ct + 1 == NT && base + 8 == Np;
+          if (last) {
+            update(0);
           } else {
-            rotate();
+            const int next = q == 2 ? (ct + 1 < NT ? ct + 1 : 0) : ct;
+            update(next);
+            s.P[row][grp] = x[next][(q + 2) & 3];
+            s.P[row][4 + grp] = x[next][((q + 2) & 3) + 1];
           }
-          s.P[row][grp] = x[0][(q + 2) & 3];
-          s.P[row][4 + grp] = x[0][((q + 2) & 3) + 1];
           __builtin_amdgcn_sched_barrier(0);  // the pending MFMAs stay behind the next panel's hand-over
         }
-      }
-    }
-    const bool wrapped = ((Np - 1) & 8) == 8;  // the last panel was its tile's last: already rotated
-    pending(wrapped);
-    if (!wrapped) rotate();
-    return kap;
-  }
-
-  // the padding's identity: ones on the diagonal beyond the block
-  __device__ __forceinline__ void pad(int N, int w, int lane) {
-    const int r16 = lane & 15, grp = lane >> 4;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-      if (t == w) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) x[t][k] = (16 * w + r16 >= N && 4 * k + grp == r16) ? T(1) : x[t][k];
       }
   }
 };
 
-// Elements (row, column) of a block in memory through a buffer descriptor of its N x N elements: those outside the block
-// read as zero and are not written, without a branch or a select per element.
+// Elements of a block in memory through a buffer descriptor of its N x N elements: those outside the block read as zero
+// and are not written, without a branch or a select per element.
 template <typename E>
 struct Window {
   __amdgpu_buffer_rsrc_t rsrc;
-  int at, step;  // byte offset of (row, group's column), bytes of one column
-  __device__ __forceinline__ Window(const E *base, int N, int row, int grp)
-      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<E *>(base), 0, N * N * (int)sizeof(E), 0x00020000)),
-        at(row < N ? (grp * N + row) * (int)sizeof(E) : (1 << 30)), step(N * (int)sizeof(E)) {}
-  __device__ __forceinline__ E load(int c) const {
-    if constexpr (sizeof(E) == 8) return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b64(rsrc, at + c * step, 0, 0));
-    else return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at + c * step, 0, 0));
+  __device__ __forceinline__ Window(const E *base, int N)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<E *>(base), 0, N * N * (int)sizeof(E), 0x00020000)) {}
+  __device__ __forceinline__ E load(int e) const {
+    if constexpr (sizeof(E) == 8) return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b64(rsrc, e * 8, 0, 0));
+    else return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b32(rsrc, e * 4, 0, 0));
   }
-  __device__ __forceinline__ void store(int c, E v) const {
+  __device__ __forceinline__ void store(int e, E v) const {
     typedef unsigned U2 __attribute__((ext_vector_type(2)));
-    if constexpr (sizeof(E) == 8) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), rsrc, at + c * step, 0, 0);
-    else __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rsrc, at + c * step, 0, 0);
+    if constexpr (sizeof(E) == 8) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), rsrc, e * 8, 0, 0);
+    else __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rsrc, e * 4, 0, 0);
   }
 };
 
 // One workgroup of 2 (NT + 1) waves per system: for the top chain NT tile waves and the wave that factors its panels, then
 // the same for the bottom chain. Both chains run max(len) inverses so that every wave passes the same barriers: the
 // shorter chain starts with one inverse of the identity, which it discards. The middle block is inverted by the top
-// chain alone, which reads the bottom chain's last inverse from LDS. While a block's first two panels are factored, the
-// tile waves store the inverse before it and load the values of the block after it.
+// chain alone, which reads the bottom chain's term from its V. A block keeps the order of rows and columns that the inverse
+// before it left (the panel wave tracks it), so the inverse never moves between lanes; the next block's values, which the
+// tile waves bring to LDS while the second panel is factored, are read in that order. Only register tile 0 of the Schur
+// update, which holds the next panel, is waited for: the others and the store follow while that panel is factored.
 template <typename T, int NT>
-__global__ void __launch_bounds__(128 * (NT + 1)) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 8 : NT == 2 ? 5 : NT == 3 ? 4 : 2)))
+__global__ void __launch_bounds__(128 * (NT + 1)) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 6 : NT == 2 ? 5 : NT == 3 ? 4 : 2)))
 twist_factor_kernel(int nsys, const int *nblocks, int n, const double *values, const long *voff, T *dinv, const long *doff) {
   using S = ChainLds<T, NT>;
-  extern __shared__ char m_raw[];
+  extern __shared__ double v_raw[];
   __shared__ S lds[2];
   // Two one-block systems share a workgroup, the second (256 further on, so that the workgroups that are left without
   // work are spread evenly over the XCDs and compute units) in the bottom chain's place.
@@ -349,8 +444,9 @@ twist_factor_kernel(int nsys, const int *nblocks, int n, const double *values, c
   S &s = lds[top ? 0 : 1];
   int N = n;
   const int Np = (n + 7) & ~7;
-  T *M = reinterpret_cast<T *>(m_raw) + (top ? 0 : S::words(Np));
-  const T *E = reinterpret_cast<const T *>(m_raw) + S::words(Np);  // the bottom chain's inverse
+  double *Vb = v_raw + S::v_words(n);  // the bottom chain's
+  double *Vl = top ? v_raw : Vb;
+  T *M = reinterpret_cast<T *>(v_raw + ((2 * S::v_words(n) + 1) & ~1)) + (top ? 0 : S::m_words(Np));
   const long NB2 = (long)n * n;
   const int nb = __builtin_amdgcn_readfirstlane(nblocks[sys]);
   const int m = (nb - 1) / 2;
@@ -360,25 +456,37 @@ twist_factor_kernel(int nsys, const int *nblocks, int n, const double *values, c
   T *Dg = dinv + doff[sys];
   const int len = top ? m : nb - 1 - m;
   const int iters = nb - 1 - m;  // >= m
-  // block t of the chain: its index, the index of the next one (the top chain's last is the middle block), whether there
-  // is a next one, and whether that has this one's Schur term (not after the leading identity)
+  // block t of the chain: its index, the index of the next one (both chains' last is the middle block), and whether that
+  // has this one's Schur term (not after the leading identity)
   auto index = [&](int t) { return t == iters ? m : (top ? t - (iters - len) : nb - 1 - (t - (iters - len))); };
-  auto more = [&](int t) { return t < iters && (t + 1 < iters || lead); };
   auto join = [&](int t) { return t >= iters - len; };
 
   if (w == NT) {  // panels
+    __builtin_amdgcn_s_setprio(3);
+    int rowid = lane, colid = lane;
     if (lane < 16 * NT) s.prow[lane] = lane;  // columns beyond the padding keep their place
     for (int t = 0; t <= iters; ++t) {
       if (t == iters && !lead) return;  // the barriers of the middle inverse wait only on the waves still running
-      double csv = 0.;
-      if (more(t) && join(t)) {
+      double rsv = 0., csv = 0.;
+      if (t < iters && join(t) && lane < N) {
         const int in = index(t + 1);
-        csv = (top ? sup + (long)(in - 1) * N : sub + (long)in * N)[min(lane, N - 1)];
+        rsv = (top ? sub + (long)(in - 1) * N : sup + (long)in * N)[lane];
+        csv = (top ? sup + (long)(in - 1) * N : sub + (long)in * N)[lane];
       }
-      factor_panels<T, NT>(s, Np, lane);
-      if (lane < 16 * NT) s.cs[lane & 3][lane >> 2] = lane < N ? csv : 0.;
+      const int kap = factor_panels<T, NT>(s, N, Np, lane);
+      const int p = s.prow[lane < 16 * NT ? lane : 0];
+      const int rn = __shfl(colid, kap), cn = lane < 16 * NT ? __shfl(rowid, p) : lane;
+      rowid = rn;
+      colid = cn;
+      const double rl = __shfl(rsv, rowid), cl = __shfl(csv, colid);
+      if (lane < 16 * NT) {
+        s.rowid[lane] = min(rowid, N);
+        s.colid[lane & 3][lane >> 2] = min(colid, N);
+        s.rs[lane] = rl;
+        s.cs[lane & 3][lane >> 2] = cl;
+      }
       __syncthreads();
-      __syncthreads();
+      if (t + 1 == iters) __syncthreads();
     }
     return;
   }
@@ -386,99 +494,111 @@ twist_factor_kernel(int nsys, const int *nblocks, int n, const double *values, c
   const int r16 = lane & 15, grp = lane >> 4, row = 16 * w + r16;
   Tiles<T, NT> b;
   {
-    const Window<double> v(V + (top ? 0 : nb - 1) * NB2, N, row, grp);
+    const Window<double> v(V + (top ? 0 : nb - 1) * NB2, N);
+    const int at = row < N ? grp * N + row : 1 << 27;
 #pragma unroll
-    for (int u = 0; u < NT; ++u)
+    for (int u = 0; u < NT; ++u) {
 #pragma unroll
       for (int k = 0; k < 4; ++k)
-        b.x[u][k] = len < iters ? (row == 16 * u + 4 * k + grp ? T(1) : T(0)) : (T)v.load(16 * u + 4 * k);
-    b.pad(N, w, lane);
+        b.x[u][k] = len < iters ? (row == 16 * u + 4 * k + grp ? T(1) : T(0)) : (T)v.load(at + (16 * u + 4 * k) * N);
+    }
   }
-  T d[NT][4];
-  bool keep = false;  // d holds the inverse of block index(t - 1), not stored yet
+  int rid = 0;
+  T sig = T(1);
+  double r = 0.;
+  bool keep = false;
+  // tile u of the inverse of block index(t): its values d and places e, and the same tile of the block after it
+  auto schur = [&](int t, int u, int (&e)[4], Vec4<T> &d) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      e[k] = s.colid[grp][4 * u + k] * N + rid;
+      d[k] = b.x[u][k] * sig;
+    }
+    if (t < iters) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) b.x[u][k] = (T)(Vl[e[k]] - r * s.cs[grp][4 * u + k] * (double)d[k]);
+      if (t + 1 == iters) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) b.x[u][k] = (T)((double)b.x[u][k] - Vb[e[k]]);
+      }
+    }
+  };
+  auto store = [&](int t, const int (&e)[4], const Vec4<T> &d) {
+    if (keep && rid < N) {
+      const Window<T> o(Dg + index(t) * NB2, N);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o.store(e[k], d[k]);
+    }
+  };
+  int e0[4];
+  Vec4<T> d0;
+  auto complete = [&](int t) {  // the other tiles
+    b.pending(0);
+    store(t, e0, d0);
+#pragma unroll
+    for (int u = 1; u < NT; ++u) {
+      int e[4];
+      Vec4<T> d;
+      schur(t, u, e, d);
+      store(t, e, d);
+    }
+  };
   for (int t = 0; t <= iters; ++t) {
     // opaque to the compiler, so that the element offsets are formed again for each block instead of being kept in
     // (and spilled from) registers through the elimination
     asm volatile("" : "+s"(N));
-    if (t == iters && !lead) {
-      if (keep) {
-        const Window<T> o(Dg + index(t - 1) * NB2, N, row, grp);
+    if (t == iters && !lead) return;
+    b.eliminate(
+        s, M, N, Np, w, lane,
+        [&] {
+          if (t > 0) complete(t - 1);
+        },
+        [&] {
+          if (t < iters && (t + 1 < iters || lead)) {
+            const Window<double> v(V + index(t + 1) * NB2, N);
+            const int e = w * 64 + lane;
+            double q[4 * NT];
 #pragma unroll
-        for (int u = 0; u < NT; ++u)
+            for (int k = 0; k < 4 * NT; ++k) q[k] = v.load(e + 64 * NT * k);
 #pragma unroll
-          for (int k = 0; k < 4; ++k) o.store(16 * u + 4 * k, d[u][k]);
-      }
-      return;
-    }
-    const bool nxt = more(t);
-    double v[NT][4], r = 0.;
-    const int kap = b.eliminate(s, M, Np, w, lane, [&](int k) {
-      if (k == 0 && keep) {
-        const Window<T> o(Dg + index(t - 1) * NB2, N, row, grp);
-#pragma unroll
-        for (int u = 0; u < NT; ++u)
-#pragma unroll
-          for (int k = 0; k < 4; ++k) o.store(16 * u + 4 * k, d[u][k]);
-      }
-      if (k == (Np > 8 ? 1 : 0) && nxt) {  // not used before the block's inverse is done
-        const int in = index(t + 1);
-        const Window<double> vi(V + in * NB2, N, row, grp);
-#pragma unroll
-        for (int u = 0; u < NT; ++u)
-#pragma unroll
-          for (int k = 0; k < 4; ++k) v[u][k] = vi.load(16 * u + 4 * k);
-        r = (top ? sub + (long)(in > 0 ? in - 1 : 0) * N : sup + (long)in * N)[min(row, N - 1)];
-      }
-    });
-    __syncthreads();  // M becomes the inverse
-    {
-      const T sig = s.sig[row];
-      T *to = M + kap;
-#pragma unroll
-      for (int u = 0; u < NT; ++u)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) to[s.prow[16 * u + 4 * k + grp] * S::IS] = b.x[u][k] * sig;
-    }
-    __syncthreads();
-    const int nat = grp * S::IS + row;
-#pragma unroll
-    for (int u = 0; u < NT; ++u)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) d[u][k] = M[nat + (16 * u + 4 * k) * S::IS];
-    keep = t >= iters - len || t == iters;
-    if (nxt) {
-      r = join(t) && row < N ? r : 0.;
-#pragma unroll
-      for (int u = 0; u < NT; ++u)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) b.x[u][k] = (T)(v[u][k] - r * s.cs[grp][4 * u + k] * (double)d[u][k]);
-      if (t + 1 == iters) {  // the top chain: the bottom chain's term of the middle block
-        const double rm = row < N ? sup[(long)m * N + row] : 0.;
+            for (int k = 0; k < 4 * NT; ++k) Vl[min(e + 64 * NT * k, N * N)] = q[k];
+          }
+        });
+    __syncthreads();  // the order of the inverse, the scales
+    rid = s.rowid[row];
+    r = s.rs[row];
+    sig = s.sig[row];
+    keep = join(t) || t == iters;
+    if (t + 1 == iters) {
+      if (!lead) {  // the bottom chain's term of the middle block, and its last store
+        b.pending(0);
 #pragma unroll
         for (int u = 0; u < NT; ++u)
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            const int c = 16 * u + 4 * k + grp;
-            const double cm = sub[(long)m * N + min(c, N - 1)];
-            b.x[u][k] = (T)((double)b.x[u][k] - (c < N ? rm * cm : 0.) * (double)E[nat + (16 * u + 4 * k) * S::IS]);
+            const int c = s.colid[grp][4 * u + k];
+            const T x = b.x[u][k] * sig;
+            if (rid < N && c < N) {
+              Vl[c * N + rid] = r * (double)x * s.cs[grp][4 * u + k];
+              Dg[index(t) * NB2 + c * N + rid] = x;
+            }
           }
       }
-      b.pad(N, w, lane);
+      __syncthreads();
+      if (!lead) return;
     }
+    schur(t, 0, e0, d0);
   }
-  const Window<T> o(Dg + m * NB2, N, row, grp);
-#pragma unroll
-  for (int u = 0; u < NT; ++u)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) o.store(16 * u + 4 * k, d[u][k]);
+  complete(iters);
 }
 
 template <typename T, int NT>
 int launch_nt(int nsys, const int *nblocks, int bs, const double *values, const long *voff, T *dinv,
               const long *doff, hipStream_t st) {
   auto kern = twist_factor_kernel<T, NT>;
-  const size_t lds = 2 * sizeof(T) * ChainLds<T, NT>::words((bs + 7) & ~7);
-  if (lds + 2 * sizeof(ChainLds<T, NT>) > 65536 &&
+  using S = ChainLds<T, NT>;
+  const size_t lds = sizeof(double) * ((2 * S::v_words(bs) + 1) & ~1) + 2 * sizeof(T) * S::m_words((bs + 7) & ~7);
+  if (lds + 2 * sizeof(S) > 65536 &&
       hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return fail(GF_ERR_UNSUPPORTED, "block too large for LDS");
   hipLaunchKernelGGL(kern, dim3(nsys), dim3(128 * (NT + 1)), lds, st, nsys, nblocks, bs, values, voff, dinv, doff);

@@ -3,7 +3,7 @@
 // tiles of sixteen and keeps several waves per chain; once the systems alone fill the chip, small blocks are faster
 // without either (launch_btd_inv_factor).
 #include "gf_internal.h"
-#include "gf_gj.h"
+#include "gf_wave.h"
 #include "../../include/griffon_amd.h"
 
 #include <utility>
@@ -13,7 +13,56 @@ namespace gfa {
 namespace {
 
 using wave::lane_value;
-using gj::reg_gj_inverse;
+using wave::wave_first_argmax;
+
+// Gauss-Jordan inverse of an N x N block held in the registers of one wave, with partial (row) pivoting.
+//
+// Layout: lane l holds one row, x[k] the entry in slot k. The entry of lane l, slot k is element
+// (rowid of lane l, colid of slot k) of the logical matrix, where colid of slot k is held by lane k of
+// `colid`. Rows are never interchanged: the pivot of step j is the unused lane with the largest |entry| in
+// the pivot column (ties: lowest lane), and the exchange at (pivot lane p, slot j) is done in place. After N
+// steps the block holds the inverse in the same kind of layout: the lane pivoted at step j holds row
+// colid_j of the inverse, slot j holds its column rowid_{p_j}.
+//
+// The slots form a queue: the pivot column is always x[0]; each step shifts the other columns down by one
+// and appends the transformed pivot column at x[N-1], so that all register indices are compile-time
+// constants and after N steps every column is back in its slot. The pivot row is broadcast through scalar
+// registers (readlane), so a step has no LDS traffic and no barrier.
+//
+// Row scaling is deferred: lane r keeps its row unscaled and a factor sig_r, the true row being sig_r times
+// the stored one. Every row is pivoted exactly once and has sig = 1 until then, so at the step that pivots
+// lane p (stored pivot value d):
+//   rows r != p:   x_r[c] -= g_r x_p[c] (c != k),  x_r[k] = -g_r,  with g_r = x_r[k] / d
+//   row p:         x_p[c] unchanged,  x_p[k] = 1,  sig_p = 1 / d
+// which is the usual step (row p divided by its pivot) with the division of row p left to the end: the update
+// of a slot is one fma, with no separate scaling of the pivot row. After N steps every row is multiplied by
+// its sig.
+template <typename T, int N>
+__device__ __forceinline__ void reg_gj_inverse(T (&x)[N], int &rowid, int &colid, int lane) {
+  bool used = lane >= N;
+  T sig = T(1);
+  for (int j = 0; j < N; ++j) {
+    const T f = x[0];
+    const T rf = T(1) / f;  // every lane's reciprocal, formed beside the pivot search instead of after it
+    const int p = wave_first_argmax(fabs(f), !used);  // N - j unused lanes remain, so p >= 0
+    const T ipv = lane_value(rf, p);
+    const bool isp = lane == p;
+    const T g = isp ? T(0) : f * ipv;  // multiplier of the broadcast pivot row (none for the pivot row)
+#pragma unroll
+    for (int c = 1; c < N; ++c) x[c - 1] = fma(-g, lane_value(x[c], p), x[c]);
+    x[N - 1] = isp ? T(1) : -g;  // the pivot column
+    if (isp) sig = ipv;
+    const int cj = __builtin_amdgcn_readlane(colid, j);
+    const int rp = __builtin_amdgcn_readlane(rowid, p);
+    if (isp) {
+      rowid = cj;
+      used = true;
+    }
+    if (lane == j) colid = rp;
+  }
+#pragma unroll
+  for (int c = 0; c < N; ++c) x[c] *= sig;
+}
 
 // Block i of the values in the identity layout (lane = row, slot = column).
 template <typename T, int N>

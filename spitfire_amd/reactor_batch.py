@@ -35,8 +35,8 @@ from .time_integration import KennedyCarpenterS6P4Q3, SimpleNewtonSolver
 
 class _BatchedLU:
     """Solves with R independent ns x ns column-major blocks: each block inverted once per factor() by the
-    register-resident Gauss-Jordan kernel with partial pivoting, each solve one matrix-vector product with the stored
-    FP64 inverse (the one-block case of the batched block-tridiagonal solve)."""
+    blocked Gauss-Jordan kernel with partial pivoting (the one-block case of the batched block-tridiagonal inverse
+    form), each solve one matrix-vector product with the stored FP64 inverse."""
 
     def __init__(self, R, ns, device):
         import torch
@@ -54,7 +54,10 @@ class _BatchedLU:
     def factor(self, values, stream):
         """values: contiguous [R, ns*ns] column-major blocks (left unmodified)"""
         self.values = values
-        self._check(self._lib.gf_batch_block_inverse(self.R, self.ns, values.data_ptr(), self.inv.data_ptr(), stream))
+        self._check(self._lib.gf_batch_btddod_inverse_factorize(self.R, self.nb.data_ptr(), self.ns,
+                                                                values.data_ptr(), self.voff.data_ptr(),
+                                                                self.inv.data_ptr(), self.voff.data_ptr(), 64,
+                                                                stream))
 
     def solve(self, rhs, out, stream):
         self._check(self._lib.gf_batch_btddod_inverse_solve(self.R, self.nb.data_ptr(), self.ns,

@@ -74,3 +74,22 @@ def test_inverse_factor_of_singular_and_nonfinite_blocks(bs):
     assert not np.isfinite(got[1]).any() and not np.isfinite(got[2]).all()
     for s in (0, 3):
         assert np.max(np.abs(got[s][0] @ blocks[s][0] - np.eye(bs))) <= 1e-12
+
+
+@pytest.mark.parametrize('precision', [64, 32])
+@pytest.mark.parametrize('bs', [1, 2, 7, 8, 9, 11])
+def test_inverse_factor_routes_are_bitwise_the_same(bs, precision):
+    """Few systems go to the panel kernel, many small ones to the one-wave kernel: the same elimination, entry by entry,
+    also where pivots tie, over chains long enough to permute rows and columns of a permuted block. Tolerance: none."""
+    rng = np.random.default_rng(bs)
+    sizes = [1, 2, 3, 6, 7, 1, 4]
+    values = []
+    for s, n in enumerate(sizes):
+        V = rng.standard_normal(n * bs * bs) if s % 2 else rng.integers(-2, 3, n * bs * bs).astype(float)
+        values.append(np.concatenate([V, rng.standard_normal(2 * (n - 1) * bs)]))
+    few = _factor(sizes, bs, values, precision)
+    many = _factor(sizes * 230, bs, values * 230, precision)  # 1,610 systems
+    for s in range(len(sizes)):
+        for k in (0, 229):
+            a, b = few[s], many[s + k * len(sizes)]
+            assert np.array_equal(np.isfinite(a), np.isfinite(b)) and np.array_equal(a[np.isfinite(a)], b[np.isfinite(b)])
