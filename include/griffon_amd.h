@@ -322,6 +322,19 @@ int gf_flamelet_batch_transient_rhs(gf_flamelet_batch *b, const int *flags, cons
 int gf_flamelet_batch_transient_setup(gf_flamelet_batch *b, const int *flags, const double *x,
                                       const double *prefactor, int lu_precision);
 int gf_flamelet_batch_transient_solve(gf_flamelet_batch *b, const int *flags, const double *r, double *out);
+/* The stage Newton method of those steps (nonlinear.py:185-268) on the same device vectors; h: host, one step size per
+ * flamelet; norms: host, one per flamelet, max |v / scale| with T scaled by 1e3, NaN where an entry is not finite.
+ *   transient_residual: r = h (gamma f + prior) - (x - xn) for the flagged flamelets
+ *   transient_newton:   one iteration of the flagged flamelets: d = (prefactor J - I)^-1 r, x -= d, f = F(x), then r as
+ *                       above and norms of r (entries of the other flamelets are left as they are)
+ *   vector_norms:       norms of v, every flamelet */
+int gf_flamelet_batch_transient_residual(gf_flamelet_batch *b, const int *flags, const double *h, double gamma,
+                                         const double *f, const double *prior, const double *x, const double *xn,
+                                         double *r);
+int gf_flamelet_batch_transient_newton(gf_flamelet_batch *b, const int *flags, const double *h, double gamma,
+                                       const double *prior, const double *xn, double *x, double *f, double *r,
+                                       double *d, double *norms);
+int gf_flamelet_batch_vector_norms(gf_flamelet_batch *b, const double *v, double *norms);
 
 #ifdef __cplusplus
 }

@@ -93,6 +93,9 @@ SIGNATURES = {
     'gf_flamelet_batch_transient_rhs': [_V, _I, _V, _V],
     'gf_flamelet_batch_transient_setup': [_V, _I, _V, _D, _int],
     'gf_flamelet_batch_transient_solve': [_V, _I, _V, _V],
+    'gf_flamelet_batch_transient_residual': [_V, _I, _D, _dbl, _V, _V, _V, _V, _V],
+    'gf_flamelet_batch_transient_newton': [_V, _I, _D, _dbl, _V, _V, _V, _V, _V, _V, _D],
+    'gf_flamelet_batch_vector_norms': [_V, _V, _D],
 }
 
 

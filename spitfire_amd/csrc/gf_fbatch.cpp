@@ -599,7 +599,10 @@ int gf_flamelet_batch_create(gf_mech *m, int nfl, const int *nzi, double pressur
   v.NI = b->NI;
   v.NV = V;
   v.NJ = Jv;
-  for (int f = 0; f < nfl; ++f) v.maxNJ = std::max(v.maxNJ, (long)ns * ((long)nzi[f] * ns + 2 * (nzi[f] - 1)));
+  for (int f = 0; f < nfl; ++f) {
+    v.maxNJ = std::max(v.maxNJ, (long)ns * ((long)nzi[f] * ns + 2 * (nzi[f] - 1)));
+    v.maxNV = std::max(v.maxNV, (long)nzi[f] * ns);
+  }
   T(launch_fb_stencils(v, b->dz, b->ddz0, nullptr, b->cmaj, b->csub, b->csup, b->mco, b->nco, st));
   if (rc == GF_OK && hipStreamSynchronize(st) != hipSuccess) rc = fail(GF_ERR_HIP, "stream synchronize failed");
   if (rc != GF_OK) {
@@ -734,6 +737,24 @@ int gf_flamelet_batch_steady_newton(gf_flamelet_batch *b, const gf_psitc_options
   return steady(b, opts, 1, select, iterations, converged, residual, nullptr, counters);
 }
 
+namespace {
+// the flagged flamelets, all of which must hold transient_setup factors
+int factored(const gf_flamelet_batch *b, const int *flags, std::vector<int> &fl) {
+  for (int f = 0; f < b->B; ++f)
+    if (flags[f]) {
+      if (!b->tr_set[f]) return fail(GF_ERR_STATE, "transient_solve before transient_setup for a flamelet");
+      fl.push_back(f);
+    }
+  return GF_OK;
+}
+
+int transient_solve(gf_flamelet_batch *b, int n, const double *r, double *out, hipStream_t st) {
+  if (b->tr_prec == 32)
+    return launch_btd_inv_solve<float>(n, b->sys_nb, b->ns, b->J, b->sys_v, b->D32, b->sys_l, r, out, b->sys_x, st);
+  return launch_btd_inv_solve<double>(n, b->sys_nb, b->ns, b->J, b->sys_v, b->L, b->sys_l, r, out, b->sys_x, st);
+}
+}  // namespace
+
 int gf_flamelet_batch_transient_rhs(gf_flamelet_batch *b, const int *flags, const double *x, double *rhs) {
   if (!b || !flags || !x || !rhs) return fail(GF_ERR_ARG, "null argument");
   Psitc s{b, {}, b->m->stream};
@@ -770,20 +791,57 @@ int gf_flamelet_batch_transient_solve(gf_flamelet_batch *b, const int *flags, co
   if (!b || !flags || !r || !out) return fail(GF_ERR_ARG, "null argument");
   Psitc s{b, {}, b->m->stream};
   std::vector<int> fl;
-  for (int f = 0; f < b->B; ++f)
-    if (flags[f]) {
-      if (!b->tr_set[f]) return fail(GF_ERR_STATE, "transient_solve before transient_setup for a flamelet");
-      fl.push_back(f);
-    }
+  GF_TRY(factored(b, flags, fl));
   if (fl.empty()) return GF_OK;
   GF_TRY(s.systems(fl));
-  if (b->tr_prec == 32)
-    GF_TRY(launch_btd_inv_solve<float>((int)fl.size(), b->sys_nb, b->ns, b->J, b->sys_v, b->D32, b->sys_l, r, out,
-                                       b->sys_x, s.st));
-  else
-    GF_TRY(launch_btd_inv_solve<double>((int)fl.size(), b->sys_nb, b->ns, b->J, b->sys_v, b->L, b->sys_l, r, out,
-                                        b->sys_x, s.st));
+  GF_TRY(transient_solve(b, (int)fl.size(), r, out, s.st));
   return s.sync();
+}
+
+int gf_flamelet_batch_transient_residual(gf_flamelet_batch *b, const int *flags, const double *h, double gamma,
+                                         const double *f, const double *prior, const double *x, const double *xn,
+                                         double *r) {
+  if (!b || !flags || !h || !f || !prior || !x || !xn || !r) return fail(GF_ERR_ARG, "null argument");
+  Psitc s{b, {}, b->m->stream};
+  std::vector<int> fl;
+  GF_TRY(s.flagged(flags, fl));
+  if (fl.empty()) return GF_OK;
+  GF_TRY(s.up(b->fval, std::vector<double>(h, h + b->B)));
+  GF_TRY(launch_fb_stage_residual(b->view, b->flag, b->fval, gamma, f, prior, x, xn, r, nullptr, s.st));
+  return s.sync();
+}
+
+int gf_flamelet_batch_transient_newton(gf_flamelet_batch *b, const int *flags, const double *h, double gamma,
+                                       const double *prior, const double *xn, double *x, double *f, double *r,
+                                       double *d, double *norms) {
+  if (!b || !flags || !h || !prior || !xn || !x || !f || !r || !d || !norms) return fail(GF_ERR_ARG, "null argument");
+  Psitc s{b, {}, b->m->stream};
+  std::vector<int> fl;
+  GF_TRY(factored(b, flags, fl));
+  if (fl.empty()) return GF_OK;
+  GF_TRY(s.up(b->flag, s.flags_of(fl)));
+  GF_TRY(s.up(b->fval, std::vector<double>(h, h + b->B)));
+  GF_TRY(s.systems(fl));
+  GF_TRY(transient_solve(b, (int)fl.size(), r, d, s.st));
+  GF_TRY(launch_fb_stage_update(b->view, b->flag, d, x, b->fres, s.st));
+  GF_TRY(launch_fb_unpack(b->view, b->flag, b->ddof0, x, b->X, 1, s.st));
+  GF_TRY(s.chem(b->X, fl, false));
+  GF_TRY(launch_fb_rhs(b->view, b->X, b->flag, f, s.st));
+  GF_TRY(launch_fb_stage_residual(b->view, b->flag, b->fval, gamma, f, prior, x, xn, r, b->fres, s.st));
+  std::vector<double> res;
+  GF_TRY(s.down(res, b->fres, b->B));
+  for (int q : fl) norms[q] = res[q];
+  return GF_OK;
+}
+
+int gf_flamelet_batch_vector_norms(gf_flamelet_batch *b, const double *v, double *norms) {
+  if (!b || !v || !norms) return fail(GF_ERR_ARG, "null argument");
+  Psitc s{b, {}, b->m->stream};
+  GF_TRY(launch_fb_vector_norms(b->view, v, b->fres, s.st));
+  std::vector<double> res;
+  GF_TRY(s.down(res, b->fres, b->B));
+  std::memcpy(norms, res.data(), res.size() * sizeof(double));
+  return GF_OK;
 }
 
 }  // extern "C"

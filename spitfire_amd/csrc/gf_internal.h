@@ -237,6 +237,7 @@ struct FlameletBatchView {
   long NI = 0;          // total interior points
   long NV = 0, NJ = 0;  // total unknowns, total Jacobian entries
   long maxNJ = 0;       // Jacobian entries of the largest flamelet
+  long maxNV = 0;       // unknowns of the largest flamelet
 };
 int launch_fb_stencils(const FlameletBatchView &b, const double *dz, const long *dz0, const double *invLe,
                        double *cmaj, double *csub, double *csup, double *mco, double *nco, hipStream_t st);
@@ -260,6 +261,14 @@ int launch_fb_ds(const FlameletBatchView &b, const int *flag, const int *global_
                  const double *diffterm, double safety, double ramp, double dsmax, double *ds, hipStream_t st);
 int launch_fb_fill_dofs(const FlameletBatchView &b, const int *flag, const double *value, double *dst,
                         hipStream_t st);
+// stage solves of implicit time stepping: x -= d and the norms cleared; r = h (gamma f + prior) - (x - xn) and its norms
+// (when given); norms of a vector
+int launch_fb_stage_update(const FlameletBatchView &b, const int *flag, const double *d, double *x, double *norm,
+                           hipStream_t st);
+int launch_fb_stage_residual(const FlameletBatchView &b, const int *flag, const double *h, double gamma,
+                             const double *f, const double *prior, const double *x, const double *xn, double *r,
+                             double *norm, hipStream_t st);
+int launch_fb_vector_norms(const FlameletBatchView &b, const double *v, double *norm, hipStream_t st);
 int launch_fb_clip_points(long n, double *X, hipStream_t st);
 // kexp (optional, laid out like out with nout = n) carries each block's balancing exponents between launches
 int launch_expeig_list(const gf_mech *m, const double *blocks, const long *boff, const long *ooff, long nblk, int n,

@@ -960,7 +960,7 @@ class FlameletBatch:
         import ctypes
         import sys
         import torch
-        from ._native import check, iptr
+        from ._native import check, dptr, iptr
         from .time_integration import KennedyCarpenterS6P4Q3, SimpleNewtonSolver
         for k in unused:
             if k not in ('write_log', 'save_first_and_last_only', 'stop_at_time', 'stop_criteria'):
@@ -972,7 +972,6 @@ class FlameletBatch:
         tab = KennedyCarpenterS6P4Q3(SimpleNewtonSolver())
         A, bw, bh, g = tab.A, tab.b, tab.bh, tab.gamma
         seg = torch.tensor(np.repeat(np.arange(B), np.diff(self._offsets)), device=dev)
-        w = 1. / torch.tensor(np.concatenate([f._variable_scales for f in self._flamelets]), device=dev)
         x = torch.tensor(self._x0, device=dev)
         maxsteps = np.inf if maximum_time_step_count is None else int(maximum_time_step_count)
         dt = np.broadcast_to(np.asarray(first_time_step, dtype=np.float64), (B,)).copy()
@@ -992,10 +991,10 @@ class FlameletBatch:
 
         def fnorm(v):
             """per flamelet max |v * 1/scale|, NaN where any entry is not finite"""
-            m = torch.zeros(B, dtype=torch.float64, device=dev).scatter_reduce_(0, seg, (v * w).abs(), 'amax')
-            bad = torch.zeros(B, dtype=torch.float64, device=dev).scatter_reduce_(
-                0, seg, (~torch.isfinite(v)).to(torch.float64), 'amax')
-            return torch.where(bad > 0, torch.full_like(m, np.nan), m).cpu().numpy()
+            out = np.empty(B)
+            torch.cuda.current_stream().synchronize()
+            check(lib.gf_flamelet_batch_vector_norms(h, v.data_ptr(), dptr(out)))
+            return out
 
         def rhs(m, xv, out):
             torch.cuda.current_stream().synchronize()
@@ -1009,11 +1008,22 @@ class FlameletBatch:
                                                         int(lu_precision)))
             stats['projector_setups'] += int(m.sum())
 
-        def solve(m, r, out):
-            torch.cuda.current_stream().synchronize()
-            check(lib.gf_flamelet_batch_transient_solve(h, iptr(mask(m)), r.data_ptr(), out.data_ptr()))
+        norms = np.zeros(B)
 
-        d = torch.zeros_like(x)
+        def residual(m, f, prior, xi, xn, r):
+            torch.cuda.current_stream().synchronize()
+            check(lib.gf_flamelet_batch_transient_residual(h, iptr(mask(m)), dptr(dt), g, f.data_ptr(),
+                                                           prior.data_ptr(), xi.data_ptr(), xn.data_ptr(),
+                                                           r.data_ptr()))
+
+        def newton(m, prior, xn, xi, f, r):
+            """one stage iteration of the flamelets in m; the norms of their residuals are left in norms"""
+            check(lib.gf_flamelet_batch_transient_newton(h, iptr(mask(m)), dptr(dt), g, prior.data_ptr(),
+                                                         xn.data_ptr(), xi.data_ptr(), f.data_ptr(), r.data_ptr(),
+                                                         d.data_ptr(), dptr(norms)))
+            stats['nonlinear_iter'] += int(m.sum())
+
+        d, r = torch.zeros_like(x), torch.zeros_like(x)
         while True:
             run = running & ~steady
             if not run.any():
@@ -1033,20 +1043,16 @@ class FlameletBatch:
             for s in range(1, 6):
                 prior = sum(A[s, j] * ks[j] for j in range(s))
                 fi = ks[-1].clone()
-                r = hd * (g * fi + prior) - (xi - xn)
+                residual(run, fi, prior, xi, xn, r)
                 done = ~run
                 for it in range(max_nonlinear_iter):
                     act = ~done
-                    solve(act, r, d)
-                    xi = torch.where(on_dofs(act), xi - d, xi)
-                    rhs(act, xi, fi)
-                    r = hd * (g * fi + prior) - (xi - xn)
-                    stats['nonlinear_iter'] += int(act.sum())
-                    done = done | (act & (fnorm(r) < nonlinear_solve_tolerance))
+                    newton(act, prior, xn, xi, fi, r)
+                    done = done | (act & (norms < nonlinear_solve_tolerance))
                     if done.all():
                         break
                 converged &= done  # a stage left unconverged also marks the step's solve slow
-                ks.append(fi.clone())
+                ks.append(fi)
             dstate = hd * sum(bw[j] * ks[j] for j in range(6))
             err = fnorm(dstate - hd * sum(bh[j] * ks[j] for j in range(6)))
             with np.errstate(invalid='ignore', divide='ignore'):

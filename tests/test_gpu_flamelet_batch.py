@@ -345,3 +345,70 @@ def test_lewis_numbers_batch_matches_oracle(mech_c1_data, oracle_lib):
         e = _scaled(states[k], f.current_interior_state, ns)
         say('  flamelet %d: batch %d iterations, oracle %s, max scaled diff %.3e' % (k, its[k], it, e))
         assert conv[k] and ok and e <= 1e-8
+
+
+@pytest.mark.parametrize('npts', [[9, 34, 4], [131]])
+def test_fused_stage_iteration_and_norms(npts, mech_c1_data):
+    """The fused stage iteration against the same step by its separate entry points and elementwise operations, and the
+    norms (workgroups of 1,024 unknowns: fewer, and several) against NumPy, with infinities and NaN; only the flagged
+    flamelets change. Tolerance: none (the same operations in the same order, and maxima)."""
+    import torch
+    from spitfire_amd import _native
+    from spitfire_amd.flamelet import FlameletBatch
+    from spitfire_amd.mechanism import ChemicalMechanismSpec
+    m = ChemicalMechanismSpec(mech_c1_data)
+    B, ns = len(npts), m.n_species
+    fb = FlameletBatch(_flamelets(m, [10.] * B, npts))
+    lib, dev = _native.lib(), torch.device('cuda:0')
+    scale = np.concatenate([f._variable_scales for f in fb._flamelets])
+    rng = np.random.default_rng(1)
+
+    def norms(v):
+        out = np.empty(B)
+        t = torch.tensor(v, device=dev)
+        torch.cuda.synchronize()
+        _native.check(lib.gf_flamelet_batch_vector_norms(fb._h, t.data_ptr(), _native.dptr(out)))
+        return out
+
+    v = rng.standard_normal(fb._x0.size)
+    ref = np.array([np.max(np.abs(q)) for q in fb.split(v / scale * 1.)])
+    assert np.allclose(norms(v), ref, rtol=2.3e-16, atol=0.) and not norms(0. * v).any()
+    for bad in (np.nan, np.inf, -np.inf):
+        w = v.copy()
+        w[-1] = bad
+        got = norms(w)
+        assert np.isnan(got[-1]) and np.isfinite(got[:-1]).all()
+
+    x0 = torch.tensor(fb._x0, device=dev)
+    flags = np.ones(B, dtype=np.int32)
+    flags[1:2] = 0
+    every = np.ones(B, dtype=np.int32)
+    gamma, h = 0.25, np.full(B, 1e-7)
+    hd = torch.tensor(np.concatenate([np.full(q.size, a) for q, a in zip(fb.split(fb._x0), h)]), device=dev)
+    on = torch.tensor(np.concatenate([np.full(q.size, bool(a)) for q, a in zip(fb.split(fb._x0), flags)]), device=dev)
+    torch.cuda.synchronize()
+    i, d = _native.iptr, _native.dptr
+    pre = h * gamma
+    _native.check(lib.gf_flamelet_batch_transient_setup(fb._h, i(every), x0.data_ptr(), d(pre), 64))
+    f0 = torch.zeros_like(x0)
+    _native.check(lib.gf_flamelet_batch_transient_rhs(fb._h, i(every), x0.data_ptr(), f0.data_ptr()))
+    prior = 0.3 * f0
+    r = torch.full_like(x0, 7.)
+    x, f, s = x0.clone(), f0.clone(), torch.zeros_like(x0)
+    torch.cuda.synchronize()
+    _native.check(lib.gf_flamelet_batch_transient_residual(fb._h, i(flags), d(h), gamma, f0.data_ptr(), prior.data_ptr(),
+                                                           x0.data_ptr(), x0.data_ptr(), r.data_ptr()))
+    rr = torch.where(on, hd * (gamma * f0 + prior) - (x0 - x0), torch.full_like(x0, 7.))
+    assert torch.equal(r, rr)
+    out = np.full(B, -1.)
+    _native.check(lib.gf_flamelet_batch_transient_newton(fb._h, i(flags), d(h), gamma, prior.data_ptr(), x0.data_ptr(),
+                                                         x.data_ptr(), f.data_ptr(), r.data_ptr(), s.data_ptr(), d(out)))
+    step = torch.zeros_like(x0)
+    _native.check(lib.gf_flamelet_batch_transient_solve(fb._h, i(flags), rr.data_ptr(), step.data_ptr()))
+    xr = torch.where(on, x0 - step, x0)
+    fr = f0.clone()
+    torch.cuda.synchronize()
+    _native.check(lib.gf_flamelet_batch_transient_rhs(fb._h, i(flags), xr.data_ptr(), fr.data_ptr()))
+    rr = torch.where(on, hd * (gamma * fr + prior) - (xr - x0), torch.full_like(x0, 7.))
+    assert torch.equal(x, xr) and torch.equal(f, fr) and torch.equal(r, rr)
+    assert np.array_equal(out, np.where(flags, norms(r.cpu().numpy()), -1.))
