@@ -19,6 +19,8 @@
 // and stored as its inverse, so no L blocks are stored and both sweeps of a solve are matrix-vector products.
 #include "gf_internal.h"
 #include "../../include/griffon_amd.h"
+
+#include <utility>
 #include "gf_wave.h"
 
 
@@ -230,120 +232,154 @@ __global__ void __launch_bounds__(BW) btd_solve_kernel(int nsys, const int *nblo
 
 // ---------------- block Thomas with explicit diagonal-block inverses ----------------
 
-// y = D v for a column-major bs x bs block and v held one entry per lane (lane = row); the entries of v are
-// broadcast through scalar registers and four partial sums keep the column loads independent.
-template <typename T>
-__device__ __forceinline__ double wave_matvec(const T *D, int bs, double v, int lane) {
-  const bool act = lane < bs;
-  double m0 = 0., m1 = 0., m2 = 0., m3 = 0.;
-  int c = 0;
-  // Sixteen columns per trip, their loads issued together before the products (column c still goes to the
-  // partial sum of c mod 4, in column order, so the result is the same as four at a time). Lanes past the block
-  // read row 0 and discard it: a load under a lane condition was compiled as a branch around each load for
-  // FP32 blocks, which serialised them.
-  const int rl = act ? lane : 0;
-  for (; c + 15 < bs; c += 16) {
-    double d[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) d[q] = (double)D[(c + q) * bs + rl];
-#pragma unroll
-    for (int q = 0; q < 16; q += 4) {
-      const double v0 = lane_value(v, c + q), v1 = lane_value(v, c + q + 1), v2 = lane_value(v, c + q + 2),
-                   v3 = lane_value(v, c + q + 3);
-      if (act) {
-        m0 += d[q] * v0;
-        m1 += d[q + 1] * v1;
-        m2 += d[q + 2] * v2;
-        m3 += d[q + 3] * v3;
-      }
-    }
-  }
-  for (; c + 3 < bs; c += 4) {
-    const double d0 = (double)D[c * bs + rl], d1 = (double)D[(c + 1) * bs + rl], d2 = (double)D[(c + 2) * bs + rl],
-                 d3 = (double)D[(c + 3) * bs + rl];
-    const double v0 = lane_value(v, c), v1 = lane_value(v, c + 1), v2 = lane_value(v, c + 2),
-                 v3 = lane_value(v, c + 3);
-    if (act) {
-      m0 += d0 * v0;
-      m1 += d1 * v1;
-      m2 += d2 * v2;
-      m3 += d3 * v3;
-    }
-  }
-  for (; c < bs; ++c) {
-    const double d0 = (double)D[c * bs + rl];
-    const double v0 = lane_value(v, c);
-    if (act) m0 += d0 * v0;
-  }
-  return (m0 + m1) + (m2 + m3);
-}
-
-// Solve with the twisted factors, one workgroup of two waves per system, lane = row:
-//   wave 0:  y_0 = b_0,  y_i = b_i - sub_{i-1} (D_{i-1}^{-1} y_{i-1}),  i < m
-//   wave 1:  y_{n-1} = b_{n-1},  y_i = b_i - sup_i (E_{i+1}^{-1} y_{i+1}),  i > m
+// Solve with the twisted factors, one workgroup of eight waves per system: waves 0 .. 3 the top chain, 4 .. 7 the bottom one,
+//   top:     y_0 = b_0,  y_i = b_i - sub_{i-1} (D_{i-1}^{-1} y_{i-1}),  i < m
+//   bottom:  y_{n-1} = b_{n-1},  y_i = b_i - sup_i (E_{i+1}^{-1} y_{i+1}),  i > m
 //   middle:  x_m = C_m^{-1} (b_m - sub_{m-1} (D_{m-1}^{-1} y_{m-1}) - sup_m (E_{m+1}^{-1} y_{m+1}))
-//   wave 0:  x_i = D_i^{-1} (y_i - sup_i x_{i+1}),  i = m-1 .. 0;   wave 1:  x_i = E_i^{-1} (y_i - sub_{i-1} x_{i-1}),  i > m
+//   top:     x_i = D_i^{-1} (y_i - sup_i x_{i+1}),  i = m-1 .. 0;   bottom:  x_i = E_i^{-1} (y_i - sub_{i-1} x_{i-1}),  i > m
+// A chain is a series of 2 len + 1 products with its blocks, inwards, the middle one, outwards again. Each is shared by four
+// waves (lane = row): wave q multiplies the columns 4 k + q of the block, the vector's entries broadcast through scalar
+// registers, and the sum of the four partial sums, exchanged through LDS behind one barrier, is formed by every wave, which
+// so holds the next vector. With few chains the steps between two products bound it (the exchange, the broadcasts, about
+// 1,000 cycles at 53), with many the two reads of the inverses: 1,024 chains move 7.1 GB in 1.8 ms. Loads are issued two
+// products ahead (FP32 three): more is no faster, and takes the registers that let two workgroups share a
+// compute unit, which batches of single blocks need. Before, two waves per system did a whole product each, in
+// batches of sixteen column loads that were waited for one after the other. Measured before and after (53x53, us):
+//   systems                     FP64             FP32
+//   one chain of 126 blocks       277 ->   150     268 -> 108
+//   48 / 192 chains of 62..254    788 / 1,079 -> 311 / 438     722 / 925 -> 231 / 267
+//   512 / 1,024 chains          1,293 / 1,931 -> 940 / 1,811   1,073 / 1,301 -> 501 / 975
+//   4,000 blocks                   19 ->    19      14 ->  13
+// The partial sums are those of columns c mod 4 in ascending order, the columns beyond the last group of four in the
+// first one, and the sum is (m0 + m1) + (m2 + m3), as before: solutions are bitwise the same.
 template <typename T>
-__global__ void __launch_bounds__(128) btd_twist_solve_kernel(int nsys, const int *nblocks, int bs,
-                                                              const double *values, const long *voff,
+constexpr int kAhead = sizeof(T) == 8 ? 2 : 3;
+
+template <typename T, int N>
+__global__ void __launch_bounds__(512) btd_twist_solve_kernel(const int *nblocks, const double *values, const long *voff,
                                                               const T *dinv, const long *doff, const double *rhs,
                                                               double *x, const long *xoff) {
-  __shared__ double mid[2][64];
-  const int sys = blockIdx.x;
-  if (sys >= nsys) return;
+  constexpr int K = N / 4, E = N % 4;
+  __shared__ double part[2][2][4][64];  // [parity of the product][chain][wave][row]
   const int lane = threadIdx.x & 63;
-  const bool top = threadIdx.x < 64;
-  const bool act = lane < bs;
-  const int nb = nblocks[sys];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int chain = wave >> 2, q = wave & 3;
+  const bool top = chain == 0;
+  const int sys = blockIdx.x;
+  const int nb = __builtin_amdgcn_readfirstlane(nblocks[sys]);
+  if (!top && nb == 1) return;  // no bottom chain
+  const bool act = lane < N;
+  const int rl = act ? lane : 0;
   const int m = (nb - 1) / 2;
-  const long nb2 = (long)bs * bs;
-  const double *V = values + voff[sys];
-  const T *DI = dinv + doff[sys];
+  const T *DI = dinv + doff[sys] + rl;
   const double *b = rhs + xoff[sys];
   double *X = x + xoff[sys];
-  const double *sub = V + (long)nb * nb2;
-  const double *sup = sub + (long)(nb - 1) * bs;
+  const double *sub = values + voff[sys] + (long)nb * (N * N);
+  const double *sup = sub + (long)(nb - 1) * N;
 
-  // sweep towards the middle; y_i is kept in X
-  const int len = top ? m : nb - 1 - m;
-  double y = 0.;
-  for (int t = 0; t < len; ++t) {
-    const int i = top ? t : nb - 1 - t;
-    const double bi = act ? b[(long)i * bs + lane] : 0.;
-    if (t == 0) {
-      y = bi;
-    } else {
-      const int prev = top ? i - 1 : i + 1;
-      const double mv = wave_matvec(DI + prev * nb2, bs, y, lane);
-      const double cpl = act ? (top ? sub[(long)(i - 1) * bs + lane] : sup[(long)i * bs + lane]) : 0.;
-      y = bi - cpl * mv;
+  // What a product needs: the block's columns of this wave (e: those beyond the groups of four, for wave 0), and the two
+  // vectors a, c that form the next product's vector a - c * (this product). y_i is kept in X. Every product loads the same
+  // number of words without a branch (clamped where there is nothing to load), so that a wait counts the loads it
+  // needs and leaves the later products' in flight.
+  struct Ahead {
+    T d[K > 0 ? K : 1], e[E > 0 ? E : 1];
+    double a, c;
+  };
+  auto columns = [&](Ahead &B, int blk) {
+    const T *D = DI + (long)blk * (N * N);
+#pragma unroll
+    for (int k = 0; k < E; ++k) B.e[k] = D[(4 * K + k) * N];
+    D += q * N;
+#pragma unroll
+    for (int k = 0; k < K; ++k) B.d[k] = D[4 * k * N];
+  };
+  double v;
+  auto multiply = [&](const Ahead &B, double *out) {
+    double acc = 0.;
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc = fma((double)B.d[k], lane_value(v, 4 * k + q), acc);
+    if (E > 0 && q == 0) {
+#pragma unroll
+      for (int k = 0; k < E; ++k) acc = fma((double)B.e[k], lane_value(v, 4 * K + k), acc);
     }
-    if (act) X[(long)i * bs + lane] = y;
+    out[lane] = acc;
+  };
+  auto sum = [&](const double (*p)[64]) { return (p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane]); };
+  if (nb == 1) {
+    Ahead B;
+    v = b[rl];
+    columns(B, 0);
+    multiply(B, part[0][0][q]);
+    __syncthreads();
+    if (q == 0 && act) X[lane] = sum(part[0][0]);
+    return;
   }
-  // this wave's term of the middle equation
-  double term = 0.;
-  if (len > 0) {
-    const int prev = top ? m - 1 : m + 1;
-    const double mv = wave_matvec(DI + prev * nb2, bs, y, lane);
-    term = act ? (top ? sub[(long)(m - 1) * bs + lane] : sup[(long)m * bs + lane]) * mv : 0.;
+
+  // Both chains run L products inwards, the middle one and L outwards; a top chain that is one shorter waits for one at
+  // either end (off). Product s of a chain is with the block of its place len - |len - s|, the next one's coupling is that
+  // between the two blocks, row min of the two of sub or sup.
+  const int L = nb - 1 - m;
+  const int len = top ? m : L, off = L - len;
+  const int first = top ? 0 : nb - 1, dir = top ? 1 : -1;
+  auto block = [&](int s) { return first + dir * max(len - abs(len - s), 0); };
+  auto at = [&](int i) { return (unsigned)(i * N + rl); };
+  const double bm = b[at(m)], ct = m > 0 ? sub[at(m - 1)] : 0., cb = sup[at(m)];
+  double last = 0.;
+  v = b[at(block(0))];
+  if (len > 0 && act) X[at(block(0))] = v;  // every wave writes, and later reads, its own
+  auto operands = [&](Ahead &B, int s) {
+    const int i = block(s), j = block(s + 1);
+    columns(B, i);
+    B.c = (top == (s < len) ? sub : sup)[at(min(min(i, j), nb - 2))];
+  };
+  auto addend = [&](Ahead &B, int s) { B.a = (s < len ? b : X)[at(block(s + 1))]; };
+  Ahead buf[kAhead<T>];
+#pragma unroll
+  for (int k = 0; k < kAhead<T>; ++k) {
+    operands(buf[k], max(k - off, 0));
+    addend(buf[k], max(k - off, 0));
   }
-  mid[top ? 0 : 1][lane] = term;
-  __syncthreads();
-  double xm = 0.;
-  {
-    const double r = act ? b[(long)m * bs + lane] - mid[0][lane] - mid[1][lane] : 0.;
-    xm = wave_matvec(DI + m * nb2, bs, r, lane);  // both waves form x_m (no second exchange)
+
+  const bool out = act && q == 0;
+  auto product = [&](Ahead &B, int g) {
+    const int s = g - off;
+    multiply(B, part[g & 1][chain][q]);
+    // Loads that do not depend on this product go before the barrier. The addend has to be here by then: x may be rhs, and
+    // behind the barrier other waves write what it was read from.
+    const double a = s == len ? last : B.a, c = B.c;
+    asm volatile("" ::"v"(B.a));
+    operands(B, s + kAhead<T>);
+    __syncthreads();
+    if (g == L - 1) {
+#pragma clang fp contract(off)
+      const double tt = m > 0 ? ct * sum(part[g & 1][0]) : 0., tb = cb * sum(part[g & 1][1]);
+      last = v;
+      v = bm - tt - tb;
+    } else if ((unsigned)s <= (unsigned)(2 * len)) {
+      const bool in = s < len;
+      const double mv = sum(part[g & 1][chain]);
+      v = fma(-c, mv, a);
+      // y of the next block or x of this one (both chains write x_m, the same)
+      if (in ? act : out) X[at(block(in ? s + 1 : s))] = in ? v : mv;
+    }
+    addend(B, s + kAhead<T>);
+  };
+  for (int g = 0; g <= 2 * L; g += kAhead<T>) {
+#pragma unroll
+    for (int k = 0; k < kAhead<T>; ++k) {
+      if (g + k > 2 * L) break;
+      product(buf[k], g + k);
+    }
   }
-  if (top && act) X[(long)m * bs + lane] = xm;
-  // sweep outwards
-  double xn = xm;
-  for (int t = len - 1; t >= 0; --t) {
-    const int i = top ? t : nb - 1 - t;
-    const double yi = act ? X[(long)i * bs + lane] : 0.;
-    const double cpl = act ? (top ? sup[(long)i * bs + lane] : sub[(long)(i - 1) * bs + lane]) : 0.;
-    xn = wave_matvec(DI + i * nb2, bs, yi - cpl * xn, lane);
-    if (act) X[(long)i * bs + lane] = xn;
-  }
+}
+
+template <typename T>
+using InvSolve = void (*)(const int *, const double *, const long *, const T *, const long *, const double *, double *,
+                          const long *);
+template <typename T, int... I>
+InvSolve<T> inv_solve_kernel(int bs, std::integer_sequence<int, I...>) {
+  constexpr InvSolve<T> tab[] = {&btd_twist_solve_kernel<T, I + 1>...};
+  return tab[bs - 1];
 }
 
 }  // namespace
@@ -396,8 +432,8 @@ int launch_btd_inv_solve(int nsys, const int *nblocks, int bs, const double *val
                          hipStream_t st) {
   if (nsys <= 0) return GF_OK;
   if (bs < 1 || bs > 64) return fail(GF_ERR_UNSUPPORTED, "block size must be in 1..64");
-  hipLaunchKernelGGL(btd_twist_solve_kernel<T>, dim3(nsys), dim3(128), 0, st, nsys, nblocks, bs, values, voff, dinv,
-                     doff, rhs, x, xoff);
+  const auto kern = inv_solve_kernel<T>(bs, std::make_integer_sequence<int, 64>{});
+  hipLaunchKernelGGL(kern, dim3(nsys), dim3(512), 0, st, nblocks, values, voff, dinv, doff, rhs, x, xoff);
   if (hipGetLastError() != hipSuccess) return fail(GF_ERR_HIP, "btd inverse solve launch failed");
   return GF_OK;
 }

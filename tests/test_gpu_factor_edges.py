@@ -93,3 +93,50 @@ def test_inverse_factor_routes_are_bitwise_the_same(bs, precision):
         for k in (0, 229):
             a, b = few[s], many[s + k * len(sizes)]
             assert np.array_equal(np.isfinite(a), np.isfinite(b)) and np.array_equal(a[np.isfinite(a)], b[np.isfinite(b)])
+
+
+@pytest.mark.parametrize('precision', [64, 32])
+@pytest.mark.parametrize('bs', [1, 3, 4, 5, 13, 52, 53, 63, 64])
+def test_inverse_solve_edges(bs, precision):
+    """Block sizes around the four columns of a group and chains from one block to some more than the loads in flight, the
+    right-hand side apart from and in place of the solution, against the dense system. Tolerance: the residual of a solve with
+    diagonally dominant blocks, 100 N eps of the inverses' precision (FP64) times the norm, 10 times that for the chain."""
+    import torch
+    from spitfire_amd import _native
+    rng = np.random.default_rng(bs)
+    sizes = [1, 2, 3, 4, 5, 6, 9, 12] + [1] * 3
+    values, dense, rhs = [], [], []
+    for n in sizes:
+        V = rng.standard_normal((n, bs, bs)) + (4. + 2. * np.sqrt(bs)) * np.eye(bs)
+        lo, up = 0.1 * rng.standard_normal((n - 1, bs)), 0.1 * rng.standard_normal((n - 1, bs))
+        values.append(np.concatenate([V.transpose(0, 2, 1).ravel(), lo.ravel(), up.ravel()]))
+        A = np.zeros((n * bs, n * bs))
+        for k in range(n):
+            A[k * bs:(k + 1) * bs, k * bs:(k + 1) * bs] = V[k]
+        for k in range(n - 1):
+            A[(k + 1) * bs:(k + 2) * bs, k * bs:(k + 1) * bs] = np.diag(lo[k])
+            A[k * bs:(k + 1) * bs, (k + 1) * bs:(k + 2) * bs] = np.diag(up[k])
+        dense.append(A)
+        rhs.append(rng.standard_normal(n * bs))
+    dev = torch.device('cuda:0')
+    nb = np.asarray(sizes)
+    offsets = [np.cumsum(np.r_[0, a])[:-1].astype(np.int64) for a in ([v.size for v in values], nb * bs * bs, nb * bs)]
+    V, b = (torch.tensor(np.concatenate(a), device=dev) for a in (values, rhs))
+    D = torch.zeros(int((nb * bs * bs).sum()), device=dev, dtype=torch.float64 if precision == 64 else torch.float32)
+    n, vo, do, xo = (torch.tensor(a, device=dev) for a in (nb.astype(np.int32), *offsets))
+    x = torch.zeros_like(b)
+    st = torch.cuda.current_stream().cuda_stream
+    lib = _native.lib()
+    _native.check(lib.gf_batch_btddod_inverse_factorize(len(sizes), n.data_ptr(), bs, V.data_ptr(), vo.data_ptr(),
+                                                        D.data_ptr(), do.data_ptr(), precision, st))
+    in_place = b.clone()
+    for r, out in ((b, x), (in_place, in_place)):
+        _native.check(lib.gf_batch_btddod_inverse_solve(len(sizes), n.data_ptr(), bs, V.data_ptr(), vo.data_ptr(),
+                                                        D.data_ptr(), do.data_ptr(), precision, r.data_ptr(),
+                                                        out.data_ptr(), xo.data_ptr(), st))
+    assert torch.equal(x, in_place)
+    got = x.cpu().numpy()
+    tol = 1e3 * bs * (2.2e-16 if precision == 64 else 6.0e-8)
+    for s in range(len(sizes)):
+        g = got[offsets[2][s]:offsets[2][s] + nb[s] * bs]
+        assert np.max(np.abs(dense[s] @ g - rhs[s])) <= tol * np.max(np.abs(rhs[s]))
