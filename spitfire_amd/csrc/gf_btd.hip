@@ -30,203 +30,277 @@ namespace {
 
 using wave::lane_value;
 
-constexpr int BW = 64;
-constexpr int BT_THREADS = 256;
+// ---------------- block Thomas with LAPACK's factors ----------------
 
-// LU with partial pivoting of a bs x bs column-major block in LDS (LAPACK dgetf2 order of operations).
-template <typename T>
-__device__ void lds_lu(T *A, int bs, int *piv_lds, int *gpiv) {
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  __shared__ int s_p;
-  for (int j = 0; j < bs; ++j) {
-    if (wave == 0) {
-      double v = -1.0;
-      int idx = bs;
-      if (lane >= j && lane < bs) { v = fabs((double)A[j * bs + lane]); idx = lane; }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const double ov = __shfl_xor(v, o, 64);
-        const int oi = __shfl_xor(idx, o, 64);
-        if (ov > v || (ov == v && oi < idx)) { v = ov; idx = oi; }
-      }
-      if (idx >= bs) idx = j;  // no comparable pivot candidate (NaN column): keep the diagonal
-      if (lane == 0) {
-        s_p = idx;
-        piv_lds[j] = idx + 1;
-        if (gpiv) gpiv[j] = idx + 1;
-      }
-    }
-    __syncthreads();
-    const int p = s_p;
-    if (p != j)
-      for (int c = t; c < bs; c += BT_THREADS) {
-        const T a0 = A[c * bs + j];
-        A[c * bs + j] = A[c * bs + p];
-        A[c * bs + p] = a0;
-      }
-    __syncthreads();
-    const T d = A[j * bs + j];
-    if (d != T(0)) {
-      const T id = T(1) / d;
-      for (int k = j + 1 + t; k < bs; k += BT_THREADS) A[j * bs + k] *= id;
-    }
-    __syncthreads();
-    const int m = bs - j - 1;
-    for (int e = t; e < m * m; e += BT_THREADS) {
-      const int c = j + 1 + e / m, k = j + 1 + e % m;
-      A[c * bs + k] -= A[j * bs + k] * A[c * bs + j];
-    }
-    __syncthreads();
-  }
-}
+constexpr int kLuWaves = 8;
 
-// X <- A^{-1} X for bs right-hand sides, A an LU factorization with pivots in LDS (LAPACK dgetrs, 'N').
-template <typename T>
-__device__ void lds_lu_solve_multi(const T *A, const int *piv, int bs, T *X) {
-  const int t = threadIdx.x;
-  for (int j = 0; j < bs; ++j) {  // row interchanges, applied in order
-    const int p = piv[j] - 1;
-    if (p != j)
-      for (int c = t; c < bs; c += BT_THREADS) {
-        const T a0 = X[c * bs + j];
-        X[c * bs + j] = X[c * bs + p];
-        X[c * bs + p] = a0;
-      }
-    __syncthreads();
-  }
-  for (int j = 0; j < bs; ++j) {  // unit lower triangular
-    const int m = bs - j - 1;
-    for (int e = t; e < m * bs; e += BT_THREADS) {
-      const int c = e / m, k = j + 1 + e % m;
-      X[c * bs + k] -= A[j * bs + k] * X[c * bs + j];
-    }
-    __syncthreads();
-  }
-  for (int j = bs - 1; j >= 0; --j) {  // upper triangular
-    for (int c = t; c < bs; c += BT_THREADS) X[c * bs + j] /= A[j * bs + j];
-    __syncthreads();
-    for (int e = t; e < j * bs; e += BT_THREADS) {
-      const int c = e / j, k = e % j;
-      X[c * bs + k] -= A[j * bs + k] * X[c * bs + j];
-    }
-    __syncthreads();
-  }
-}
-
-// Factors of system sys: D blocks to dout + doff[sys] (for FP64 the values array itself, in place), L blocks to
-// lout + loff[sys]; the input blocks and off-diagonals are the FP64 values array.
-template <typename T>
-__global__ void __launch_bounds__(BT_THREADS) btd_factor_kernel(const int *nblocks, int bs, double *values,
-                                                               const long *voff, T *dout, const long *doff, T *lout,
-                                                               const long *loff, int *piv, const long *poff) {
-  extern __shared__ double sm_raw[];
-  T *sm = reinterpret_cast<T *>(sm_raw);
+// Factors of one system per workgroup: LU with partial pivoting of every diagonal block (LAPACK dgetf2's order of operations,
+// interchanges as dgetrf returns them), in place in values; the L blocks sub_{i-1} D_{i-1}^{-1}, to l; and the
+// pivots. A block is in registers, lane = row, wave w of eight holding columns w, 8 + w, .. (C of them) of it (a) and of what
+// becomes its inverse (x, the identity at first, eliminated along with it). Rows stay in their lanes: `cur` is the
+// position that LAPACK's interchanges have given a row, and where they end is the next block's order of rows.
+// What bounds it is the chain of pivots, blocks after blocks: the wave with column j searches it, publishes the
+// multipliers in LDS, and one barrier later all waves update their columns. The next column's owner does that column first
+// and searches it before its other ones. The back substitution of the inverse needs no barrier: every wave has the
+// columns of U that it wants from LDS, scaled by the reciprocal pivots (so the inverse's rows are scaled once at the end,
+// instead of a division for every entry). The next block's values are loaded while a block is factored. Before, a block in
+// LDS took four barriers a pivot, two more and a division for the substitutions. About 1,000 cycles a pivot now: the two LDS words, the update,
+// search and reciprocal of one column and the way back, one after the other. Measured before and after (us): one
+// system of 60 blocks of 53 10,450 -> 2,260, 24 of 30..61 9,960 -> 2,160, 2,000 of 2..4 1,840 -> 690; 24 of 24x24 blocks
+// 2,850 -> 805, of 10x10 1,050 -> 346. Putting a searching wave's other columns off behind the next barrier gained nothing.
+template <int C>
+__global__ void __launch_bounds__(64 * kLuWaves) btd_factor_kernel(const int *nblocks, int bs, double *values,
+                                                                   const long *voff, double *lout, const long *loff,
+                                                                   int *piv, const long *poff) {
+  __shared__ double A[8 * C][64], gb[2][64];  // columns of U for the substitution, [column][lane]; what a step publishes, by
+  __shared__ int pb[2];                       // parity of the step
   const int sys = blockIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nb = nblocks[sys];
-  const int nb2 = bs * bs;
-  const double *V = values + voff[sys];
-  T *Dg = dout + doff[sys];
-  T *L = lout + loff[sys];
+  const long nb2 = (long)bs * bs;
+  double *V = values + voff[sys];
+  double *L = lout + loff[sys];
   int *P = piv + poff[sys];
-  const double *sub = V + (long)nb * nb2;
+  const double *sub = V + nb * nb2;
   const double *sup = sub + (long)(nb - 1) * bs;
-  T *D = sm, *Lb = sm + nb2;                // factored diagonal block, L block
-  int *pv = reinterpret_cast<int *>(sm + 2 * nb2);
-  const int t = threadIdx.x;
-
-  for (int e = t; e < nb2; e += BT_THREADS) D[e] = (T)V[e];
-  __syncthreads();
-  lds_lu(D, bs, pv, P);
-  for (int e = t; e < nb2; e += BT_THREADS) Dg[e] = D[e];
-  for (int i = 1; i < nb; ++i) {
-    const long o1 = (long)i * nb2;
-    for (int e = t; e < nb2; e += BT_THREADS) Lb[e] = ((e % bs) == (e / bs)) ? T(1) : T(0);
-    __syncthreads();
-    lds_lu_solve_multi(D, pv, bs, Lb);  // Lb = D_{i-1}^{-1}
-    const int b1 = (i - 1) * bs;
-    for (int e = t; e < nb2; e += BT_THREADS) {
-      const int j = e / bs, k = e % bs;
-      const T l = Lb[e] * (T)sub[b1 + k];
-      L[o1 + e] = l;
-      D[e] = (T)(V[o1 + e] + (-sup[b1 + j]) * (double)l);
+  const bool act = lane < bs;
+  const int rl = act ? lane : 0;
+  int cur = act ? lane : -1;
+  double a[C], x[C], v[C], idl = 0.;
+  int pivot = 0, row_of = 0;  // of step = lane: LAPACK's interchange, and the lane of the row
+  auto load = [&](double(&to)[C], const double *from) {
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      const double t = from[min(8 * k + w, bs - 1) * bs + rl];
+      to[k] = act && 8 * k + w < bs ? t : 0.;
     }
+  };
+  // pivot of column j = f: the multipliers (the reciprocal for the pivot row) and its lane to LDS; returns the column as the
+  // factors have it
+  auto publish = [&](double f, int j) {
+    const bool cand = cur >= j;
+    const unsigned key = cand & (f == f) ? (unsigned)__double2hiint(f) & 0x7fffffffu : 0u;
+    unsigned most = key;
+    auto rc = wave::recip_of(f);
+    rc.template step<0>(); most = wave::max_step<0>(most);
+    rc.template step<1>(); most = wave::max_step<1>(most);
+    rc.template step<2>(); most = wave::max_step<2>(most);
+    rc.template step<3>(); most = wave::max_step<3>(most);
+    rc.template step<4>(); most = wave::max_step<4>(most);
+    rc.template step<5>(); most = wave::max_step<5>(most);
+    rc.template step<6>();
+    const unsigned top = (unsigned)__builtin_amdgcn_readlane((int)most, 63);
+    unsigned long long hit = __ballot(key == top);
+    if (hit & (hit - 1)) {  // rare: the low words decide, then the position
+      const bool in = cand & (key == top);
+      const unsigned lo = in & (f == f) ? (unsigned)__double2loint(f) : 0u;
+      const unsigned big = wave::dpp_wave_max_u32(lo);
+      const unsigned at = in & (lo == big) ? 64u - (unsigned)cur : 0u;
+      const unsigned low = wave::dpp_wave_max_u32(at);
+      hit = __ballot(in & (at == low));
+    }
+    const int p = __builtin_ctzll(hit);
+    const double id = lane_value(rc.r, p);
+    const double l = f * (top != 0u || lane_value(f, p) != 0. ? id : 1.);
+    const bool below = cand & (lane != p);
+    gb[j & 1][lane] = lane == p ? id : below ? l : 0.;
+    pb[j & 1] = p;
+    return below ? l : f;
+  };
+  load(a, V);
+  for (int i = 0; i < nb; ++i) {
+    asm volatile("" : "+s"(bs));  // opaque: addresses and conditions are formed anew rather than kept (and spilled)
+    double subv = 0., supv = 0.;
+    if (i + 1 < nb) {
+      load(v, V + (i + 1) * nb2);
+      subv = sub[(long)i * bs + rl];
+      supv = sup[(long)i * bs + rl];
+    }
+#pragma unroll
+    for (int k = 0; k < C; ++k) x[k] = cur == 8 * k + w ? 1. : 0.;
+    if (w == 0) a[0] = publish(a[0], 0);
+    double l = 0.;
+    int p = 0;
+    auto begin = [&](int j) {
+      __syncthreads();
+      p = __builtin_amdgcn_readfirstlane(pb[j & 1]);
+      const double g = gb[j & 1][lane];
+      l = lane == p ? 0. : g;
+      const int at = __builtin_amdgcn_readlane(cur, p);
+      idl = lane == p ? g : idl;
+      pivot = lane == j ? at + 1 : pivot;
+      row_of = lane == j ? p : row_of;
+      cur = lane == p ? j : cur == j ? at : cur;
+    };
+    auto update = [&](double &y) { y = fma(-l, lane_value(y, p), y); };
+    auto rest = [&](int after) {
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        if (c > after) update(a[c]);
+        update(x[c]);
+      }
+    };
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+#pragma unroll 1
+      for (int q = 0; q < 7; ++q) {
+        const int j = 8 * k + q;
+        if (j >= bs) break;
+        begin(j);
+        if (w > q) update(a[k]);
+        if (w == q + 1 && j + 1 < bs) a[k] = publish(a[k], j + 1);
+        rest(k);
+      }
+      const int j = 8 * k + 7;
+      if (j < bs) {
+        begin(j);
+        constexpr int last = C - 1;
+        if (k < last) update(a[k < last ? k + 1 : last]);
+        if (w == 0 && j + 1 < bs) a[k < last ? k + 1 : last] = publish(a[k < last ? k + 1 : last], j + 1);
+        rest(k + 1);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      if (act && 8 * k + w < bs) V[i * nb2 + (8 * k + w) * bs + cur] = a[k];
+      // (the reciprocal is its row's; rows at and below the diagonal have no part in the substitution)
+      const double id = lane_value(idl, __builtin_amdgcn_readlane(row_of, 8 * k + w));
+      A[8 * k + w][lane] = cur < 8 * k + w ? a[k] * id : 0.;
+    }
+    if (w == 0 && act) P[(long)i * bs + lane] = pivot;
+    if (i + 1 == nb) break;
     __syncthreads();
-    lds_lu(D, bs, pv, P + i * bs);
-    for (int e = t; e < nb2; e += BT_THREADS) Dg[o1 + e] = D[e];
+#pragma unroll 4
+    for (int j = bs - 1; j >= 0; --j) {
+      p = __builtin_amdgcn_readlane(row_of, j);
+      l = A[j][lane];
+#pragma unroll
+      for (int c = 0; c < C; ++c) update(x[c]);
+    }
+    const double subr = __shfl(subv, cur, 64);
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      const int c = 8 * k + w;
+      const double lx = x[k] * idl * subr;
+      if (act && c < bs) L[(i + 1) * nb2 + c * bs + cur] = lx;
+      const double up = lane_value(supv, min(c, 63));
+      a[k] = act && c < bs ? fma(-up, lx, __shfl(v[k], cur, 64)) : 0.;
+    }
   }
 }
 
-// One wave per system, lane = row; each block is staged in LDS with one coalesced load before it is used.
-// FP64 arithmetic; FP32 factors are widened on load.
-template <typename T>
-__global__ void __launch_bounds__(BW) btd_solve_kernel(int nsys, const int *nblocks, int bs, const double *values,
-                                                      const long *voff, const T *dfac, const long *doff,
-                                                      const T *lval, const long *loff, const int *piv,
-                                                      const long *poff, const double *rhs, double *x,
-                                                      const long *xoff) {
-  extern __shared__ double sm_raw[];
-  T *Bk = reinterpret_cast<T *>(sm_raw);
-  int *pvs = reinterpret_cast<int *>(Bk + bs * bs);
+// Solve with these factors, one workgroup per system. Wave 0 runs the chain, lane = row, with the columns of a block in
+// registers (NC >= bs of them; those beyond are zero) and the next block's on their way:
+//   y_i = b_i - L_i y_{i-1}, forward;  x_i = D_i^{-1} (y_i - sup_i x_{i+1}), backward: interchanges, unit lower, upper.
+// What bounds it is the substitutions: a broadcast through scalar registers and a fused multiply-add for every column, for the
+// upper one the division as well. Wave 1 prepares the next block meanwhile: the interchanges as one permutation, and
+// the reciprocals of U's diagonal, so that a division is a product and one correction step. Before, blocks were
+// staged in LDS by the wave that used them, interchanges were 53 shuffles of the vector one after the other and
+// divisions whole. Measured before and after (us): 24 systems of 30..61 blocks of 53 2,460 -> 296, 2,000 of 2..4 268 -> 91;
+// solutions are bitwise the same.
+template <int NC>
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1)))
+btd_solve_kernel(const int *nblocks, int bs, const double *factors, const long *voff, const double *lval, const long *loff,
+                 const int *piv, const long *poff, const double *rhs, double *x, const long *xoff) {
+  __shared__ double diag[2][64], inverse[2][64];
+  __shared__ int order[2][64];
   const int sys = blockIdx.x;
-  if (sys >= nsys) return;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   const int nb = nblocks[sys];
-  const int nb2 = bs * bs;
-  const double *V = values + voff[sys];
-  const T *DF = dfac + doff[sys];
-  const T *L = lval + loff[sys];
-  const int *P = piv + poff[sys];
+  const long nb2 = (long)bs * bs;
+  const double *D = factors + voff[sys];
+  const bool act = lane < bs;
+  const int rl = act ? lane : 0;
+  if (threadIdx.x >= 64) {
+    const int *P = piv + poff[sys];
+    for (int i = nb - 1; i >= 0; --i) {
+      const int p = act ? (P[(long)i * bs + lane] - 1) & 63 : lane;
+      const double u = act ? D[i * nb2 + lane * bs + lane] : 1.;
+      int from = lane;
+      for (int j = 0; j < bs; ++j) {
+        const int q = __builtin_amdgcn_readlane(p, j);
+        if (q != j) {
+          const int a = __builtin_amdgcn_readlane(from, j), b = __builtin_amdgcn_readlane(from, q);
+          from = lane == j ? b : lane == q ? a : from;
+        }
+      }
+      order[i & 1][lane] = from;
+      diag[i & 1][lane] = u;
+      inverse[i & 1][lane] = 1. / u;
+      __syncthreads();  // block i is ready, and i + 1 done with
+    }
+    return;
+  }
+  const double *L = lval + loff[sys];
   const double *b = rhs + xoff[sys];
   double *X = x + xoff[sys];
-  const double *sup = V + (long)nb * nb2 + (long)(nb - 1) * bs;
-  const bool act = lane < bs;
+  const double *sup = D + nb * nb2 + (long)(nb - 1) * bs;
+  double B[2][NC];
+  auto load = [&](double(&to)[NC], const double *from) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) to[c] = from[min(c, bs - 1) * bs + rl];
+  };
+  auto column = [&](const double(&of)[NC], int c, bool in) { return in & (c < bs) ? of[c] : 0.; };
 
-  // forward: y_i = b_i - L_i y_{i-1}; y kept in X
   double y = act ? b[lane] : 0.;
   if (act) X[lane] = y;
-  for (int i = 1; i < nb; ++i) {
-    const T *Li = L + (long)i * nb2;
-    for (int e = lane; e < nb2; e += BW) Bk[e] = Li[e];
-    __syncthreads();
-    double yi = act ? b[(long)i * bs + lane] : 0.;
-    for (int c = 0; c < bs; ++c) {
-      const double yc = __shfl(y, c, 64);
-      if (act) yi = yi + (double)Bk[c * bs + lane] * (-1. * yc);
-    }
-    y = yi;
+  auto forward = [&](const double(&of)[NC], int i, double bi) {
+    double t = act ? bi : 0.;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) t = fma(column(of, c, act), -lane_value(y, c), t);
+    y = t;
     if (act) X[(long)i * bs + lane] = y;
-    __syncthreads();
+  };
+  if (nb > 1) {
+    load(B[0], L + nb2);
+    double b0 = b[bs + rl], b1 = 0.;
+    for (int i = 1; i < nb; i += 2) {
+      const int n1 = min(i + 1, nb - 1), n2 = min(i + 2, nb - 1);
+      load(B[1], L + n1 * nb2);
+      b1 = b[(long)n1 * bs + rl];
+      forward(B[0], i, b0);
+      if (i + 1 == nb) break;
+      load(B[0], L + n2 * nb2);
+      b0 = b[(long)n2 * bs + rl];
+      forward(B[1], i + 1, b1);
+    }
   }
-  // backward
   double xn = 0.;
-  for (int i = nb - 1; i >= 0; --i) {
-    const T *Dg = DF + (long)i * nb2;
-    for (int e = lane; e < nb2; e += BW) Bk[e] = Dg[e];
-    if (act) pvs[lane] = P[i * bs + lane];
+  auto backward = [&](const double(&of)[NC], int i, double yi, double s) {
     __syncthreads();
-    double r = act ? X[(long)i * bs + lane] : 0.;
-    if (i < nb - 1 && act) r = r - sup[(long)i * bs + lane] * xn;
-    for (int j = 0; j < bs; ++j) {  // row interchanges
-      const int p = pvs[j] - 1;
-      if (p != j) {
-        const double vj = __shfl(r, j, 64), vp = __shfl(r, p, 64);
-        if (lane == j) r = vp;
-        else if (lane == p) r = vj;
-      }
-    }
-    for (int j = 0; j < bs; ++j) {  // unit lower
-      const double rj = __shfl(r, j, 64);
-      if (act && lane > j) r -= (double)Bk[j * bs + lane] * rj;
-    }
-    for (int j = bs - 1; j >= 0; --j) {  // upper
-      if (lane == j) r /= (double)Bk[j * bs + j];
-      const double rj = __shfl(r, j, 64);
-      if (act && lane < j) r -= (double)Bk[j * bs + lane] * rj;
+    const int from = order[i & 1][lane];
+    const double u = diag[i & 1][lane], v = inverse[i & 1][lane];
+    double r = i == nb - 1 ? yi : fma(-s, xn, yi);
+    r = act ? r : 0.;
+    r = __shfl(r, from, 64);
+    int ln = lane;
+    asm volatile("" : "+v"(ln));  // opaque: the comparisons below are not kept (and spilled) over the blocks
+#pragma unroll
+    for (int j = 0; j < NC; ++j) r = fma(-column(of, j, ln > j), lane_value(r, j), r);
+#pragma unroll
+    for (int j = NC - 1; j >= 0; --j) {
+      double q = r * v;
+      q = fma(fma(-u, q, r), v, q);
+      r = ln == j ? q : r;
+      r = fma(-column(of, j, ln < j), lane_value(q, j), r);
     }
     xn = r;
     if (act) X[(long)i * bs + lane] = r;
-    __syncthreads();
+  };
+  load(B[0], D + (nb - 1) * nb2);
+  double y0 = y, y1 = 0., s0 = 0., s1 = 0.;
+  for (int i = nb - 1; i >= 0; i -= 2) {
+    const int n1 = max(i - 1, 0), n2 = max(i - 2, 0);
+    load(B[1], D + n1 * nb2);
+    y1 = X[(long)n1 * bs + rl];
+    s1 = sup[(long)n1 * bs + rl];
+    backward(B[0], i, y0, s0);
+    if (i == 0) break;
+    load(B[0], D + n2 * nb2);
+    y0 = X[(long)n2 * bs + rl];
+    s0 = sup[(long)n2 * bs + rl];
+    backward(B[1], i - 1, y1, s1);
   }
 }
 
@@ -384,44 +458,37 @@ InvSolve<T> inv_solve_kernel(int bs, std::integer_sequence<int, I...>) {
 
 }  // namespace
 
+template <int... I>
+static auto factor_kernel(int c, std::integer_sequence<int, I...>) {
+  constexpr decltype(&btd_factor_kernel<1>) tab[] = {&btd_factor_kernel<I + 1>...};
+  return tab[c - 1];
+}
+
 int launch_btd_factor(int nsys, const int *nblocks, int bs, double *values, const long *voff, double *l_values,
                       const long *loff, int *pivots, const long *poff, hipStream_t st) {
-  return launch_btd_factor_t<double>(nsys, nblocks, bs, values, voff, values, voff, l_values, loff, pivots, poff, st);
+  if (nsys <= 0) return GF_OK;
+  if (bs < 1 || bs > 64) return fail(GF_ERR_UNSUPPORTED, "block size must be in 1..64");
+  const auto kern = factor_kernel((bs + 7) / 8, std::make_integer_sequence<int, 8>{});
+  hipLaunchKernelGGL(kern, dim3(nsys), dim3(64 * kLuWaves), 0, st, nblocks, bs, values, voff, l_values, loff, pivots,
+                     poff);
+  if (hipGetLastError() != hipSuccess) return fail(GF_ERR_HIP, "btd factor launch failed");
+  return GF_OK;
+}
+
+template <int... I>
+static auto solve_kernel(int c, std::integer_sequence<int, I...>) {
+  constexpr decltype(&btd_solve_kernel<8>) tab[] = {&btd_solve_kernel<8 * (I + 1)>...};
+  return tab[c - 1];
 }
 
 int launch_btd_solve(int nsys, const int *nblocks, int bs, const double *values, const long *voff,
                      const double *l_values, const long *loff, const int *pivots, const long *poff, const double *rhs,
                      double *x, const long *xoff, hipStream_t st) {
-  return launch_btd_solve_t<double>(nsys, nblocks, bs, values, voff, values, voff, l_values, loff, pivots, poff, rhs,
-                                    x, xoff, st);
-}
-
-template <typename T>
-int launch_btd_factor_t(int nsys, const int *nblocks, int bs, double *values, const long *voff, T *dfac,
-                        const long *doff, T *l_values, const long *loff, int *pivots, const long *poff,
-                        hipStream_t st) {
   if (nsys <= 0) return GF_OK;
   if (bs < 1 || bs > 64) return fail(GF_ERR_UNSUPPORTED, "block size must be in 1..64");
-  const size_t lds = sizeof(T) * 2 * bs * bs + sizeof(int) * 64 + 16;
-  auto kern = btd_factor_kernel<T>;
-  if (lds > 65536)
-    if (hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-      return fail(GF_ERR_UNSUPPORTED, "block too large for LDS");
-  hipLaunchKernelGGL(kern, dim3(nsys), dim3(BT_THREADS), lds, st, nblocks, bs, values, voff, dfac, doff, l_values,
-                     loff, pivots, poff);
-  if (hipGetLastError() != hipSuccess) return fail(GF_ERR_HIP, "btd factor launch failed");
-  return GF_OK;
-}
-
-template <typename T>
-int launch_btd_solve_t(int nsys, const int *nblocks, int bs, const double *values, const long *voff, const T *dfac,
-                       const long *doff, const T *l_values, const long *loff, const int *pivots, const long *poff,
-                       const double *rhs, double *x, const long *xoff, hipStream_t st) {
-  if (nsys <= 0) return GF_OK;
-  if (bs < 1 || bs > 64) return fail(GF_ERR_UNSUPPORTED, "block size must be in 1..64");
-  const size_t lds = sizeof(T) * bs * bs + sizeof(int) * 64 + 16;
-  hipLaunchKernelGGL(btd_solve_kernel<T>, dim3(nsys), dim3(BW), lds, st, nsys, nblocks, bs, values, voff, dfac, doff,
-                     l_values, loff, pivots, poff, rhs, x, xoff);
+  const auto kern = solve_kernel((bs + 7) / 8, std::make_integer_sequence<int, 8>{});
+  hipLaunchKernelGGL(kern, dim3(nsys), dim3(128), 0, st, nblocks, bs, values, voff, l_values, loff, pivots, poff, rhs, x,
+                     xoff);
   if (hipGetLastError() != hipSuccess) return fail(GF_ERR_HIP, "btd solve launch failed");
   return GF_OK;
 }
@@ -442,10 +509,5 @@ template int launch_btd_inv_solve<double>(int, const int *, int, const double *,
                                           const long *, const double *, double *, const long *, hipStream_t);
 template int launch_btd_inv_solve<float>(int, const int *, int, const double *, const long *, const float *,
                                          const long *, const double *, double *, const long *, hipStream_t);
-template int launch_btd_factor_t<float>(int, const int *, int, double *, const long *, float *, const long *, float *,
-                                        const long *, int *, const long *, hipStream_t);
-template int launch_btd_solve_t<float>(int, const int *, int, const double *, const long *, const float *,
-                                       const long *, const float *, const long *, const int *, const long *,
-                                       const double *, double *, const long *, hipStream_t);
 
 }  // namespace gfa

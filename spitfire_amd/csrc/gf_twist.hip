@@ -48,6 +48,8 @@ namespace gfa {
 namespace {
 
 using wave::lane_value;
+using wave::max_step;
+using wave::recip_of;
 
 template <typename T>
 using Vec4 = T __attribute__((ext_vector_type(4)));
@@ -63,13 +65,6 @@ __device__ __forceinline__ Vec4<float> mfma4(float a, float b, Vec4<float> c) {
 // holds the exponent under its mask, which is 0 once the row is used.
 __device__ __forceinline__ unsigned key_of(double f, unsigned mask) { return (unsigned)__double2hiint(f) & mask; }
 __device__ __forceinline__ unsigned key_of(float f, unsigned mask) { return (unsigned)__float_as_int(f) & mask; }
-// step k = 0 .. 5 of the wave-wide maximum, complete in lane 63 after step 5
-template <int K>
-__device__ __forceinline__ unsigned max_step(unsigned v) {
-  constexpr int ctrl[6] = {0x111, 0x112, 0x114, 0x118, 0x142, 0x143};  // row_shr 1, 2, 4, 8, row_bcast 15, 31
-  constexpr int rows[6] = {0xF, 0xF, 0xF, 0xF, 0xA, 0xC};
-  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl[K], rows[K], 0xF, false));
-}
 template <typename T>
 __device__ __forceinline__ int pivot_of(unsigned scanned, unsigned key, T f, unsigned mask) {
   const unsigned top = (unsigned)__builtin_amdgcn_readlane((int)scanned, 63);
@@ -86,49 +81,6 @@ __device__ __forceinline__ int pivot_of(unsigned scanned, unsigned key, T f, uns
   }
   return __builtin_ctzll(hit);
 }
-
-// 1 / x as a division gives it, in steps that are spread between other work.
-struct Recip64 {
-  double x, n, m, r, e;
-  bool flag;
-  template <int K>
-  __device__ __forceinline__ void step() {
-    if constexpr (K == 0) {
-      bool unused;
-      n = __builtin_amdgcn_div_scale(1., x, false, &unused);
-      m = __builtin_amdgcn_div_scale(1., x, true, &flag);
-      r = __builtin_amdgcn_rcp(n);
-    } else if constexpr (K == 1 || K == 3) e = fma(-n, r, 1.);
-    else if constexpr (K == 2) r = fma(r, e, r);
-    else if constexpr (K == 4) {
-      r = fma(r, e, r);
-      e = m * r;
-    } else if constexpr (K == 5) m = fma(-n, e, m);
-    else r = __builtin_amdgcn_div_fixup(__builtin_amdgcn_div_fmas(m, r, e, flag), x, 1.);
-  }
-};
-struct Recip32 {
-  float x, n, m, r, e, q;
-  bool flag;
-  template <int K>
-  __device__ __forceinline__ void step() {
-    if constexpr (K == 0) {
-      bool unused;
-      n = __builtin_amdgcn_div_scalef(1.f, x, false, &unused);
-      m = __builtin_amdgcn_div_scalef(1.f, x, true, &flag);
-      r = __builtin_amdgcn_rcpf(n);
-    } else if constexpr (K == 1) e = fmaf(-n, r, 1.f);
-    else if constexpr (K == 2) {
-      r = fmaf(e, r, r);
-      q = m * r;
-    } else if constexpr (K == 3) e = fmaf(-n, q, m);
-    else if constexpr (K == 4) q = fmaf(e, r, q);
-    else if constexpr (K == 5) e = fmaf(-n, q, m);
-    else r = __builtin_amdgcn_div_fixupf(__builtin_amdgcn_div_fmasf(e, r, q, flag), x, 1.f);
-  }
-};
-__device__ __forceinline__ Recip64 recip_of(double x) { return Recip64{x}; }
-__device__ __forceinline__ Recip32 recip_of(float x) { return Recip32{x}; }
 
 // One chain's LDS. Rows and columns are padded to Np = 8 ceil(N / 8) by an identity, so that every panel is full: the
 // padding's pivots are its own ones. Two more arrays are in dynamic LDS: M, the block before each panel's update, a row as

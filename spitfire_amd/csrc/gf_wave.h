@@ -69,5 +69,55 @@ __device__ __forceinline__ int wave_first_argmax(float a, bool cand) {
   return hit ? __ffsll((long long)hit) - 1 : -1;
 }
 
+// step k = 0 .. 5 of the wave-wide maximum, complete in lane 63 after step 5
+template <int K>
+__device__ __forceinline__ unsigned max_step(unsigned v) {
+  constexpr int ctrl[6] = {0x111, 0x112, 0x114, 0x118, 0x142, 0x143};  // row_shr 1, 2, 4, 8, row_bcast 15, 31
+  constexpr int rows[6] = {0xF, 0xF, 0xF, 0xF, 0xA, 0xC};
+  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl[K], rows[K], 0xF, false));
+}
+// 1 / x as a division gives it, in steps that are spread between other work.
+struct Recip64 {
+  double x, n, m, r, e;
+  bool flag;
+  template <int K>
+  __device__ __forceinline__ void step() {
+    if constexpr (K == 0) {
+      bool unused;
+      n = __builtin_amdgcn_div_scale(1., x, false, &unused);
+      m = __builtin_amdgcn_div_scale(1., x, true, &flag);
+      r = __builtin_amdgcn_rcp(n);
+    } else if constexpr (K == 1 || K == 3) e = fma(-n, r, 1.);
+    else if constexpr (K == 2) r = fma(r, e, r);
+    else if constexpr (K == 4) {
+      r = fma(r, e, r);
+      e = m * r;
+    } else if constexpr (K == 5) m = fma(-n, e, m);
+    else r = __builtin_amdgcn_div_fixup(__builtin_amdgcn_div_fmas(m, r, e, flag), x, 1.);
+  }
+};
+struct Recip32 {
+  float x, n, m, r, e, q;
+  bool flag;
+  template <int K>
+  __device__ __forceinline__ void step() {
+    if constexpr (K == 0) {
+      bool unused;
+      n = __builtin_amdgcn_div_scalef(1.f, x, false, &unused);
+      m = __builtin_amdgcn_div_scalef(1.f, x, true, &flag);
+      r = __builtin_amdgcn_rcpf(n);
+    } else if constexpr (K == 1) e = fmaf(-n, r, 1.f);
+    else if constexpr (K == 2) {
+      r = fmaf(e, r, r);
+      q = m * r;
+    } else if constexpr (K == 3) e = fmaf(-n, q, m);
+    else if constexpr (K == 4) q = fmaf(e, r, q);
+    else if constexpr (K == 5) e = fmaf(-n, q, m);
+    else r = __builtin_amdgcn_div_fixupf(__builtin_amdgcn_div_fmasf(e, r, q, flag), x, 1.f);
+  }
+};
+__device__ __forceinline__ Recip64 recip_of(double x) { return Recip64{x}; }
+__device__ __forceinline__ Recip32 recip_of(float x) { return Recip32{x}; }
+
 }  // namespace wave
 }  // namespace gfa

@@ -140,3 +140,60 @@ def test_inverse_solve_edges(bs, precision):
     for s in range(len(sizes)):
         g = got[offsets[2][s]:offsets[2][s] + nb[s] * bs]
         assert np.max(np.abs(dense[s] @ g - rhs[s])) <= tol * np.max(np.abs(rhs[s]))
+
+
+@pytest.mark.parametrize('bs', [1, 2, 7, 8, 9, 53, 56, 57, 64])
+def test_lapack_factor_and_solve_edges(bs):
+    """Block sizes around the eight waves' columns, chains of one to five blocks, rows permuted so that pivots interchange and
+    with exact ties (integer blocks): pivots equal to LAPACK's, factors, L blocks and solutions against NumPy. Tolerance: 100 N
+    eps times the condition (at most 1e4 here) of the blocks, 10 times that for the chain."""
+    import torch
+    from scipy.linalg import lu_factor
+    from spitfire_amd import _native
+    rng = np.random.default_rng(bs)
+    sizes = [1, 2, 5, 1, 3]
+    parts, values, rhs = [], [], []
+    for s, n in enumerate(sizes):
+        V = rng.standard_normal((n, bs, bs)) if s % 2 else rng.integers(-1, 2, (n, bs, bs)).astype(float)
+        V = (V + (2. + 2. * bs) * np.eye(bs))[:, rng.permutation(bs)]
+        lo, up = 0.1 * rng.standard_normal((n - 1, bs)), 0.1 * rng.standard_normal((n - 1, bs))
+        parts.append((V, lo, up))
+        values.append(np.concatenate([V.transpose(0, 2, 1).ravel(), lo.ravel(), up.ravel()]))
+        rhs.append(rng.standard_normal(n * bs))
+    dev = torch.device('cuda:0')
+    nb = np.asarray(sizes)
+    offsets = [np.cumsum(np.r_[0, a])[:-1].astype(np.int64) for a in ([v.size for v in values], nb * bs * bs, nb * bs)]
+    V, b = (torch.tensor(np.concatenate(a), device=dev) for a in (values, rhs))
+    n, vo, lo, xo = (torch.tensor(a, device=dev) for a in (nb.astype(np.int32), *offsets))
+    L = torch.zeros(int((nb * bs * bs).sum()), device=dev, dtype=torch.float64)
+    P = torch.zeros(int((nb * bs).sum()), device=dev, dtype=torch.int32)
+    x = torch.zeros_like(b)
+    st = torch.cuda.current_stream().cuda_stream
+    lib = _native.lib()
+    _native.check(lib.gf_batch_btddod_full_factorize(len(sizes), n.data_ptr(), bs, V.data_ptr(), vo.data_ptr(), L.data_ptr(),
+                                                     lo.data_ptr(), P.data_ptr(), xo.data_ptr(), st))
+    _native.check(lib.gf_batch_btddod_full_solve(len(sizes), n.data_ptr(), bs, V.data_ptr(), vo.data_ptr(), L.data_ptr(),
+                                                 lo.data_ptr(), P.data_ptr(), xo.data_ptr(), b.data_ptr(), x.data_ptr(),
+                                                 xo.data_ptr(), st))
+    v, l, p, g = (t.cpu().numpy() for t in (V, L, P, x))
+    tol = 1e3 * bs * 2.2e-16 * 1e4
+    for s, (B, sub, sup) in enumerate(parts):
+        y, inv, A = None, None, None
+        for i in range(sizes[s]):
+            at = offsets[1][s] + i * bs * bs
+            blk = lambda a, o: a[o:o + bs * bs].reshape(bs, bs).T
+            D = B[i]
+            if i > 0:
+                Li = sub[i - 1][:, None] * inv
+                assert np.max(np.abs(blk(l, at) - Li)) <= tol * np.max(np.abs(Li))
+                D = D - Li * sup[i - 1][None, :]
+            lu, piv = lu_factor(D)
+            assert np.array_equal(p[offsets[2][s] + i * bs:offsets[2][s] + (i + 1) * bs], piv + 1)
+            assert np.max(np.abs(blk(v, offsets[0][s] + i * bs * bs) - lu)) <= tol * np.max(np.abs(lu))
+            inv = np.linalg.inv(D)
+        xs = g[offsets[2][s]:offsets[2][s] + sizes[s] * bs].reshape(sizes[s], bs)
+        r = np.einsum('nij,nj->ni', B, xs)
+        if sizes[s] > 1:
+            r[1:] += sub * xs[:-1]
+            r[:-1] += sup * xs[1:]
+        assert np.max(np.abs(r.ravel() - rhs[s])) <= tol * np.max(np.abs(rhs[s]))
