@@ -603,28 +603,40 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
         }
       }
       if (a.sens) {
-        // raw option-0 sensitivities, (ns+1)^2 column-major with stride ns+1 (rates_sensitivities_exact.cpp:1011-1026)
-        for (int s = 0; s < nact; ++s) {
-          const double *sp = sbase + s * stride;
-          const double *v = sp + NSA * SP_STRIDE + N_SCAL + 5 * nr;
-          const long q = a.sel ? (long)a.sel[first + s] : first + s;
-          double *so = a.sens + q * (long)(ns + 1) * (ns + 1);
-          for (int e = threadIdx.x; e < (ns + 1) * (ns + 1); e += THREADS) {
-            const int c = e / (ns + 1), k = e - c * (ns + 1);
-            double val = 0.;
-            if (k < ns) {
-              if (c == 0) val = sp[WS0_ * SP_STRIDE + k];
-              else if (c == 1) val = sp[WS1_ * SP_STRIDE + k];
-              else {
-                const int j = c - 2;
-                const int ee = j * ns + k;
-                double spv = 0.;
-                for (int t = mv.eg_off[ee]; t < mv.eg_off[ee + 1]; ++t) spv += mv.eg_coef[t] * v[mv.eg_slot[t]];
-                val = spv + mv.dinvm[j] * sp[A_ * SP_STRIDE + k] + sp[B_ * SP_STRIDE + k];
+        // raw option-0 sensitivities, (ns+1)^2 column-major with stride ns+1 (rates_sensitivities_exact.cpp:1011-1026); wave =
+        // column, lane = row, gathered from the tables in LDS as the Jacobian's species rows are
+        constexpr int NW = THREADS / 64;
+        const double Mk = lane < ns ? mv.mw[lane] : 0.;
+        for (int c = wave; c <= ns; c += NW) {
+          double val[S];
+          for (int s = 0; s < S; ++s) val[s] = 0.;
+          if (lane < ns) {
+            if (c < 2) {
+              for (int s = 0; s < S; ++s) val[s] = sbase[s * stride + (c == 0 ? WS0_ : WS1_) * SP_STRIDE + lane];
+            } else {
+              const int j = c - 2;
+              const double dj = mv.dinvm[j];
+              const double *vb = sbase + NSA * SP_STRIDE + N_SCAL + 5 * nr;
+              if (lane == j)
+                for (int s = 0; s < S; ++s) val[s] = sbase[s * stride + DG_ * SP_STRIDE + j];
+              const int t1 = exo[j * ns + lane + 1];
+              for (int t = exo[j * ns + lane]; t < t1; ++t) {
+                const uint32_t rec = exx[t];
+                const int slot = (int)(rec & 0xFFFFu);
+                const double coef = -(double)(int8_t)(rec >> 16) * Mk;
+                for (int s = 0; s < S; ++s) val[s] = fma(coef, vb[s * stride + slot], val[s]);
+              }
+              for (int s = 0; s < S; ++s) {
+                const double *sp = sbase + s * stride;
+                val[s] = fma(dj, sp[A_ * SP_STRIDE + lane], val[s]) + sp[B_ * SP_STRIDE + lane];
               }
             }
-            so[e] = val;
           }
+          if (lane <= ns)
+            for (int s = 0; s < nact; ++s) {
+              const long q = a.sel ? (long)a.sel[first + s] : first + s;
+              a.sens[(q * (ns + 1) + c) * (ns + 1) + lane] = val[s];
+            }
         }
       }
     }

@@ -61,11 +61,6 @@ struct MechView {
   const int *sp_idx;        // special-order lists
   const double *sp_ord;
   const double *sp_invmw;
-  // sensitivity entry (species row i < ns, species column j < ns-1) <- slots: entry e = j*ns + i
-  // (drop-in raw sensitivities only)
-  const int *eg_off;        // [(ns-1)*ns+1]
-  const int *eg_slot;
-  const double *eg_coef;
   // Compact gather tables, copied into LDS by the chemistry kernel (byte image at tbl, tbl_bytes long):
   //   u32 sgx_off[ns+1]; u64 sgx[n_sgx]   species k <- reactions with k in their net stoichiometry:
   //       bits 0-15 reaction, 16-31 slot of species k in that reaction (0xFFFF: none), 32-39 net

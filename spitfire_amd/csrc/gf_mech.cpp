@@ -170,10 +170,8 @@ int finalize(gf_mech *m) {
       sgx.insert(sgx.end(), L[k].begin(), L[k].end());
     }
   }
-  // eg: all terms of raw sensitivity entry (i, j); exx: the off-diagonal ones in compact form (the
+  // exx: the off-diagonal terms of raw sensitivity entry (i, j) in compact form (the
   // diagonal terms are summed in the species gather above)
-  std::vector<int> eg_off(nm * ns + 1, 0), eg_slot;
-  std::vector<double> eg_coef;
   std::vector<uint16_t> exx_off(nm * ns + 1, 0);
   std::vector<uint32_t> exx;
   {
@@ -187,8 +185,6 @@ int finalize(gf_mech *m) {
     }
     for (int e = 0; e < nm * ns; ++e) {
       const int i = e % ns;
-      eg_off[e + 1] = eg_off[e] + (int)E[e].size();
-      for (auto &t : E[e]) { eg_slot.push_back(t.first); eg_coef.push_back(-t.second * mw[i]); }
       const bool diag = (e / ns) == i;
       if (!diag)
         for (auto &t : E[e]) exx.push_back((uint32_t)t.first | ((uint32_t)(uint8_t)(int8_t)t.second << 16));
@@ -260,9 +256,6 @@ int finalize(gf_mech *m) {
   v.sp_idx = (const int *)P(a.put(sp_idx));
   v.sp_ord = (const double *)P(a.put(sp_ord));
   v.sp_invmw = (const double *)P(a.put(sp_invmw));
-  v.eg_off = (const int *)P(a.put(eg_off));
-  v.eg_slot = (const int *)P(a.put(eg_slot));
-  v.eg_coef = (const double *)P(a.put(eg_coef));
   v.tbl = (const char *)P(a.put(tbl));
   v.tbl_bytes = (int)tbl.size();
   v.sgx_at = sgx_at; v.exo_at = exo_at; v.exx_at = exx_at;
@@ -310,7 +303,6 @@ int ensure_device(gf_mech *m) {
   v.Tmin = rebase(v.Tmin, b); v.Tmax = rebase(v.Tmax, b); v.cpkind = rebase(v.cpkind, b); v.rx = rebase(v.rx, b);
   v.tb_idx = rebase(v.tb_idx, b); v.tb_eff = rebase(v.tb_eff, b); v.tb_slot = rebase(v.tb_slot, b);
   v.sp_idx = rebase(v.sp_idx, b); v.sp_ord = rebase(v.sp_ord, b); v.sp_invmw = rebase(v.sp_invmw, b);
-  v.eg_off = rebase(v.eg_off, b); v.eg_slot = rebase(v.eg_slot, b); v.eg_coef = rebase(v.eg_coef, b);
   v.tbl = rebase(v.tbl, b);
   m->view = v;
   if (!m->stream) {

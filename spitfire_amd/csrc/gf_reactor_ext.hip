@@ -5,8 +5,11 @@
 //     operation, and the (rho, T, Y) -> (T, Y) transform (isobaric_reactor_kernels.cpp:19-343);
 //   - the isochoric reactor in (rho, T, Y) with the same options (isochoric_reactor_kernels.cpp:18-333);
 // from the chemistry kernel's per-state production rates, raw option-0/1 sensitivities (ns+1)^2, mixture scalars
-// {rho, cp, dcp/dT, M} and species cp and h. One 64-thread workgroup per state; thread t owns primitive-Jacobian
-// columns t, t+64, ...; inner products run serially in the reference's summation order.
+// {rho, cp, dcp/dT, M} and species cp and h. One workgroup per state. The sensitivities are staged in LDS with coalesced
+// loads; the energy row's inner products run serially in the reference's summation order, thread t for columns t,
+// t+256, ...; the species rows are elementwise in the order of the output. (One wave per state, each lane reading
+// and writing its columns in memory, was bound by uncoalesced access: 1,200 isochoric states of 53 species
+// 73 us, the whole call with rates and sensitivities 268; now 114, this kernel and the sensitivities' gather from LDS.)
 //
 // thermo_getters_kernel evaluates the getters of griffon.pyx:684-758 for one (T, y): mixture molecular weight, mole
 // fractions, ideal-gas density and pressure, cp/cv/h/e of the mixture and of the species, and dcp/dT of the species
@@ -30,22 +33,30 @@ __device__ inline double dotp(int n, const double *a, const double *b) {
   return d;
 }
 
+constexpr int kExtThreads = 256;
+
 template <bool ISOCHORIC>
-__global__ void __launch_bounds__(64) reactor_ext_kernel(MechView mv, ReactorExtIO a) {
+__global__ void __launch_bounds__(kExtThreads) reactor_ext_kernel(MechView mv, ReactorExtIO a) {
   const int ns = mv.ns, nm = ns - 1;
   const int np = ns + 1;                   // columns of the primitive Jacobian (rho, T, Y_0..Y_{ns-2})
   const int n = ISOCHORIC ? ns + 1 : ns;   // equations
   const long s = blockIdx.x;
   const int t = threadIdx.x;
-  __shared__ double y[NS_MAX], ue[NS_MAX], cvi[NS_MAX], w[NS_MAX], uin[NS_MAX], yin[NS_MAX], extra[8];
-  extern __shared__ double pj[];  // isobaric: ns x (ns+1) primitive Jacobian; isochoric: unused
+  __shared__ double y[NS_MAX], ue[NS_MAX], cvi[NS_MAX], w[NS_MAX], uin[NS_MAX], yin[NS_MAX], extra[8], er[NS_MAX + 1];
+  extern __shared__ double sl[];  // with a Jacobian: sensitivities, column-major with stride ld (odd: spreads the banks)
+  const int ld = np | 1;
+  double *pj = sl + ld * np;      // isobaric: ns x (ns+1) primitive Jacobian
 
   const double *st = a.state + s * a.state_stride;
-  const double *ws = a.sens + s * (long)np * np;
   const double rho = a.aux[s * 4 + 0], cp = a.aux[s * 4 + 1], cpsT = a.aux[s * 4 + 2], mmw = a.aux[s * 4 + 3];
   const double T = ISOCHORIC ? st[1] : st[0];
   const double *ystate = ISOCHORIC ? st + 2 : st + 1;
   const double Ru = mv.Ru;
+  if (a.jac) {
+    const double *ws = a.sens + s * (long)np * np;
+    for (int e = t; e < np * np; e += kExtThreads) sl[e / np * ld + e % np] = ws[e];
+  }
+  if (t < nm) y[t] = ystate[t];
   if (t < ns) {
     // species heat capacity (cv for the isochoric reactor) and enthalpy (energy), at T and at the inflow temperature
     const double c = a.cpi[s * ns + t], h = a.hsp[s * ns + t];
@@ -61,15 +72,12 @@ __global__ void __launch_bounds__(64) reactor_ext_kernel(MechView mv, ReactorExt
       uin[t] = ISOCHORIC ? h2 - Ru * Ti * mv.invmw[t] : h2;
     }
   }
-  if (t == 0) {  // y_{ns-1} = 1 - sum of the others, in extract_y's order (combustion_kernels.h:526-530)
+  __syncthreads();
+  if (t == 64) {  // y_{ns-1} = 1 - sum of the others, in extract_y's order (combustion_kernels.h:526-530)
     double last = 1.;
-    for (int j = 0; j < nm; ++j) {
-      y[j] = ystate[j];
-      last -= y[j];
-    }
+    for (int j = 0; j < nm; ++j) last -= y[j];
     y[nm] = last;
   }
-  __syncthreads();
 
   const double cm = ISOCHORIC ? cp - Ru / mmw : cp;  // cv or cp of the mixture
   const double iR = 1. / rho, iC = 1. / cm, iRC = 1. / (rho * cm);
@@ -103,7 +111,7 @@ __global__ void __launch_bounds__(64) reactor_ext_kernel(MechView mv, ReactorExt
   if (a.rhs) {
     double *out = a.rhs + s * n;
     const int e0 = ISOCHORIC ? 1 : 0;  // energy equation index
-    for (int i = t; i < n; i += 64) {
+    for (int i = t; i < n; i += kExtThreads) {
       double v;
       if (ISOCHORIC && i == 0) {
         v = 0. + (a.open ? m_rho : 0.);
@@ -119,38 +127,47 @@ __global__ void __launch_bounds__(64) reactor_ext_kernel(MechView mv, ReactorExt
   }
   if (!a.jac) return;
 
+  // Rows of species: iR (wc - iR w) for the density column, iR wc for the others, and the mass exchange; every product that
+  // another term is added to is rounded by itself, so that the compiler's contractions are those of separate passes.
+  auto species = [&](int c, int i) {
+    const double wc = sl[c * ld + i];
+    if (c == 0) {
+      double v = __dmul_rn(iR, fma(-iR, w[i], wc));
+      if (ISOCHORIC && a.open) v = fma(-iR, __dmul_rn(yin[i] - y[i], mscale), v);
+      return v;
+    }
+    double v = __dmul_rn(iR, wc);
+    if (a.open && c >= 2 && i == c - 2) v += ISOCHORIC ? -it * a.rho_in / rho : -it;
+    return v;
+  };
+
   if (!ISOCHORIC) {
     // primitive Jacobian n x (n+1) column-major (isobaric_reactor_kernels.cpp:58-168), then the transform
-    for (int c = t; c < np; c += 64) {
-      double *col = pj + (long)c * ns;
-      const double *wc = ws + (long)c * np;
+    for (int c = t; c < np; c += kExtThreads) {
+      const double *wc = sl + c * ld;
+      double v;
       if (c == 0) {
-        col[0] = -iRC * dotp(ns, wc, ue) - iR * r_e;
-        for (int i = 0; i < nm; ++i) col[1 + i] = iR * (wc[i] - iR * w[i]);
-        if (a.heat == 2) col[0] += -q / rho;
+        v = -iRC * dotp(ns, wc, ue) - iR * r_e;
+        if (a.heat == 2) v += -q / rho;
       } else if (c == 1) {
-        col[0] = -iRC * (dotp(ns, wc, ue) + dotp(ns, w, cvi)) - r_e * cpsT * iC;
-        for (int i = 0; i < nm; ++i) col[1 + i] = wc[i] * iR;
-        if (a.open) col[0] += -iC * (cpsT * m_e + it * dotp(ns, yin, cvi));
+        v = -iRC * (dotp(ns, wc, ue) + dotp(ns, w, cvi)) - r_e * cpsT * iC;
+        if (a.open) v += -iC * (cpsT * m_e + it * dotp(ns, yin, cvi));
         if (a.heat == 2)
-          col[0] += -iC * cpsT * q - a.sov * iRC * (a.hc + 4. * a.eps * kStefanBoltzmann * T * T * T);
+          v += -iC * cpsT * q - a.sov * iRC * (a.hc + 4. * a.eps * kStefanBoltzmann * T * T * T);
       } else {
         const int k = c - 2;
-        col[0] = -iRC * dotp(ns, wc, ue) - r_e * (cvi[k] - cvi[nm]) * iC;
-        for (int i = 0; i < nm; ++i) col[1 + i] = iR * wc[i];
-        if (a.open) {
-          col[0] += -m_e * (cvi[k] - cvi[nm]) * iC;
-          col[1 + k] += -it;
-        }
-        if (a.heat == 2) col[0] += iC * q * (cvi[nm] - cvi[k]);
+        v = -iRC * dotp(ns, wc, ue) - r_e * (cvi[k] - cvi[nm]) * iC;
+        if (a.open) v += -m_e * (cvi[k] - cvi[nm]) * iC;
+        if (a.heat == 2) v += iC * q * (cvi[nm] - cvi[k]);
       }
-      if (a.heat == 1) col[0] = 0.;
+      pj[c * ns] = a.heat == 1 ? 0. : v;
     }
+    for (int e = t; e < np * nm; e += kExtThreads) pj[e / nm * ns + 1 + e % nm] = species(e / nm, e % nm);
     __syncthreads();
     // (rho, T, Y) -> (T, Y) at constant pressure (isobaric_reactor_kernels.cpp:319-343)
     double *J = a.jac + s * (long)ns * ns;
     const double roT = rho / T, nrm = -rho * mmw;
-    for (int e = t; e < ns * ns; e += 64) {
+    for (int e = t; e < ns * ns; e += kExtThreads) {
       const int c = e / ns, i = e - c * ns;
       J[e] = (c == 0) ? pj[ns + i] - roT * pj[i] : pj[(1 + c) * ns + i] + nrm * mv.dinvm[c - 1] * pj[i];
     }
@@ -158,36 +175,30 @@ __global__ void __launch_bounds__(64) reactor_ext_kernel(MechView mv, ReactorExt
   }
 
   // isochoric: (ns+1) x (ns+1) column-major in (rho, T, Y) (isochoric_reactor_kernels.cpp:60-333)
-  double *J = a.jac + s * (long)np * np;
-  for (int c = t; c < np; c += 64) {
-    double *col = J + (long)c * np;
-    const double *wc = ws + (long)c * np;
-    col[0] = 0.;
+  for (int c = t; c < np; c += kExtThreads) {
+    const double *wc = sl + c * ld;
+    double v;
     if (c == 0) {
-      col[1] = -iRC * dotp(ns, ue, wc) - iR * r_e;
-      for (int i = 0; i < nm; ++i) col[2 + i] = iR * (wc[i] - iR * w[i]);
-      if (a.open) {
-        col[0] = -it;
-        col[1] += -iR * m_e;
-        for (int i = 0; i < nm; ++i) col[2 + i] += -iR * ((yin[i] - y[i]) * mscale);
-      }
-      if (a.heat == 2) col[1] += -q / rho;
+      v = -iRC * dotp(ns, ue, wc) - iR * r_e;
+      if (a.open) v += -iR * m_e;
+      if (a.heat == 2) v += -q / rho;
     } else if (c == 1) {
-      col[1] = -iC * (iR * (dotp(ns, ue, wc) + dotp(ns, cvi, w)) + r_e * cpsT);
-      for (int i = 0; i < nm; ++i) col[2 + i] = iR * wc[i];
-      if (a.open) col[1] += -iC * (it * iR * (a.rho_in * dotp(ns, cvi, yin)) + cpsT * m_e);
-      if (a.heat == 2) col[1] += -iC * cpsT * q - a.sov * iRC * (a.hc + 4. * a.eps * kStefanBoltzmann * T * T * T);
+      v = -iC * (iR * (dotp(ns, ue, wc) + dotp(ns, cvi, w)) + r_e * cpsT);
+      if (a.open) v += -iC * (it * iR * (a.rho_in * dotp(ns, cvi, yin)) + cpsT * m_e);
+      if (a.heat == 2) v += -iC * cpsT * q - a.sov * iRC * (a.hc + 4. * a.eps * kStefanBoltzmann * T * T * T);
     } else {
       const int k = c - 2;
-      col[1] = -iRC * dotp(ns, ue, wc) - r_e * (cvi[k] - cvi[nm]) * iC;
-      for (int i = 0; i < nm; ++i) col[2 + i] = iR * wc[i];
-      if (a.open) {
-        col[1] += -iC * m_e * (cvi[k] - cvi[nm]);
-        col[2 + k] += -it * a.rho_in / rho;
-      }
-      if (a.heat == 2) col[1] += iC * q * (cvi[nm] - cvi[k]);
+      v = -iRC * dotp(ns, ue, wc) - r_e * (cvi[k] - cvi[nm]) * iC;
+      if (a.open) v += -iC * m_e * (cvi[k] - cvi[nm]);
+      if (a.heat == 2) v += iC * q * (cvi[nm] - cvi[k]);
     }
-    if (a.heat == 1) col[1] = 0.;
+    er[c] = a.heat == 1 ? 0. : v;
+  }
+  __syncthreads();
+  double *J = a.jac + s * (long)np * np;
+  for (int e = t; e < np * np; e += kExtThreads) {
+    const int c = e / np, i = e - c * np;
+    J[e] = i == 0 ? (c == 0 && a.open ? -it : 0.) : i == 1 ? er[c] : species(c, i - 2);
   }
 }
 
@@ -259,13 +270,12 @@ __global__ void __launch_bounds__(64) thermo_getters_kernel(MechView mv, const d
 
 int launch_reactor_ext(const gf_mech *m, const ReactorExtIO &a, hipStream_t st) {
   if (a.n <= 0) return GF_OK;
-  const int ns = m->view.ns;
-  if (a.isochoric) {
-    hipLaunchKernelGGL(reactor_ext_kernel<true>, dim3((unsigned)a.n), dim3(64), 0, st, m->view, a);
-  } else {
-    const size_t lds = (size_t)ns * (ns + 1) * sizeof(double);
-    hipLaunchKernelGGL(reactor_ext_kernel<false>, dim3((unsigned)a.n), dim3(64), lds, st, m->view, a);
-  }
+  const int ns = m->view.ns, np = ns + 1;
+  const size_t lds = a.jac ? sizeof(double) * ((np | 1) * np + (a.isochoric ? 0 : ns * np)) : 0;
+  auto kern = a.isochoric ? reactor_ext_kernel<true> : reactor_ext_kernel<false>;
+  if (lds > 60000 && hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    return fail(GF_ERR_UNSUPPORTED, "mechanism needs more LDS per workgroup than the device allows");
+  hipLaunchKernelGGL(kern, dim3((unsigned)a.n), dim3(kExtThreads), lds, st, m->view, a);
   if (hipGetLastError() != hipSuccess) return fail(GF_ERR_HIP, "reactor kernel launch failed");
   return GF_OK;
 }
