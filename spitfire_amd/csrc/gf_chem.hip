@@ -13,13 +13,24 @@
 //       action and all partial derivatives.
 //       dq_r/dY_s = sum_p v_{r,p} delta(s,p) + a_r (1/M_s - 1/M_last) + b_r, so each reaction stores five
 //       scalars (q, dq/drho, dq/dT, a, b) and one value v per participant slot.
-//   P2  one wave per state, lane = species k: gathers over the reactions with k in their net
+//   P2  lane = (species k, state): gathers over the reactions with k in their net
 //       stoichiometry give w_k, dw_k/drho, dw_k/dT, the rank-1 coefficients and the diagonal sensitivity
-//       entry of column k; wave reductions give the enthalpy-weighted sums; the RHS is written here.
+//       entry of column k; then one wave per state, lane = species: wave reductions give the enthalpy-weighted sums;
+//       the RHS is written here.
 //   P3  one wave per Jacobian column, lane = row (plus one lane for the last species), looping over the S
 //       states: off-diagonal sparse gather + rank-1 part give the species rows (chem_jac_isobaric + the
 //       (rho,T,Y)->(T,Y) transform at constant pressure); the temperature row is the enthalpy-weighted
 //       wave sum of the column; each column of each state is one contiguous 53-double store.
+//
+// What bounds it is latency, with few wavefronts: the Jacobian kernel's state (28 KB of LDS a state, 250 registers) leaves room
+// for eight waves per compute unit, the rates' registers for twelve (held to 168: at 186 they were eight and
+// 100,003 states took 1,033 us instead of 803). The states of a group are interleaved in LDS, so that neighbouring lanes read
+// neighbouring words, and a reaction's record is read whole, its short lists unrolled with factors of one beyond their
+// ends: field by field, with loops of one to four trips around dependent loads, P1 took 41,000 cycles for a group
+// of four states with derivatives and now takes 32,000. 53 species, 325 reactions, before and after (us): RHS of 512 / 7,600 /
+// 100,003 states 16.5 / 85 / 880 -> 14.7 / 78 / 803; with Jacobian 512 / 4,000 / 100,000 38 / 169 / 3,938 -> 33 / 155 / 3,596.
+// Tried without gain: P3's slot sums dealt to the lanes by length through LDS (every lane busy, but the same words through
+// the banks again: 38,000 -> 45,000 cycles a group); 16 waves at 128 registers (226 spilled).
 #include "gf_internal.h"
 #include "gf_thermo.h"
 #include "../../include/griffon_amd.h"
@@ -133,14 +144,13 @@ __device__ __forceinline__ double troe_fcent(const DevRxn &R, double T, double i
 }
 
 template <int S, int THREADS, bool JAC>
-__global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, long groups_per_wg) {
+__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(JAC ? 1 : 3))) chem_kernel(MechView mv, ChemArgs a, long groups_per_wg) {
   static_assert(S >= 1 && S <= 4, "the temperature-row sums take at most four states at once");
   extern __shared__ double lds[];
   const int ns = mv.ns, nr = mv.nr, nm = ns - 1;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   constexpr int NSA = JAC ? N_SPEC_ARR : N_SPEC_ARR_RHS;
-  const long stride = NSA * SP_STRIDE + N_SCAL + (JAC ? 5L * nr + mv.nslot : (long)nr);
   const long ngroups = (a.n + S - 1) / S;
   // each workgroup owns a contiguous range of state groups (neighbouring states share SoA input lines)
   const long g0 = (long)blockIdx.x * groups_per_wg;
@@ -159,7 +169,12 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
   const int *tbi = reinterpret_cast<const int *>(tb + mv.tbi_at);
   const int *tbsl = reinterpret_cast<const int *>(tb + mv.tbs_at);
   const double *imw = reinterpret_cast<const double *>(tb + mv.imw_at);
+  // a group's S states are interleaved: entry e of state s at e * S + s
   double *sbase = lds + tcopy / 8;
+  auto SP = [&](int array, int k, int s) -> double & { return sbase[(array * SP_STRIDE + k) * S + s]; };
+  auto SC = [&](int e, int s) -> double & { return sbase[(NSA * SP_STRIDE + e) * S + s]; };
+  double *rqb = sbase + (NSA * SP_STRIDE + N_SCAL) * S;  // per reaction: rate and its derivatives
+  double *vb = rqb + 5L * nr * S;                       // per slot
   __syncthreads();
 
   for (long group = g0; group < g1; ++group) {
@@ -168,8 +183,6 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
     // ---------------- P0: mixture thermo (wave per state, lane = species) ----------------
     if (wave < S) {
       const long il = first + wave;
-      double *sp = sbase + wave * stride;
-      double *sc = sp + NSA * SP_STRIDE;
       if (il < a.n) {
         const long i = a.sel ? (long)a.sel[il] : il;
         const double *xi = a.x + i * a.xs_i;
@@ -189,11 +202,11 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
         double cp = 0., cps = 0., h = 0., Gk = 0., dB = 0.;
         if (lane < ns) species_thermo(mv, lane, T, logT, invT, cp, cps, h, Gk, dB);
         if (lane < ns) {
-          sp[Y_ * SP_STRIDE + lane] = yk;
-          sp[H_ * SP_STRIDE + lane] = h;
-          sp[CPI_ * SP_STRIDE + lane] = cp;
-          sp[G_ * SP_STRIDE + lane] = Gk;
-          if (JAC) sp[DBDT_ * SP_STRIDE + lane] = dB;
+          SP(Y_, lane, wave) = yk;
+          SP(H_, lane, wave) = h;
+          SP(CPI_, lane, wave) = cp;
+          SP(G_, lane, wave) = Gk;
+          if (JAC) SP(DBDT_, lane, wave) = dB;
         }
         const double cpm = wave_sum(lane < ns ? yk * cp : 0.);
         // a constant-cp species resets the dcp/dT accumulation (thermodynamics_kernels.cpp:200-203)
@@ -202,9 +215,9 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
         if (a.cpi && lane < ns) a.cpi[i * ns + lane] = cp;
         if (a.hsp && lane < ns) a.hsp[i * ns + lane] = h;
         if (lane == 0) {
-          sc[S_T] = T; sc[S_RHO] = rho; sc[S_MMW] = mmw; sc[S_CP] = cpm; sc[S_CPST] = cpsm;
-          sc[S_INVT] = invT; sc[S_LOGT] = logT; sc[S_CT] = rho * mm; sc[S_INVM] = mm;
-          sc[S_LOGPORT] = log(mv.pref * invT * mv.invRu);
+          SC(S_T, wave) = T; SC(S_RHO, wave) = rho; SC(S_MMW, wave) = mmw; SC(S_CP, wave) = cpm; SC(S_CPST, wave) = cpsm;
+          SC(S_INVT, wave) = invT; SC(S_LOGT, wave) = logT; SC(S_CT, wave) = rho * mm; SC(S_INVM, wave) = mm;
+          SC(S_LOGPORT, wave) = log(mv.pref * invT * mv.invRu);
         }
       }
     }
@@ -215,19 +228,51 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
       const int r = it / S, s = it - r * S;
       const long i = first + s;
       if (i >= a.n) continue;
-      double *sp = sbase + s * stride;
-      const double *sc = sp + NSA * SP_STRIDE;
-      double *rq = sp + NSA * SP_STRIDE + N_SCAL;
-      double *v = rq + 5 * nr;
-      const double *y = sp + Y_ * SP_STRIDE;
-      const double T = sc[S_T], rho = sc[S_RHO], invT = sc[S_INVT], logT = sc[S_LOGT], ct = sc[S_CT],
-                   invM = sc[S_INVM];
-      const DevRxn &R = mv.rx[r];
+      auto y = [&](int k) { return SP(Y_, k, s); };
+      auto rq = [&](int e) -> double & { return rqb[e * S + s]; };
+      const double T = SC(S_T, s), rho = SC(S_RHO, s), invT = SC(S_INVT, s), logT = SC(S_LOGT, s), ct = SC(S_CT, s),
+                   invM = SC(S_INVM, s);
+      const DevRxn R = mv.rx[r];  // the whole record at once; arrays in it are indexed by constants below
       const double kf = kf_of(R, T, logT, invT);
 
       // third-body / falloff multiplier
       double tbsum = 0.;
-      for (int q = 0; q < R.n_tb; ++q) tbsum += tbe[R.tb_off + q] * y[tbi[R.tb_off + q]];
+      for (int q = 0; q < R.n_tb; q += 4) {  // four at a time, so that their loads overlap; missing ones add zero
+        double e[4], ye[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int at = R.tb_off + min(q + u, R.n_tb - 1);
+          e[u] = tbe[at];
+          ye[u] = y(tbi[at]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) tbsum = q + u < R.n_tb ? fma(e[u], ye[u], tbsum) : tbsum;
+      }
+      // concentration factors of the reactants and products (1 beyond the list), and the net Gibbs function
+      double C[NRC_MAX], F[NRC_MAX], Cp[NPD_MAX], Fp[NPD_MAX], sg = 0., sb = 0.;
+      if (!R.hasOrders) {
+#pragma unroll
+        for (int j = 0; j < NRC_MAX; ++j) {
+          C[j] = y(R.rc_idx[j]) * rho * imw[R.rc_idx[j]];
+          F[j] = j < R.n_rc ? ipow3(C[j], R.rc_st[j]) : 1.;
+        }
+        if (R.reversible) {
+#pragma unroll
+          for (int j = 0; j < NPD_MAX; ++j) {
+            Cp[j] = y(R.pd_idx[j]) * rho * imw[R.pd_idx[j]];
+            Fp[j] = j < R.n_pd ? ipow3(Cp[j], R.pd_st[j]) : 1.;
+          }
+#pragma unroll
+          for (int q = 0; q < NNET_MAX; ++q) {
+            const double g = SP(G_, R.net_idx[q], s);
+            sg = q < R.n_net ? fma(R.net_st[q], g, sg) : sg;
+            if (JAC) {
+              const double d = SP(DBDT_, R.net_idx[q], s);
+              sb = q < R.n_net ? fma(R.net_st[q], d, sb) : sb;
+            }
+          }
+        }
+      }
 
       if (!JAC) {
         // production_rates formulation (chemistry_kernels.cpp:140-461)
@@ -246,27 +291,21 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
           k = k * pow(10., logFc / (1 + F1 * F1)) * pr / (1 + pr);
         }
         if (R.hasOrders) {
+#pragma unroll 1
           for (int q = 0; q < R.n_sp; ++q) {
             const int sidx = mv.sp_idx[R.sp_off + q];
-            k *= pow(fmax(y[sidx] * rho * mv.sp_invmw[R.sp_off + q], 0.), mv.sp_ord[R.sp_off + q]);
+            k *= pow(fmax(y(sidx) * rho * mv.sp_invmw[R.sp_off + q], 0.), mv.sp_ord[R.sp_off + q]);
           }
         } else {
+          if (R.reversible) kr = k * exp(R.sumStoich * SC(S_LOGPORT, s) - invT * mv.invRu * sg);
+#pragma unroll
+          for (int j = 0; j < NRC_MAX; ++j) k *= F[j];
           if (R.reversible) {
-            double sg = 0.;
-            for (int q = 0; q < R.n_net; ++q) sg += R.net_st[q] * sp[G_ * SP_STRIDE + R.net_idx[q]];
-            kr = k * exp(R.sumStoich * sc[S_LOGPORT] - invT * mv.invRu * sg);
+#pragma unroll
+            for (int j = 0; j < NPD_MAX; ++j) kr *= Fp[j];
           }
-          for (int j = 0; j < R.n_rc; ++j) {
-            const int sidx = R.rc_idx[j];
-            k *= ipow3(y[sidx] * rho * imw[sidx], R.rc_st[j]);
-          }
-          if (R.reversible)
-            for (int j = 0; j < R.n_pd; ++j) {
-              const int sidx = R.pd_idx[j];
-              kr *= ipow3(y[sidx] * rho * imw[sidx], R.pd_st[j]);
-            }
         }
-        rq[r] = k - kr;
+        rq(r) = k - kr;
         continue;
       }
 
@@ -318,152 +357,192 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
         cdense = 0.;
         tbs = 0.;
       }
-      double *vr = v + R.slot_off;
-      for (int q = 0; q < R.n_slot; ++q) vr[q] = 0.;
+      auto vr = [&](int q) -> double & { return vb[(R.slot_off + q) * S + s]; };
+      for (int q = 0; q < R.n_slot; ++q) vr(q) = 0.;
       double Rnet, dRdrho, dRdT, U = 0.;
       const double ksens = arrh_sens_over_k(R.kf, invT);
       if (R.hasOrders) {  // rates_sensitivities_exact.cpp:198-281
-        double C[NSP_MAX], ordv[NSP_MAX];
-        int sidx[NSP_MAX];
+        auto conc = [&](int q) { return y(mv.sp_idx[R.sp_off + q]) * rho * mv.sp_invmw[R.sp_off + q]; };
+        auto order = [&](int q) { return mv.sp_ord[R.sp_off + q]; };
         Rnet = kf;
         double sumO = 0.;
+#pragma unroll 1
         for (int q = 0; q < R.n_sp; ++q) {
-          sidx[q] = mv.sp_idx[R.sp_off + q];
-          ordv[q] = mv.sp_ord[R.sp_off + q];
-          C[q] = y[sidx[q]] * rho * mv.sp_invmw[R.sp_off + q];
-          Rnet *= pow(fmax(C[q], 0.), ordv[q]);
-          sumO += ordv[q];
+          Rnet *= pow(fmax(conc(q), 0.), order(q));
+          sumO += order(q);
         }
         dRdrho = Rnet / ct * invM * sumO;
         dRdT = Rnet * ksens;
+#pragma unroll 1
         for (int j = 0; j < R.n_sp; ++j) {
           const double im = mv.sp_invmw[R.sp_off + j];
-          const bool last = (sidx[j] == ns - 1);
+          const bool last = (mv.sp_idx[R.sp_off + j] == ns - 1);
           double m = kf;
+#pragma unroll 1
           for (int l = 0; l < R.n_sp; ++l) {
-            if (l != j) {
-              m *= last ? pow(C[l], ordv[l]) : pow(fmax(C[l], 0.), ordv[l]);
-            } else {
-              if (last || ordv[l] > 1) m *= ordv[l] * rho * im * pow(fmax(C[l], 1.e-16), ordv[l] - 1.);
-              else m *= ordv[l] * rho * im / pow(fmax(C[l], 1.e-16), 1. - ordv[l]);
-            }
+            const double o = order(l), cl = conc(l);
+            // of its own species the derivative o C^(o-1), of the others the factor itself
+            const bool own = l == j, inv = own && !(last || o > 1);
+            const double f = pow(own ? fmax(cl, 1.e-16) : last ? cl : fmax(cl, 0.), own ? (inv ? 1. - o : o - 1.) : o);
+            if (!own) m *= f;
+            else if (inv) m *= o * rho * im / f;
+            else m *= o * rho * im * f;
           }
           if (last) U -= m;
-          else vr[R.sp_slot[j]] += Ctbaf * m;
+          else {
+            int slot = R.sp_slot[0];
+#pragma unroll
+            for (int u = 1; u < NSP_MAX; ++u) slot = j == u ? R.sp_slot[u] : slot;
+            vr(slot) += Ctbaf * m;
+          }
         }
       } else {
-        double C[NRC_MAX];
         Rnet = kf;
-        for (int j = 0; j < R.n_rc; ++j) {
-          C[j] = y[R.rc_idx[j]] * rho * imw[R.rc_idx[j]];
-          Rnet *= ipow3(C[j], R.rc_st[j]);
-        }
+#pragma unroll
+        for (int j = 0; j < NRC_MAX; ++j) Rnet *= F[j];
         dRdrho = Rnet / ct * invM * R.sumRc;
         dRdT = Rnet * ksens;
-        for (int j = 0; j < R.n_rc; ++j) {
-          double d = kf * rho * imw[R.rc_idx[j]] * R.rc_st[j] * (R.rc_st[j] == 1 ? 1. : ipow3(C[j], R.rc_st[j] - 1));
-          for (int l = 0; l < R.n_rc; ++l)
-            if (l != j) d *= ipow3(C[l], R.rc_st[l]);
-          if (R.rc_slot[j] >= 0) vr[R.rc_slot[j]] += Ctbaf * d;
-          else U -= d;
-        }
+#pragma unroll
+        for (int j = 0; j < NRC_MAX; ++j)
+          if (j < R.n_rc) {
+            double d = kf * rho * imw[R.rc_idx[j]] * R.rc_st[j] * (R.rc_st[j] == 1 ? 1. : ipow3(C[j], R.rc_st[j] - 1));
+#pragma unroll
+            for (int l = 0; l < NRC_MAX; ++l)
+              if (l != j) d *= F[l];
+            if (R.rc_slot[j] >= 0) vr(R.rc_slot[j]) += Ctbaf * d;
+            else U -= d;
+          }
         if (R.reversible) {
-          double sg = 0., sb = 0.;
-          for (int q = 0; q < R.n_net; ++q) {
-            sg += R.net_st[q] * sp[G_ * SP_STRIDE + R.net_idx[q]];
-            sb += R.net_st[q] * sp[DBDT_ * SP_STRIDE + R.net_idx[q]];
-          }
-          const double Kc = exp(-(R.sumStoich * sc[S_LOGPORT] - invT * mv.invRu * sg));
+          const double Kc = exp(-(R.sumStoich * SC(S_LOGPORT, s) - invT * mv.invRu * sg));
           const double kr = kf / Kc;
-          double Cp[NPD_MAX];
           double Rr = kr;
-          for (int j = 0; j < R.n_pd; ++j) {
-            Cp[j] = y[R.pd_idx[j]] * rho * imw[R.pd_idx[j]];
-            Rr *= ipow3(Cp[j], R.pd_st[j]);
-          }
+#pragma unroll
+          for (int j = 0; j < NPD_MAX; ++j) Rr *= Fp[j];
           Rnet -= Rr;
           dRdrho -= Rr / ct * invM * R.sumPd;
           dRdT -= Rr * (ksens + sb);
-          for (int j = 0; j < R.n_pd; ++j) {
-            double d = kr * rho * imw[R.pd_idx[j]] * R.pd_st[j] * (R.pd_st[j] == 1 ? 1. : ipow3(Cp[j], R.pd_st[j] - 1));
-            for (int l = 0; l < R.n_pd; ++l)
-              if (l != j) d *= ipow3(Cp[l], R.pd_st[l]);
-            if (R.pd_slot[j] >= 0) vr[R.pd_slot[j]] -= Ctbaf * d;
-            else U += d;
-          }
+#pragma unroll
+          for (int j = 0; j < NPD_MAX; ++j)
+            if (j < R.n_pd) {
+              double d = kr * rho * imw[R.pd_idx[j]] * R.pd_st[j] * (R.pd_st[j] == 1 ? 1. : ipow3(Cp[j], R.pd_st[j] - 1));
+#pragma unroll
+              for (int l = 0; l < NPD_MAX; ++l)
+                if (l != j) d *= Fp[l];
+              if (R.pd_slot[j] >= 0) vr(R.pd_slot[j]) -= Ctbaf * d;
+              else U += d;
+            }
         }
       }
       double Elast = 0.;
-      for (int q = 0; q < R.n_tb; ++q) {
-        const int slot = tbsl[R.tb_off + q];
-        const double e = tbe[R.tb_off + q];
-        if (slot >= 0) vr[slot] += Rnet * tbs * e;
-        else if (q == R.tb_last) Elast = tbs * e;
+      for (int q = 0; q < R.n_tb; q += 4) {
+        int slot[4];
+        double e[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int at = R.tb_off + min(q + u, R.n_tb - 1);
+          slot[u] = tbsl[at];
+          e[u] = tbe[at];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (q + u < R.n_tb) {
+            if (slot[u] >= 0) vr(slot[u]) += Rnet * tbs * e[u];
+            else if (q + u == R.tb_last) Elast = tbs * e[u];
+          }
       }
-      rq[r] = Rnet * Ctbaf;
+      rq(r) = Rnet * Ctbaf;
       if (a.qa) {
         const long q = a.sel ? (long)a.sel[i] : i;
         a.qa[q * nr + R.orig] = Rnet * ((R.type == RK_LINDEMANN || R.type == RK_TROE) ? qaC : Ctbaf);
       }
-      rq[nr + r] = dRdrho * Ctbaf + dCdrho * Rnet;
-      rq[2 * nr + r] = dRdT * Ctbaf + dCdT * Rnet;
-      rq[3 * nr + r] = Rnet * cdense;
-      rq[4 * nr + r] = Ctbaf * U - Rnet * Elast;
+      rq(nr + r) = dRdrho * Ctbaf + dCdrho * Rnet;
+      rq(2 * nr + r) = dRdT * Ctbaf + dCdT * Rnet;
+      rq(3 * nr + r) = Rnet * cdense;
+      rq(4 * nr + r) = Ctbaf * U - Rnet * Elast;
     }
     __syncthreads();
 
-    // ---------------- P2: species gathers + reductions (wave per state, lane = species) ----------------
-    if (wave < S) {
-      const long il = first + wave;
-      double *sp = sbase + wave * stride;
-      double *sc = sp + NSA * SP_STRIDE;
-      const double *rq = sc + N_SCAL;
-      const double *v = rq + 5 * nr;
-      if (il < a.n) {
-        const long i = a.sel ? (long)a.sel[il] : il;
-        double w = 0., w0 = 0., w1 = 0., A = 0., B = 0., DG = 0.;
-        if (lane < ns) {
-          const double Mk = mv.mw[lane];
-          const uint32_t e0 = sgx_off[lane], e1 = sgx_off[lane + 1];
-          uint32_t e = e0;
+    // ---------------- P2: species gathers (lane = (species, state), as in P1) ----------------
+    // With room for two lanes each, half of the waves gather the rates and half the rank-1 and diagonal terms.
+    {
+      constexpr int HALF = THREADS / 2;
+      const bool two = JAC && HALF >= ns * S;
+      const int part = two && threadIdx.x >= HALF ? 1 : 0;
+      for (int it = threadIdx.x - part * HALF; it < ns * S; it += two ? HALF : THREADS) {
+        const int k = it / S, s = it - k * S;
+        const double Mk = mv.mw[k];
+        const uint32_t e0 = sgx_off[k], e1 = sgx_off[k + 1];
+        auto rq = [&](int e) { return rqb[e * S + s]; };
+        uint32_t e = e0;
+        if (!JAC || !two || part == 0) {
+          double w = 0., w0 = 0., w1 = 0.;
           for (; e + 1 < e1; e += 2) {  // two reactions per trip: their LDS loads overlap (same summation order)
             const uint64_t ra = sgx[e], rb = sgx[e + 1];
             const int r0 = (int)(ra & 0xFFFFu), r1 = (int)(rb & 0xFFFFu);
             const double c0 = -(double)(int8_t)(ra >> 32) * Mk, c1 = -(double)(int8_t)(rb >> 32) * Mk;
-            const double q0 = rq[r0], q1 = rq[r1];
+            const double q0 = rq(r0), q1 = rq(r1);
             if (JAC) {
-              const int d0 = (int)((ra >> 16) & 0xFFFFu), d1 = (int)((rb >> 16) & 0xFFFFu);
-              const double a00 = rq[nr + r0], a01 = rq[nr + r1], a10 = rq[2 * nr + r0], a11 = rq[2 * nr + r1];
-              const double a20 = rq[3 * nr + r0], a21 = rq[3 * nr + r1], a30 = rq[4 * nr + r0], a31 = rq[4 * nr + r1];
-              const double v0 = d0 != 0xFFFF ? v[d0] : 0., v1 = d1 != 0xFFFF ? v[d1] : 0.;
-              w += c0 * q0; w += c1 * q1;
+              const double a00 = rq(nr + r0), a01 = rq(nr + r1), a10 = rq(2 * nr + r0), a11 = rq(2 * nr + r1);
               w0 += c0 * a00; w0 += c1 * a01;
               w1 += c0 * a10; w1 += c1 * a11;
-              A += c0 * a20; A += c1 * a21;
-              B += c0 * a30; B += c1 * a31;
-              if (d0 != 0xFFFF) DG += c0 * v0;
-              if (d1 != 0xFFFF) DG += c1 * v1;
-            } else {
-              w += c0 * q0; w += c1 * q1;
             }
+            w += c0 * q0; w += c1 * q1;
           }
-          for (; e < e1; ++e) {
+          if (e < e1) {
             const uint64_t rec = sgx[e];
             const int r = (int)(rec & 0xFFFFu);
             const double c = -(double)(int8_t)(rec >> 32) * Mk;  // -nu * M_k (rates_sensitivities_exact.cpp:1018)
-            w += c * rq[r];
+            w += c * rq(r);
             if (JAC) {
-              w0 += c * rq[nr + r];
-              w1 += c * rq[2 * nr + r];
-              A += c * rq[3 * nr + r];
-              B += c * rq[4 * nr + r];
-              const int ds = (int)((rec >> 16) & 0xFFFFu);
-              if (ds != 0xFFFF) DG += c * v[ds];
+              w0 += c * rq(nr + r);
+              w1 += c * rq(2 * nr + r);
             }
           }
+          SP(JAC ? W_ : G_, k, s) = w;  // (the rates need G no more)
+          if (JAC) {
+            SP(WS0_, k, s) = w0;
+            SP(WS1_, k, s) = w1;
+          }
         }
-        const double h = lane < ns ? sp[H_ * SP_STRIDE + lane] : 0.;
-        const double rho = sc[S_RHO], cp = sc[S_CP];
+        if (JAC && (!two || part == 1)) {
+          double A = 0., B = 0., DG = 0.;
+          for (e = e0; e + 1 < e1; e += 2) {
+            const uint64_t ra = sgx[e], rb = sgx[e + 1];
+            const int r0 = (int)(ra & 0xFFFFu), r1 = (int)(rb & 0xFFFFu);
+            const double c0 = -(double)(int8_t)(ra >> 32) * Mk, c1 = -(double)(int8_t)(rb >> 32) * Mk;
+            const int d0 = (int)((ra >> 16) & 0xFFFFu), d1 = (int)((rb >> 16) & 0xFFFFu);
+            const double a20 = rq(3 * nr + r0), a21 = rq(3 * nr + r1), a30 = rq(4 * nr + r0), a31 = rq(4 * nr + r1);
+            const double v0 = d0 != 0xFFFF ? vb[d0 * S + s] : 0., v1 = d1 != 0xFFFF ? vb[d1 * S + s] : 0.;
+            A += c0 * a20; A += c1 * a21;
+            B += c0 * a30; B += c1 * a31;
+            if (d0 != 0xFFFF) DG += c0 * v0;
+            if (d1 != 0xFFFF) DG += c1 * v1;
+          }
+          if (e < e1) {
+            const uint64_t rec = sgx[e];
+            const int r = (int)(rec & 0xFFFFu);
+            const double c = -(double)(int8_t)(rec >> 32) * Mk;
+            A += c * rq(3 * nr + r);
+            B += c * rq(4 * nr + r);
+            const int ds = (int)((rec >> 16) & 0xFFFFu);
+            if (ds != 0xFFFF) DG += c * vb[ds * S + s];
+          }
+          SP(A_, k, s) = A;
+          SP(B_, k, s) = B;
+          SP(DG_, k, s) = DG;
+        }
+      }
+    }
+    __syncthreads();
+    // reductions over the species (wave per state, lane = species)
+    if (wave < S) {
+      const long il = first + wave;
+      if (il < a.n) {
+        const long i = a.sel ? (long)a.sel[il] : il;
+        const double w = lane < ns ? SP(JAC ? W_ : G_, lane, wave) : 0.;
+        const double w0 = JAC && lane < ns ? SP(WS0_, lane, wave) : 0., w1 = JAC && lane < ns ? SP(WS1_, lane, wave) : 0.;
+        const double h = lane < ns ? SP(H_, lane, wave) : 0.;
+        const double rho = SC(S_RHO, wave), cp = SC(S_CP, wave);
         const double HW = wave_sum(h * w);
         const double rhs0 = -HW / (rho * cp);
         const double iR = 1. / rho;
@@ -474,21 +553,13 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
         }
         if (a.wout && lane < ns) a.wout[i * ns + lane] = w;
         if (JAC) {
-          const double cpi = lane < ns ? sp[CPI_ * SP_STRIDE + lane] : 0.;
+          const double cpi = lane < ns ? SP(CPI_, lane, wave) : 0.;
           const double HS0 = wave_sum(h * w0), HS1 = wave_sum(h * w1), WCP = wave_sum(w * cpi);
-          if (lane < ns) {
-            sp[W_ * SP_STRIDE + lane] = w;
-            sp[WS0_ * SP_STRIDE + lane] = w0;
-            sp[WS1_ * SP_STRIDE + lane] = w1;
-            sp[A_ * SP_STRIDE + lane] = A;
-            sp[B_ * SP_STRIDE + lane] = B;
-            sp[DG_ * SP_STRIDE + lane] = DG;
-          }
           const double iRC = 1. / (rho * cp);
-          if (lane < nm) sp[PR_ * SP_STRIDE + 1 + lane] = iR * (w0 - iR * w);
+          if (lane < nm) SP(PR_, 1 + lane, wave) = iR * (w0 - iR * w);
           if (lane == 0) {
-            sp[PR_ * SP_STRIDE] = -iRC * HS0 - iR * rhs0;
-            sc[S_RHS0] = rhs0; sc[S_HS0] = HS0; sc[S_HS1] = HS1; sc[S_WCP] = WCP;
+            SP(PR_, 0, wave) = -iRC * HS0 - iR * rhs0;
+            SC(S_RHS0, wave) = rhs0; SC(S_HS0, wave) = HS0; SC(S_HS1, wave) = HS1; SC(S_WCP, wave) = WCP;
           }
         }
       }
@@ -511,11 +582,10 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
             if (off >= 0) jb[s] = a.jac + off;
           }
         }
-        const double *sc = sbase + s * stride + NSA * SP_STRIDE;
-        iR[s] = 1. / sc[S_RHO];
-        iRC[s] = 1. / (sc[S_RHO] * sc[S_CP]);
-        ric[s] = sc[S_RHS0] / sc[S_CP];
-        rmw[s] = -sc[S_RHO] * sc[S_MMW];
+        iR[s] = 1. / SC(S_RHO, s);
+        iRC[s] = 1. / (SC(S_RHO, s) * SC(S_CP, s));
+        ric[s] = SC(S_RHS0, s) / SC(S_CP, s);
+        rmw[s] = -SC(S_RHO, s) * SC(S_MMW, s);
       }
       if (a.jac) {
         constexpr int NW = THREADS / 64;
@@ -526,23 +596,19 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
         // the row's molecular weight (loaded here: in the column loop the Jacobian stores could alias it)
         const double MiL = rowL ? mv.mw[iiL] : 0.;
         for (int s = 0; s < S; ++s) {
-          const double *sp = sbase + s * stride;
-          rA[s] = rowL ? sp[A_ * SP_STRIDE + iiL] : 0.;
-          rB[s] = rowL ? sp[B_ * SP_STRIDE + iiL] : 0.;
-          rH[s] = rowL ? sp[H_ * SP_STRIDE + iiL] : 0.;
-          rP[s] = lane < ns ? sp[PR_ * SP_STRIDE + lane] : 0.;
+          rA[s] = rowL ? SP(A_, iiL, s) : 0.;
+          rB[s] = rowL ? SP(B_, iiL, s) : 0.;
+          rH[s] = rowL ? SP(H_, iiL, s) : 0.;
+          rP[s] = lane < ns ? SP(PR_, lane, s) : 0.;
         }
         for (int c = wave; c < ns; c += NW) {
           double val[S];
           if (c == 0) {
             for (int s = 0; s < S; ++s) {
-              const double *sp = sbase + s * stride;
-              const double *sc = sp + NSA * SP_STRIDE;
-              const double *pr = sp + PR_ * SP_STRIDE;
-              const double roT = sc[S_RHO] / sc[S_T];
-              const double T00 = fma(-iRC[s], sc[S_HS1] + sc[S_WCP], -__dmul_rn(ric[s], sc[S_CPST]));
-              val[s] = (lane == 0) ? fma(-roT, pr[0], T00)
-                                   : (lane < ns ? fma(-roT, pr[lane], __dmul_rn(sp[WS1_ * SP_STRIDE + lane - 1], iR[s]))
+              const double roT = SC(S_RHO, s) / SC(S_T, s);
+              const double T00 = fma(-iRC[s], SC(S_HS1, s) + SC(S_WCP, s), -__dmul_rn(ric[s], SC(S_CPST, s)));
+              val[s] = (lane == 0) ? fma(-roT, SP(PR_, 0, s), T00)
+                                   : (lane < ns ? fma(-roT, SP(PR_, lane, s), __dmul_rn(SP(WS1_, lane - 1, s), iR[s]))
                                                 : 0.);
             }
           } else {
@@ -553,11 +619,10 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
             double full[S];
             for (int s = 0; s < S; ++s) full[s] = 0.;
             if (row) {
-              for (int s = 0; s < S; ++s) full[s] = (ii == j) ? sbase[s * stride + DG_ * SP_STRIDE + j] : 0.;
+              for (int s = 0; s < S; ++s) full[s] = (ii == j) ? SP(DG_, j, s) : 0.;
               const double Mi = MiL;
               const int ee = j * ns + ii;
               const int t0 = exo[ee], t1 = exo[ee + 1];
-              const double *vb = sbase + NSA * SP_STRIDE + N_SCAL + 5 * nr;
               int t = t0;
               for (; t + 1 < t1; t += 2) {  // two entries per trip: their LDS loads overlap (same summation order)
                 const uint32_t ra = exx[t], rb = exx[t + 1];
@@ -565,8 +630,8 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
                 const double ca = -(double)(int8_t)(ra >> 16) * Mi, cb = -(double)(int8_t)(rb >> 16) * Mi;
                 double va[S], vbv[S];
                 for (int s = 0; s < S; ++s) {
-                  va[s] = vb[s * stride + sa];
-                  vbv[s] = vb[s * stride + sb];
+                  va[s] = vb[sa * S + s];
+                  vbv[s] = vb[sb * S + s];
                 }
                 for (int s = 0; s < S; ++s) {
                   full[s] = fma(ca, va[s], full[s]);
@@ -577,7 +642,7 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
                 const uint32_t rec = exx[t];
                 const int slot = (int)(rec & 0xFFFFu);
                 const double coef = -(double)(int8_t)(rec >> 16) * Mi;
-                for (int s = 0; s < S; ++s) full[s] = fma(coef, vb[s * stride + slot], full[s]);
+                for (int s = 0; s < S; ++s) full[s] = fma(coef, vb[slot * S + s], full[s]);
               }
               for (int s = 0; s < S; ++s) full[s] += fma(dj, rA[s], rB[s]);
             }
@@ -588,12 +653,11 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
             for (int s = 0; s < 4; ++s) hv[s] = (s < S && row) ? __dmul_rn(rH[s < S ? s : 0], full[s < S ? s : 0]) : 0.;
             wave_sum4(hv, hsum);
             for (int s = 0; s < S; ++s) {
-              const double *sp = sbase + s * stride;
               const double hs = hsum[s];
               const double rd = __dmul_rn(rmw[s], dj);
               val[s] = (lane == 0)
-                           ? fma(-iRC[s], hs, __dmul_rn(rd, sp[PR_ * SP_STRIDE]) -
-                                                  __dmul_rn(ric[s], sp[CPI_ * SP_STRIDE + j] - sp[CPI_ * SP_STRIDE + nm]))
+                           ? fma(-iRC[s], hs, __dmul_rn(rd, SP(PR_, 0, s)) -
+                                                  __dmul_rn(ric[s], SP(CPI_, j, s) - SP(CPI_, nm, s)))
                            : (lane < ns ? fma(iR[s], full[s], __dmul_rn(rd, rP[s])) : 0.);
             }
           }
@@ -612,24 +676,20 @@ __global__ void __launch_bounds__(THREADS) chem_kernel(MechView mv, ChemArgs a, 
           for (int s = 0; s < S; ++s) val[s] = 0.;
           if (lane < ns) {
             if (c < 2) {
-              for (int s = 0; s < S; ++s) val[s] = sbase[s * stride + (c == 0 ? WS0_ : WS1_) * SP_STRIDE + lane];
+              for (int s = 0; s < S; ++s) val[s] = SP(c == 0 ? WS0_ : WS1_, lane, s);
             } else {
               const int j = c - 2;
               const double dj = mv.dinvm[j];
-              const double *vb = sbase + NSA * SP_STRIDE + N_SCAL + 5 * nr;
               if (lane == j)
-                for (int s = 0; s < S; ++s) val[s] = sbase[s * stride + DG_ * SP_STRIDE + j];
+                for (int s = 0; s < S; ++s) val[s] = SP(DG_, j, s);
               const int t1 = exo[j * ns + lane + 1];
               for (int t = exo[j * ns + lane]; t < t1; ++t) {
                 const uint32_t rec = exx[t];
                 const int slot = (int)(rec & 0xFFFFu);
                 const double coef = -(double)(int8_t)(rec >> 16) * Mk;
-                for (int s = 0; s < S; ++s) val[s] = fma(coef, vb[s * stride + slot], val[s]);
+                for (int s = 0; s < S; ++s) val[s] = fma(coef, vb[slot * S + s], val[s]);
               }
-              for (int s = 0; s < S; ++s) {
-                const double *sp = sbase + s * stride;
-                val[s] = fma(dj, sp[A_ * SP_STRIDE + lane], val[s]) + sp[B_ * SP_STRIDE + lane];
-              }
+              for (int s = 0; s < S; ++s) val[s] = fma(dj, SP(A_, lane, s), val[s]) + SP(B_, lane, s);
             }
           }
           if (lane <= ns)
