@@ -329,11 +329,45 @@ btd_solve_kernel(const int *nblocks, int bs, const double *factors, const long *
 template <typename T>
 constexpr int kAhead = sizeof(T) == 8 ? 2 : 3;
 
+// One wave's share of a product with a block: what it loads (d: the columns 4 k + q, e: those beyond the groups of four, for
+// wave 0; a, c: the vectors that form the next product's vector a - c * (this product)), and the arithmetic.
+template <typename T, int N>
+struct Product {
+  static constexpr int K = N / 4, E = N % 4;
+  struct Ahead {
+    T d[K > 0 ? K : 1], e[E > 0 ? E : 1];
+    double a, c;
+  };
+  const T *DI;  // the lane's row of the system's inverses
+  int q, lane;
+  double v;  // the vector, lane = row
+  __device__ __forceinline__ void columns(Ahead &B, int blk) const {
+    const T *D = DI + (long)blk * (N * N);
+#pragma unroll
+    for (int k = 0; k < E; ++k) B.e[k] = D[(4 * K + k) * N];
+    D += q * N;
+#pragma unroll
+    for (int k = 0; k < K; ++k) B.d[k] = D[4 * k * N];
+  }
+  __device__ __forceinline__ void multiply(const Ahead &B, double *out) const {
+    double acc = 0.;
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc = fma((double)B.d[k], lane_value(v, 4 * k + q), acc);
+    if (E > 0 && q == 0) {
+#pragma unroll
+      for (int k = 0; k < E; ++k) acc = fma((double)B.e[k], lane_value(v, 4 * K + k), acc);
+    }
+    out[lane] = acc;
+  }
+  __device__ __forceinline__ double sum(const double (*p)[64]) const {
+    return (p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane]);
+  }
+};
+
 template <typename T, int N>
 __global__ void __launch_bounds__(512) btd_twist_solve_kernel(const int *nblocks, const double *values, const long *voff,
                                                               const T *dinv, const long *doff, const double *rhs,
                                                               double *x, const long *xoff) {
-  constexpr int K = N / 4, E = N % 4;
   __shared__ double part[2][2][4][64];  // [parity of the product][chain][wave][row]
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -345,47 +379,23 @@ __global__ void __launch_bounds__(512) btd_twist_solve_kernel(const int *nblocks
   const bool act = lane < N;
   const int rl = act ? lane : 0;
   const int m = (nb - 1) / 2;
-  const T *DI = dinv + doff[sys] + rl;
   const double *b = rhs + xoff[sys];
   double *X = x + xoff[sys];
   const double *sub = values + voff[sys] + (long)nb * (N * N);
   const double *sup = sub + (long)(nb - 1) * N;
 
-  // What a product needs: the block's columns of this wave (e: those beyond the groups of four, for wave 0), and the two
-  // vectors a, c that form the next product's vector a - c * (this product). y_i is kept in X. Every product loads the same
-  // number of words without a branch (clamped where there is nothing to load), so that a wait counts the loads it
-  // needs and leaves the later products' in flight.
-  struct Ahead {
-    T d[K > 0 ? K : 1], e[E > 0 ? E : 1];
-    double a, c;
-  };
-  auto columns = [&](Ahead &B, int blk) {
-    const T *D = DI + (long)blk * (N * N);
-#pragma unroll
-    for (int k = 0; k < E; ++k) B.e[k] = D[(4 * K + k) * N];
-    D += q * N;
-#pragma unroll
-    for (int k = 0; k < K; ++k) B.d[k] = D[4 * k * N];
-  };
-  double v;
-  auto multiply = [&](const Ahead &B, double *out) {
-    double acc = 0.;
-#pragma unroll
-    for (int k = 0; k < K; ++k) acc = fma((double)B.d[k], lane_value(v, 4 * k + q), acc);
-    if (E > 0 && q == 0) {
-#pragma unroll
-      for (int k = 0; k < E; ++k) acc = fma((double)B.e[k], lane_value(v, 4 * K + k), acc);
-    }
-    out[lane] = acc;
-  };
-  auto sum = [&](const double (*p)[64]) { return (p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane]); };
+  // Every product loads the same number of words without a branch (clamped where there is nothing to load), so that a
+  // wait counts the loads it needs and leaves the later products' in flight. y_i is kept in X.
+  using Ahead = typename Product<T, N>::Ahead;
+  Product<T, N> w{dinv + doff[sys] + rl, q, lane};
+  double &v = w.v;
   if (nb == 1) {
     Ahead B;
     v = b[rl];
-    columns(B, 0);
-    multiply(B, part[0][0][q]);
+    w.columns(B, 0);
+    w.multiply(B, part[0][0][q]);
     __syncthreads();
-    if (q == 0 && act) X[lane] = sum(part[0][0]);
+    if (q == 0 && act) X[lane] = w.sum(part[0][0]);
     return;
   }
 
@@ -403,7 +413,7 @@ __global__ void __launch_bounds__(512) btd_twist_solve_kernel(const int *nblocks
   if (len > 0 && act) X[at(block(0))] = v;  // every wave writes, and later reads, its own
   auto operands = [&](Ahead &B, int s) {
     const int i = block(s), j = block(s + 1);
-    columns(B, i);
+    w.columns(B, i);
     B.c = (top == (s < len) ? sub : sup)[at(min(min(i, j), nb - 2))];
   };
   auto addend = [&](Ahead &B, int s) { B.a = (s < len ? b : X)[at(block(s + 1))]; };
@@ -417,7 +427,7 @@ __global__ void __launch_bounds__(512) btd_twist_solve_kernel(const int *nblocks
   const bool out = act && q == 0;
   auto product = [&](Ahead &B, int g) {
     const int s = g - off;
-    multiply(B, part[g & 1][chain][q]);
+    w.multiply(B, part[g & 1][chain][q]);
     // Loads that do not depend on this product go before the barrier. The addend has to be here by then: x may be rhs, and
     // behind the barrier other waves write what it was read from.
     const double a = s == len ? last : B.a, c = B.c;
@@ -426,12 +436,12 @@ __global__ void __launch_bounds__(512) btd_twist_solve_kernel(const int *nblocks
     __syncthreads();
     if (g == L - 1) {
 #pragma clang fp contract(off)
-      const double tt = m > 0 ? ct * sum(part[g & 1][0]) : 0., tb = cb * sum(part[g & 1][1]);
+      const double tt = m > 0 ? ct * w.sum(part[g & 1][0]) : 0., tb = cb * w.sum(part[g & 1][1]);
       last = v;
       v = bm - tt - tb;
     } else if ((unsigned)s <= (unsigned)(2 * len)) {
       const bool in = s < len;
-      const double mv = sum(part[g & 1][chain]);
+      const double mv = w.sum(part[g & 1][chain]);
       v = fma(-c, mv, a);
       // y of the next block or x of this one (both chains write x_m, the same)
       if (in ? act : out) X[at(block(in ? s + 1 : s))] = in ? v : mv;
@@ -445,6 +455,108 @@ __global__ void __launch_bounds__(512) btd_twist_solve_kernel(const int *nblocks
       product(buf[k], g + k);
     }
   }
+}
+
+// The same solve with the two chains of a system on two compute units, for few systems of long chains: inwards and outwards one
+// workgroup of four waves per chain (blockIdx.x = 2 system + chain), in between the middle block. Both chains of a system
+// on one compute unit are bound by its cache fills (45 KB a product at 53); three launches cost about 8 us more.
+// Measured (53x53, us, FP64 / FP32): one chain of 126 blocks 150 -> 100 / 108 -> 82, 48 chains of 62..254 312 -> 215 / 232 -> 176,
+// 128 chains 397 -> 263 / 238 -> 184. Bitwise the same.
+template <typename T, int N>
+__global__ void __launch_bounds__(256) btd_chain_solve_kernel(const int *nblocks, const double *values, const long *voff,
+                                                              const T *dinv, const long *doff, const double *rhs,
+                                                              double *x, const long *xoff, int inwards) {
+  __shared__ double part[2][4][64];
+  const int sys = blockIdx.x >> 1;
+  const bool top = (blockIdx.x & 1) == 0;
+  const int lane = threadIdx.x & 63;
+  const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nb = __builtin_amdgcn_readfirstlane(nblocks[sys]);
+  const int m = (nb - 1) / 2, len = top ? m : nb - 1 - m;
+  if (len == 0) return;
+  const bool act = lane < N;
+  const int rl = act ? lane : 0;
+  const double *b = rhs + xoff[sys];
+  double *X = x + xoff[sys];
+  const double *sub = values + voff[sys] + (long)nb * (N * N);
+  const double *sup = sub + (long)(nb - 1) * N;
+  Product<T, N> w{dinv + doff[sys] + rl, q, lane};
+  const int first = top ? 0 : nb - 1, dir = top ? 1 : -1;
+  auto block = [&](int s) { return first + dir * max(len - abs(len - s), 0); };
+  auto at = [&](int i) { return (unsigned)(i * N + rl); };
+  auto coupling = [&](int s) { return (top == (s < len) ? sub : sup)[at(min(min(block(s), block(s + 1)), nb - 2))]; };
+  const double *from = inwards ? b : X;
+  const int s0 = inwards ? 0 : len + 1, s1 = inwards ? len - 1 : 2 * len + 1;  // products s0 .. s1 - 1
+  if (inwards) {
+    w.v = b[at(block(0))];
+    if (act) X[at(block(0))] = w.v;  // every wave writes, and later reads, its own
+  } else {
+    w.v = fma(-coupling(len), X[at(m)], X[at(block(s0))]);
+  }
+  typename Product<T, N>::Ahead buf[kAhead<T>];
+#pragma unroll
+  for (int k = 0; k < kAhead<T>; ++k) {
+    w.columns(buf[k], block(s0 + k));
+    buf[k].c = coupling(s0 + k);
+    buf[k].a = from[at(block(s0 + k + 1))];
+  }
+  auto product = [&](typename Product<T, N>::Ahead &B, int s) {
+    w.multiply(B, part[s & 1][q]);
+    const double a = B.a, c = B.c;
+    asm volatile("" ::"v"(B.a));  // as above: x may be rhs
+    w.columns(B, block(s + kAhead<T>));
+    B.c = coupling(s + kAhead<T>);
+    __syncthreads();
+    const double mv = w.sum(part[s & 1]);
+    w.v = fma(-c, mv, a);
+    if (inwards ? act : act && q == 0) X[at(block(inwards ? s + 1 : s))] = inwards ? w.v : mv;
+    B.a = from[at(block(s + kAhead<T> + 1))];
+  };
+  for (int s = s0; s < s1; s += kAhead<T>) {
+#pragma unroll
+    for (int k = 0; k < kAhead<T>; ++k) {
+      if (s + k >= s1) break;
+      product(buf[k], s + k);
+    }
+  }
+}
+
+template <typename T, int N>
+__global__ void __launch_bounds__(512) btd_middle_solve_kernel(const int *nblocks, const double *values, const long *voff,
+                                                               const T *dinv, const long *doff, const double *rhs,
+                                                               double *x, const long *xoff) {
+  __shared__ double part[2][2][4][64];
+  const int sys = blockIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int chain = wave >> 2, q = wave & 3;
+  const int nb = __builtin_amdgcn_readfirstlane(nblocks[sys]);
+  const int m = (nb - 1) / 2;
+  const bool act = lane < N, below = nb > 1;
+  const int rl = act ? lane : 0;
+  const double *b = rhs + xoff[sys];
+  double *X = x + xoff[sys];
+  const double *sub = values + voff[sys] + (long)nb * (N * N);
+  const double *sup = sub + (long)(nb - 1) * N;
+  auto at = [&](int i) { return (unsigned)(i * N + rl); };
+  Product<T, N> w{dinv + doff[sys] + rl, q, lane};
+  typename Product<T, N>::Ahead A, B;
+  const int near = chain == 0 ? max(m - 1, 0) : min(m + 1, nb - 1);
+  w.columns(A, near);
+  w.columns(B, m);
+  const double bm = b[at(m)], ct = m > 0 ? sub[at(m - 1)] : 0., cb = below ? sup[at(m)] : 0.;
+  w.v = X[at(near)];
+  w.multiply(A, part[0][chain][q]);
+  asm volatile("" ::"v"(bm));
+  __syncthreads();
+  {
+#pragma clang fp contract(off)
+    const double tt = m > 0 ? ct * w.sum(part[0][0]) : 0., tb = below ? cb * w.sum(part[0][1]) : 0.;
+    w.v = bm - tt - tb;
+  }
+  w.multiply(B, part[1][chain][q]);
+  __syncthreads();
+  if (wave == 0 && act) X[at(m)] = w.sum(part[1][0]);
 }
 
 template <typename T>
@@ -494,20 +606,46 @@ int launch_btd_solve(int nsys, const int *nblocks, int bs, const double *values,
 }
 
 template <typename T>
+using ChainSolve = void (*)(const int *, const double *, const long *, const T *, const long *, const double *, double *,
+                            const long *, int);
+template <typename T, int... I>
+static ChainSolve<T> chain_solve_kernel(int bs, std::integer_sequence<int, I...>) {
+  constexpr ChainSolve<T> tab[] = {&btd_chain_solve_kernel<T, I + 1>...};
+  return tab[bs - 1];
+}
+template <typename T, int... I>
+static InvSolve<T> middle_solve_kernel(int bs, std::integer_sequence<int, I...>) {
+  constexpr InvSolve<T> tab[] = {&btd_middle_solve_kernel<T, I + 1>...};
+  return tab[bs - 1];
+}
+
+template <typename T>
 int launch_btd_inv_solve(int nsys, const int *nblocks, int bs, const double *values, const long *voff,
                          const T *dinv, const long *doff, const double *rhs, double *x, const long *xoff,
-                         hipStream_t st) {
+                         hipStream_t st, long blocks) {
   if (nsys <= 0) return GF_OK;
   if (bs < 1 || bs > 64) return fail(GF_ERR_UNSUPPORTED, "block size must be in 1..64");
-  const auto kern = inv_solve_kernel<T>(bs, std::make_integer_sequence<int, 64>{});
-  hipLaunchKernelGGL(kern, dim3(nsys), dim3(512), 0, st, nblocks, values, voff, dinv, doff, rhs, x, xoff);
+  constexpr auto sizes = std::make_integer_sequence<int, 64>{};
+  // Where the caller knows the number of blocks: a compute unit per chain while there are enough of them (256; 192 systems
+  // of 53: 433 against 431 us, 512: 966 against 987), and chains long enough for the two launches more (one workgroup per
+  // system against this, one system of 10 blocks of 10: 8 / 11 us, of 40: 22 / 21, of 40 of 53: 51 / 38).
+  if (nsys <= 128 && blocks >= 40L * nsys) {
+    const auto chain = chain_solve_kernel<T>(bs, sizes);
+    hipLaunchKernelGGL(chain, dim3(2 * nsys), dim3(256), 0, st, nblocks, values, voff, dinv, doff, rhs, x, xoff, 1);
+    hipLaunchKernelGGL(middle_solve_kernel<T>(bs, sizes), dim3(nsys), dim3(512), 0, st, nblocks, values, voff, dinv, doff,
+                       rhs, x, xoff);
+    hipLaunchKernelGGL(chain, dim3(2 * nsys), dim3(256), 0, st, nblocks, values, voff, dinv, doff, rhs, x, xoff, 0);
+  } else {
+    hipLaunchKernelGGL(inv_solve_kernel<T>(bs, sizes), dim3(nsys), dim3(512), 0, st, nblocks, values, voff, dinv, doff,
+                       rhs, x, xoff);
+  }
   if (hipGetLastError() != hipSuccess) return fail(GF_ERR_HIP, "btd inverse solve launch failed");
   return GF_OK;
 }
 
 template int launch_btd_inv_solve<double>(int, const int *, int, const double *, const long *, const double *,
-                                          const long *, const double *, double *, const long *, hipStream_t);
+                                          const long *, const double *, double *, const long *, hipStream_t, long);
 template int launch_btd_inv_solve<float>(int, const int *, int, const double *, const long *, const float *,
-                                         const long *, const double *, double *, const long *, hipStream_t);
+                                         const long *, const double *, double *, const long *, hipStream_t, long);
 
 }  // namespace gfa

@@ -288,14 +288,20 @@ struct Psitc {
     return factor(fl, o.lu_precision);
   }
 
+  long blocks(const std::vector<int> &fl) const {
+    long n = 0;
+    for (int f : fl) n += b->nzi[f];
+    return n;
+  }
+
   int solve(const std::vector<int> &fl, int precision) {
     if (fl.empty()) return GF_OK;
     GF_TRY(systems(fl));
     if (precision == 32)
       return launch_btd_inv_solve<float>((int)fl.size(), b->sys_nb, b->ns, b->J, b->sys_v, b->D32, b->sys_l, b->R,
-                                         b->dX, b->sys_x, st);
+                                         b->dX, b->sys_x, st, blocks(fl));
     return launch_btd_inv_solve<double>((int)fl.size(), b->sys_nb, b->ns, b->J, b->sys_v, b->L, b->sys_l, b->R, b->dX,
-                                        b->sys_x, st);
+                                        b->sys_x, st, blocks(fl));
   }
 
   int run(int *iterations, int *converged, double *residual, double *min_ds) {
@@ -748,10 +754,12 @@ int factored(const gf_flamelet_batch *b, const int *flags, std::vector<int> &fl)
   return GF_OK;
 }
 
-int transient_solve(gf_flamelet_batch *b, int n, const double *r, double *out, hipStream_t st) {
+int transient_solve(gf_flamelet_batch *b, int n, long blocks, const double *r, double *out, hipStream_t st) {
   if (b->tr_prec == 32)
-    return launch_btd_inv_solve<float>(n, b->sys_nb, b->ns, b->J, b->sys_v, b->D32, b->sys_l, r, out, b->sys_x, st);
-  return launch_btd_inv_solve<double>(n, b->sys_nb, b->ns, b->J, b->sys_v, b->L, b->sys_l, r, out, b->sys_x, st);
+    return launch_btd_inv_solve<float>(n, b->sys_nb, b->ns, b->J, b->sys_v, b->D32, b->sys_l, r, out, b->sys_x, st,
+                                       blocks);
+  return launch_btd_inv_solve<double>(n, b->sys_nb, b->ns, b->J, b->sys_v, b->L, b->sys_l, r, out, b->sys_x, st,
+                                      blocks);
 }
 }  // namespace
 
@@ -794,7 +802,7 @@ int gf_flamelet_batch_transient_solve(gf_flamelet_batch *b, const int *flags, co
   GF_TRY(factored(b, flags, fl));
   if (fl.empty()) return GF_OK;
   GF_TRY(s.systems(fl));
-  GF_TRY(transient_solve(b, (int)fl.size(), r, out, s.st));
+  GF_TRY(transient_solve(b, (int)fl.size(), s.blocks(fl), r, out, s.st));
   return s.sync();
 }
 
@@ -822,7 +830,7 @@ int gf_flamelet_batch_transient_newton(gf_flamelet_batch *b, const int *flags, c
   GF_TRY(s.up(b->flag, s.flags_of(fl)));
   GF_TRY(s.up(b->fval, std::vector<double>(h, h + b->B)));
   GF_TRY(s.systems(fl));
-  GF_TRY(transient_solve(b, (int)fl.size(), r, d, s.st));
+  GF_TRY(transient_solve(b, (int)fl.size(), s.blocks(fl), r, d, s.st));
   GF_TRY(launch_fb_stage_update(b->view, b->flag, d, x, b->fres, s.st));
   GF_TRY(launch_fb_unpack(b->view, b->flag, b->ddof0, x, b->X, 1, s.st));
   GF_TRY(s.chem(b->X, fl, false));

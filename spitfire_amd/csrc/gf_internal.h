@@ -287,5 +287,5 @@ int launch_btd_inv_factor_small(int nsys, const int *nblocks, int bs, const doub
 template <typename T>
 int launch_btd_inv_solve(int nsys, const int *nblocks, int bs, const double *values, const long *voff,
                          const T *dinv, const long *doff, const double *rhs, double *x, const long *xoff,
-                         hipStream_t st);
+                         hipStream_t st, long blocks = 0);  // blocks: of all systems together, 0 if not known
 }  // namespace gfa

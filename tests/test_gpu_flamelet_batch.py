@@ -412,3 +412,34 @@ def test_fused_stage_iteration_and_norms(npts, mech_c1_data):
     rr = torch.where(on, hd * (gamma * fr + prior) - (xr - x0), torch.full_like(x0, 7.))
     assert torch.equal(x, xr) and torch.equal(f, fr) and torch.equal(r, rr)
     assert np.array_equal(out, np.where(flags, norms(r.cpu().numpy()), -1.))
+
+
+@pytest.mark.parametrize('precision', [64, 32])
+def test_solve_routes_of_few_and_many_flamelets_agree_bitwise(precision, mech_c1_data):
+    """A few long flamelets are solved with a compute unit per chain, more than 128 with one per system: the same sums in the same
+    order. Lengths around the middle block and the products in flight. Tolerance: none."""
+    import torch
+    from spitfire_amd import _native
+    from spitfire_amd.flamelet import FlameletBatch
+    from spitfire_amd.mechanism import ChemicalMechanismSpec
+    m = ChemicalMechanismSpec(mech_c1_data)
+    npts, ns = [90, 61, 60, 4, 5], m.n_species
+    lib, dev = _native.lib(), torch.device('cuda:0')
+    rng = np.random.default_rng(2)
+    few = [rng.standard_normal((n - 2) * ns) for n in npts]
+    got = []
+    for copies in (1, 26):
+        fb = FlameletBatch(_flamelets(m, [10.] * len(npts) * copies, npts * copies))
+        B = len(npts) * copies
+        flags, pre = np.ones(B, dtype=np.int32), np.full(B, 1e-7)
+        x, r = torch.tensor(fb._x0, device=dev), torch.tensor(np.concatenate(few * copies), device=dev)
+        out = torch.zeros_like(r)
+        torch.cuda.synchronize()
+        # (as a time step does: the right-hand side, which also forms the boundary points' mixtures, comes first)
+        _native.check(lib.gf_flamelet_batch_transient_rhs(fb._h, _native.iptr(flags), x.data_ptr(), out.data_ptr()))
+        _native.check(lib.gf_flamelet_batch_transient_setup(fb._h, _native.iptr(flags), x.data_ptr(), _native.dptr(pre),
+                                                            precision))
+        _native.check(lib.gf_flamelet_batch_transient_solve(fb._h, _native.iptr(flags), r.data_ptr(), out.data_ptr()))
+        got.append(out.cpu().numpy())
+    n = few[0].size + few[1].size + few[2].size + few[3].size + few[4].size
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1][:n]) and np.array_equal(got[0], got[1][-n:])
