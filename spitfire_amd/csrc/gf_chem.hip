@@ -28,7 +28,10 @@
 // neighbouring words, and a reaction's record is read whole, its short lists unrolled with factors of one beyond their
 // ends: field by field, with loops of one to four trips around dependent loads, P1 took 41,000 cycles for a group
 // of four states with derivatives and now takes 32,000. 53 species, 325 reactions, before and after (us): RHS of 512 / 7,600 /
-// 100,003 states 16.5 / 85 / 880 -> 14.7 / 78 / 803; with Jacobian 512 / 4,000 / 100,000 38 / 169 / 3,938 -> 33 / 155 / 3,596.
+// 100,003 states 16.5 / 85 / 880 -> 14.7 / 78 / 795; with Jacobian 512 / 4,000 / 100,000 38 / 169 / 3,938 -> 31 / 138 / 3,196.
+// Of the latter, P3: the blocks' offsets instead of pointers that may be null (those were stored through as flat addresses,
+// which every later LDS load waits for) 3,572 -> 3,429, and what only lane 0 needs read by all lanes ahead of a column's
+// sums instead of under its condition, four times 200 cycles a column, -> 3,196.
 // Tried without gain: P3's slot sums dealt to the lanes by length through LDS (every lane busy, but the same words through
 // the banks again: 38,000 -> 45,000 cycles a group); 16 waves at 128 registers (226 spilled).
 #include "gf_internal.h"
@@ -571,16 +574,13 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(JA
       // contraction choices cannot differ between launch shapes and every shape gives bitwise the same Jacobian.
       int nact = 0;
       double iR[S], iRC[S], ric[S], rmw[S];  // 1/rho, 1/(rho cp), rhs0/cp, -rho M of each state
-      double *jb[S];  // Jacobian block of each state (nullptr: none)
+      long jo[S];  // offset of each state's Jacobian block (negative: none)
       for (int s = 0; s < S; ++s) {
-        jb[s] = nullptr;
+        jo[s] = -1;
         if (first + s < a.n) {
           nact = s + 1;
           const long q = a.sel ? (long)a.sel[first + s] : first + s;
-          if (a.jac) {
-            const long off = a.js_off ? a.js_off[q] : q * a.js_i;
-            if (off >= 0) jb[s] = a.jac + off;
-          }
+          if (a.jac) jo[s] = a.js_off ? a.js_off[q] : q * a.js_i;
         }
         iR[s] = 1. / SC(S_RHO, s);
         iRC[s] = 1. / (SC(S_RHO, s) * SC(S_CP, s));
@@ -592,7 +592,7 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(JA
         // per-row values of every state, loaded once for all the columns this wave assembles
         const int iiL = lane - 1;
         const bool rowL = lane >= 1 && lane <= ns;
-        double rA[S], rB[S], rH[S], rP[S];
+        double rA[S], rB[S], rH[S], rP[S], rD[S], cn[S];
         // the row's molecular weight (loaded here: in the column loop the Jacobian stores could alias it)
         const double MiL = rowL ? mv.mw[iiL] : 0.;
         for (int s = 0; s < S; ++s) {
@@ -600,6 +600,8 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(JA
           rB[s] = rowL ? SP(B_, iiL, s) : 0.;
           rH[s] = rowL ? SP(H_, iiL, s) : 0.;
           rP[s] = lane < ns ? SP(PR_, lane, s) : 0.;
+          rD[s] = rowL ? SP(DG_, iiL, s) : 0.;
+          cn[s] = SP(CPI_, nm, s);
         }
         for (int c = wave; c < ns; c += NW) {
           double val[S];
@@ -613,13 +615,16 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(JA
             }
           } else {
             const int j = c - 1;
-            const double dj = mv.dinvm[j];
+            const double dj = imw[j] - imw[nm];
             const int ii = lane - 1;  // species row; lane ns is the last species (temperature row only)
             const bool row = lane >= 1 && lane <= ns;
-            double full[S];
-            for (int s = 0; s < S; ++s) full[s] = 0.;
+            // (what lane 0 alone needs is read by all, ahead of the sums: a load under its condition waits by itself)
+            double full[S], cj[S];
+            for (int s = 0; s < S; ++s) {
+              full[s] = (row && ii == j) ? rD[s] : 0.;
+              cj[s] = SP(CPI_, j, s) - cn[s];
+            }
             if (row) {
-              for (int s = 0; s < S; ++s) full[s] = (ii == j) ? SP(DG_, j, s) : 0.;
               const double Mi = MiL;
               const int ee = j * ns + ii;
               const int t0 = exo[ee], t1 = exo[ee + 1];
@@ -654,16 +659,16 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(JA
             wave_sum4(hv, hsum);
             for (int s = 0; s < S; ++s) {
               const double hs = hsum[s];
-              const double rd = __dmul_rn(rmw[s], dj);
-              val[s] = (lane == 0)
-                           ? fma(-iRC[s], hs, __dmul_rn(rd, SP(PR_, 0, s)) -
-                                                  __dmul_rn(ric[s], SP(CPI_, j, s) - SP(CPI_, nm, s)))
-                           : (lane < ns ? fma(iR[s], full[s], __dmul_rn(rd, rP[s])) : 0.);
+              const double rd = __dmul_rn(rmw[s], dj), rp = __dmul_rn(rd, rP[s]);
+              const double t = fma(-iRC[s], hs, fma(rd, rP[s], -__dmul_rn(ric[s], cj[s])));
+              val[s] = lane == 0 ? t : fma(iR[s], full[s], rp);
             }
           }
-          if (lane < ns)
-            for (int s = 0; s < nact; ++s)
-              if (jb[s]) jb[s][(long)c * ns + lane] = val[s];
+          if (lane < ns) {
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+              if (jo[s] >= 0) a.jac[jo[s] + c * ns + lane] = val[s];
+          }
         }
       }
       if (a.sens) {
@@ -679,7 +684,7 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(JA
               for (int s = 0; s < S; ++s) val[s] = SP(c == 0 ? WS0_ : WS1_, lane, s);
             } else {
               const int j = c - 2;
-              const double dj = mv.dinvm[j];
+              const double dj = imw[j] - imw[nm];
               if (lane == j)
                 for (int s = 0; s < S; ++s) val[s] = SP(DG_, j, s);
               const int t1 = exo[j * ns + lane + 1];
