@@ -17,12 +17,12 @@
 // eliminated from both ends at once (twisted factorisation, halving the serial chain), every Schur-updated
 // diagonal block is inverted by blocked Gauss-Jordan elimination with partial pivoting on the matrix cores (gf_twist.hip)
 // and stored as its inverse, so no L blocks are stored and both sweeps of a solve are matrix-vector products.
+#include "gf_btd_index.h"
 #include "gf_internal.h"
+#include "gf_wave.h"
 #include "../../include/griffon_amd.h"
 
 #include <utility>
-#include "gf_wave.h"
-
 
 namespace gfa {
 
@@ -235,7 +235,7 @@ btd_solve_kernel(const int *nblocks, int bs, const double *factors, const long *
   const double *L = lval + loff[sys];
   const double *b = rhs + xoff[sys];
   double *X = x + xoff[sys];
-  const double *sup = D + nb * nb2 + (long)(nb - 1) * bs;
+  auto sup = [&](int i) { return D[btd_sup(nb, bs, i) + rl]; };
   double B[2][NC];
   auto load = [&](double(&to)[NC], const double *from) {
 #pragma unroll
@@ -294,12 +294,12 @@ btd_solve_kernel(const int *nblocks, int bs, const double *factors, const long *
     const int n1 = max(i - 1, 0), n2 = max(i - 2, 0);
     load(B[1], D + n1 * nb2);
     y1 = X[(long)n1 * bs + rl];
-    s1 = sup[(long)n1 * bs + rl];
+    s1 = sup(n1);
     backward(B[0], i, y0, s0);
     if (i == 0) break;
     load(B[0], D + n2 * nb2);
     y0 = X[(long)n2 * bs + rl];
-    s0 = sup[(long)n2 * bs + rl];
+    s0 = sup(n2);
     backward(B[1], i - 1, y1, s1);
   }
 }

@@ -197,3 +197,45 @@ def test_lapack_factor_and_solve_edges(bs):
             r[1:] += sub * xs[:-1]
             r[:-1] += sup * xs[1:]
         assert np.max(np.abs(r.ravel() - rhs[s])) <= tol * np.max(np.abs(rhs[s]))
+
+
+@pytest.mark.parametrize('sizes', [[1], [3, 1], [1, 2, 1]])
+@pytest.mark.parametrize('bs', [1, 8, 53, 64])
+def test_lapack_solve_ends_on_a_one_block_system(bs, sizes):
+    """A one-block system has no couplings, and as the last of its batch nothing behind its block. Tolerance: 1,000 N eps of the
+    diagonally dominant systems' right-hand sides."""
+    import torch
+    from spitfire_amd import _native
+    rng = np.random.default_rng(bs)
+    values, dense, rhs = [], [], []
+    for n in sizes:
+        V = rng.standard_normal((n, bs, bs)) + (4. + 2. * bs) * np.eye(bs)
+        lo, up = 0.1 * rng.standard_normal((n - 1, bs)), 0.1 * rng.standard_normal((n - 1, bs))
+        values.append(np.concatenate([V.transpose(0, 2, 1).ravel(), lo.ravel(), up.ravel()]))
+        A = np.zeros((n * bs, n * bs))
+        for k in range(n):
+            A[k * bs:(k + 1) * bs, k * bs:(k + 1) * bs] = V[k]
+        for k in range(n - 1):
+            A[(k + 1) * bs:(k + 2) * bs, k * bs:(k + 1) * bs] = np.diag(lo[k])
+            A[k * bs:(k + 1) * bs, (k + 1) * bs:(k + 2) * bs] = np.diag(up[k])
+        dense.append(A)
+        rhs.append(rng.standard_normal(n * bs))
+    dev = torch.device('cuda:0')
+    nb = np.asarray(sizes)
+    offsets = [np.cumsum(np.r_[0, a])[:-1].astype(np.int64) for a in ([v.size for v in values], nb * bs * bs, nb * bs)]
+    V, b = (torch.tensor(np.concatenate(a), device=dev) for a in (values, rhs))
+    n, vo, lo, xo = (torch.tensor(a, device=dev) for a in (nb.astype(np.int32), *offsets))
+    L = torch.zeros(int((nb * bs * bs).sum()), device=dev, dtype=torch.float64)
+    P = torch.zeros(int((nb * bs).sum()), device=dev, dtype=torch.int32)
+    x = torch.zeros_like(b)
+    st = torch.cuda.current_stream().cuda_stream
+    lib = _native.lib()
+    _native.check(lib.gf_batch_btddod_full_factorize(len(sizes), n.data_ptr(), bs, V.data_ptr(), vo.data_ptr(), L.data_ptr(),
+                                                     lo.data_ptr(), P.data_ptr(), xo.data_ptr(), st))
+    _native.check(lib.gf_batch_btddod_full_solve(len(sizes), n.data_ptr(), bs, V.data_ptr(), vo.data_ptr(), L.data_ptr(),
+                                                 lo.data_ptr(), P.data_ptr(), xo.data_ptr(), b.data_ptr(), x.data_ptr(),
+                                                 xo.data_ptr(), st))
+    got = x.cpu().numpy()
+    for s in range(len(sizes)):
+        g = got[offsets[2][s]:offsets[2][s] + nb[s] * bs]
+        assert np.max(np.abs(dense[s] @ g - rhs[s])) <= 1e3 * bs * 2.2e-16 * np.max(np.abs(rhs[s]))
