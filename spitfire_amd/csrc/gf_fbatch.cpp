@@ -191,9 +191,26 @@ struct Psitc {
       else
         for (int i = 0; i < b->nzi[f] + 2; ++i) sel.push_back((int)(p0 + i));
     }
+    return chem_at(X, sel, jac);
+  }
+
+  // The streams of the boundary points never change, and neither do their mixtures. Every right-hand side forms them again with
+  // its flamelet's interior points; a Jacobian forms interior points only and reads the boundary ones from here or there.
+  // (Launch shape untimed: timing a handful of points would cost a batch's creation fifteen launches.)
+  int boundary_mixtures() {
+    std::vector<int> sel;
+    for (int f = 0; f < b->B; ++f) {
+      sel.push_back((int)b->pt0[f]);
+      sel.push_back((int)(b->pt0[f] + b->nzi[f] + 1));
+    }
+    return chem_at(b->X, sel, false, true);
+  }
+
+  int chem_at(const double *X, const std::vector<int> &sel, bool jac, bool untimed = false) {
     if (sel.empty()) return GF_OK;
     GF_TRY(up(b->sel, sel));
     ChemIO io;
+    io.no_tune = untimed;
     io.n = (int)sel.size();
     io.x = X;
     io.xs_i = b->ns;
@@ -610,6 +627,7 @@ int gf_flamelet_batch_create(gf_mech *m, int nfl, const int *nzi, double pressur
     v.maxNV = std::max(v.maxNV, (long)nzi[f] * ns);
   }
   T(launch_fb_stencils(v, b->dz, b->ddz0, nullptr, b->cmaj, b->csub, b->csup, b->mco, b->nco, st));
+  if (rc == GF_OK) rc = Psitc{b, {}, st}.boundary_mixtures();
   if (rc == GF_OK && hipStreamSynchronize(st) != hipSuccess) rc = fail(GF_ERR_HIP, "stream synchronize failed");
   if (rc != GF_OK) {
     hipFree(b->dmem);

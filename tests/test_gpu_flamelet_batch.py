@@ -443,3 +443,32 @@ def test_solve_routes_of_few_and_many_flamelets_agree_bitwise(precision, mech_c1
         got.append(out.cpu().numpy())
     n = few[0].size + few[1].size + few[2].size + few[3].size + few[4].size
     assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1][:n]) and np.array_equal(got[0], got[1][-n:])
+
+
+@pytest.mark.parametrize('precision', [64, 32])
+def test_time_step_matrix_of_a_fresh_batch(precision, mech_c1_data):
+    """The enthalpy-flux term of the first and last interior points reads the boundary points' heat capacities, also in the
+    matrix that a batch forms before any right-hand side, as integrate_to_steady does: the solution with that matrix is the one
+    after a right-hand side, whatever the batch's memory held. Tolerance: none (the same kernels on the same values)."""
+    import torch
+    from spitfire_amd import _native
+    from spitfire_amd.flamelet import FlameletBatch
+    from spitfire_amd.mechanism import ChemicalMechanismSpec
+    m = ChemicalMechanismSpec(mech_c1_data)
+    npts = [5, 12, 4]
+    fb = FlameletBatch(_flamelets(m, [10.] * 3, npts))
+    lib, dev = _native.lib(), torch.device('cuda:0')
+    flags, pre = np.ones(3, dtype=np.int32), np.full(3, 1e-5)
+    x = torch.tensor(fb._x0, device=dev)
+    r = torch.tensor(np.random.default_rng(3).standard_normal(fb._x0.size), device=dev)
+    got = []
+    for formed in (False, True):
+        out = torch.zeros_like(x)
+        torch.cuda.synchronize()
+        if formed:
+            _native.check(lib.gf_flamelet_batch_transient_rhs(fb._h, _native.iptr(flags), x.data_ptr(), out.data_ptr()))
+        _native.check(lib.gf_flamelet_batch_transient_setup(fb._h, _native.iptr(flags), x.data_ptr(), _native.dptr(pre),
+                                                            precision))
+        _native.check(lib.gf_flamelet_batch_transient_solve(fb._h, _native.iptr(flags), r.data_ptr(), out.data_ptr()))
+        got.append(out.cpu().numpy())
+    assert np.isfinite(got[1]).all() and np.array_equal(got[0], got[1])
