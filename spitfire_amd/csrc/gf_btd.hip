@@ -34,6 +34,109 @@ using wave::lane_value;
 
 constexpr int kLuWaves = 8;
 
+// Whether the magnitude of f is outside 2^-range .. 2^range (zero, infinities and NaN are)
+template <int range>
+__device__ __forceinline__ bool extreme(double f) {
+  const unsigned e = (unsigned)__double2hiint(f) & 0x7fffffffu;
+  return e - ((unsigned)(1023 - range) << 20) > ((unsigned)(2 * range) << 20);
+}
+__device__ __forceinline__ bool finite_bits(unsigned hi) { return (hi & 0x7fffffffu) < 0x7ff00000u; }
+
+// A block in LDS, [column][row], factored by a workgroup step by step as LAPACK's dgetf2 does: nothing but the rows and columns
+// beyond a pivot is touched, so an infinity goes no further than there, and a pivot of zero leaves its column as it is.
+__device__ void plain_lu(double (*A)[64], int *piv, int bs, int t) {
+  constexpr int NT = 64 * kLuWaves;
+  const int lane = t & 63;
+#pragma unroll 1
+  for (int j = 0; j < bs; ++j) {
+    if (t < 64) {
+      double v = -1.;
+      int idx = bs;
+      const double q = lane < bs ? fabs(A[j][lane]) : -1.;
+      if (lane >= j && q >= 0.) {
+        v = q;
+        idx = lane;
+      }
+#pragma unroll 1
+      for (int o = 32; o > 0; o >>= 1) {
+        const double ov = __shfl_xor(v, o, 64);
+        const int oi = __shfl_xor(idx, o, 64);
+        if (ov > v || (ov == v && oi < idx)) {
+          v = ov;
+          idx = oi;
+        }
+      }
+      if (lane == 0) piv[j] = idx >= bs ? j : idx;  // (NaN is not chosen; of nothing else, the diagonal is)
+    }
+    __syncthreads();
+    const int p = piv[j];
+    if (p != j)
+#pragma unroll 1
+      for (int c = t; c < bs; c += NT) {
+        const double q = A[c][j];
+        A[c][j] = A[c][p];
+        A[c][p] = q;
+      }
+    __syncthreads();
+    const double d = A[j][j];
+    if (d != 0.) {
+      const double id = 1. / d;
+#pragma unroll 1
+      for (int k = j + 1 + t; k < bs; k += NT) A[j][k] *= id;
+    }
+    __syncthreads();
+    const int m = bs - j - 1;
+#pragma unroll 1
+    for (int e = t; e < m * m; e += NT) {
+      const int c = j + 1 + e / m, k = j + 1 + e % m;
+      A[c][k] = fma(-A[j][k], A[c][j], A[c][k]);
+    }
+    __syncthreads();
+  }
+}
+
+// X = A^{-1}, column-major in memory, from these factors, with a division for every entry
+__device__ void plain_inverse(const double (*A)[64], const int *piv, int bs, int t, double *X) {
+  constexpr int NT = 64 * kLuWaves;
+#pragma unroll 1
+  for (int e = t; e < bs * bs; e += NT) X[e] = e / bs == e % bs ? 1. : 0.;
+  __syncthreads();
+#pragma unroll 1
+  for (int j = 0; j < bs; ++j) {
+    const int p = piv[j];
+    if (p != j)
+#pragma unroll 1
+      for (int c = t; c < bs; c += NT) {
+        const double q = X[c * bs + j];
+        X[c * bs + j] = X[c * bs + p];
+        X[c * bs + p] = q;
+      }
+    __syncthreads();
+  }
+#pragma unroll 1
+  for (int j = 0; j < bs; ++j) {
+    const int m = bs - j - 1;
+#pragma unroll 1
+    for (int e = t; e < m * bs; e += NT) {
+      const int c = e / m, k = j + 1 + e % m;
+      X[c * bs + k] = fma(-A[j][k], X[c * bs + j], X[c * bs + k]);
+    }
+    __syncthreads();
+  }
+#pragma unroll 1
+  for (int j = bs - 1; j >= 0; --j) {
+#pragma unroll 1
+    for (int c = t; c < bs; c += NT) X[c * bs + j] /= A[j][j];
+    __syncthreads();
+#pragma unroll 1
+    for (int e = t; e < j * bs; e += NT) {
+      const int c = e / j, k = e % j;
+      X[c * bs + k] = fma(-A[j][k], X[c * bs + j], X[c * bs + k]);
+    }
+    __syncthreads();
+  }
+}
+
 // Factors of one system per workgroup: LU with partial pivoting of every diagonal block (LAPACK dgetf2's order of operations,
 // interchanges as dgetrf returns them), in place in values; the L blocks sub_{i-1} D_{i-1}^{-1}, to l; and the
 // pivots. A block is in registers, lane = row, wave w of eight holding columns w, 8 + w, .. (C of them) of it (a) and of what
@@ -48,12 +151,17 @@ constexpr int kLuWaves = 8;
 // search and reciprocal of one column and the way back, one after the other. Measured before and after (us): one
 // system of 60 blocks of 53 10,450 -> 2,260, 24 of 30..61 9,960 -> 2,160, 2,000 of 2..4 1,840 -> 690; 24 of 24x24 blocks
 // 2,850 -> 805, of 10x10 1,050 -> 346. Putting a searching wave's other columns off behind the next barrier gained nothing.
+// Finished rows are updated along with the others, with a multiplier of zero, and U is scaled by reciprocals: where a block has
+// infinities, NaN or a pivot outside 2^-300 .. 2^300 (a singular one among them), that is not what LAPACK's order of operations
+// gives. Such a block is found when it is done, before it is stored; from there on the system is factored in LDS by plain_lu and
+// plain_inverse (behind the loop of the others, so that nothing of it takes their registers).
 template <int C>
-__global__ void __launch_bounds__(64 * kLuWaves) btd_factor_kernel(const int *nblocks, int bs, double *values,
-                                                                   const long *voff, double *lout, const long *loff,
-                                                                   int *piv, const long *poff) {
+__global__ void __launch_bounds__(64 * kLuWaves) __attribute__((amdgpu_waves_per_eu(C == 7 ? 6 : 1)))
+btd_factor_kernel(const int *nblocks, int bs, double *values, const long *voff, double *lout, const long *loff, int *piv,
+                  const long *poff) {
   __shared__ double A[8 * C][64], gb[2][64];  // columns of U for the substitution, [column][lane]; what a step publishes, by
   __shared__ int pb[2];                       // parity of the step
+  __shared__ int odd[2], plain_piv[64];       // by parity of the block: whether it has to be factored plainly
   const int sys = blockIdx.x;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -108,6 +216,8 @@ __global__ void __launch_bounds__(64 * kLuWaves) btd_factor_kernel(const int *nb
     pb[j & 1] = p;
     return below ? l : f;
   };
+  if (threadIdx.x == 0) odd[0] = odd[1] = 0;
+  int plain = nb;
   load(a, V);
   for (int i = 0; i < nb; ++i) {
     asm volatile("" : "+s"(bs));  // opaque: addresses and conditions are formed anew rather than kept (and spilled)
@@ -161,16 +271,26 @@ __global__ void __launch_bounds__(64 * kLuWaves) btd_factor_kernel(const int *nb
         rest(k + 1);
       }
     }
+    unsigned most = 0u;
 #pragma unroll
     for (int k = 0; k < C; ++k) {
-      if (act && 8 * k + w < bs) V[i * nb2 + (8 * k + w) * bs + cur] = a[k];
+      most = max(most, max((unsigned)__double2hiint(a[k]) & 0x7fffffffu, (unsigned)__double2hiint(x[k]) & 0x7fffffffu));
       // (the reciprocal is its row's; rows at and below the diagonal have no part in the substitution)
       const double id = lane_value(idl, __builtin_amdgcn_readlane(row_of, 8 * k + w));
       A[8 * k + w][lane] = cur < 8 * k + w ? a[k] * id : 0.;
     }
+    if (__any((act && extreme<300>(idl)) || !finite_bits(most))) odd[i & 1] = 1;
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(odd[i & 1])) {
+      plain = i;
+      break;
+    }
+    if (threadIdx.x == 0) odd[(i + 1) & 1] = 0;  // read before this block, set again behind the next one's barriers
+#pragma unroll
+    for (int k = 0; k < C; ++k)
+      if (act && 8 * k + w < bs) V[i * nb2 + (8 * k + w) * bs + cur] = a[k];
     if (w == 0 && act) P[(long)i * bs + lane] = pivot;
     if (i + 1 == nb) break;
-    __syncthreads();
 #pragma unroll 4
     for (int j = bs - 1; j >= 0; --j) {
       p = __builtin_amdgcn_readlane(row_of, j);
@@ -188,6 +308,25 @@ __global__ void __launch_bounds__(64 * kLuWaves) btd_factor_kernel(const int *nb
       a[k] = act && c < bs ? fma(-up, lx, __shfl(v[k], cur, 64)) : 0.;
     }
   }
+  // that block and those behind it: A = V_i - L_i diag(sup_{i-1}), its factors, L_{i+1}
+  const int t = threadIdx.x;
+#pragma unroll 1
+  for (int i = plain; i < nb; ++i) {
+    double *Vi = V + i * nb2, *Li = L + i * nb2;
+#pragma unroll 1
+    for (int e = t; e < bs * bs; e += 64 * kLuWaves)
+      A[e / bs][e % bs] = i == 0 ? Vi[e] : fma(-sup[(long)(i - 1) * bs + e / bs], Li[e], Vi[e]);
+    __syncthreads();
+    plain_lu(A, plain_piv, bs, t);
+#pragma unroll 1
+    for (int e = t; e < bs * bs; e += 64 * kLuWaves) Vi[e] = A[e / bs][e % bs];
+    if (t < bs) P[(long)i * bs + t] = plain_piv[t] + 1;
+    if (i + 1 == nb) break;
+    plain_inverse(A, plain_piv, bs, t, Li + nb2);
+#pragma unroll 1
+    for (int e = t; e < bs * bs; e += 64 * kLuWaves) Li[nb2 + e] *= sub[(long)i * bs + e % bs];
+    __syncthreads();
+  }
 }
 
 // Solve with these factors, one workgroup per system. Wave 0 runs the chain, lane = row, with the columns of a block in
@@ -198,7 +337,9 @@ __global__ void __launch_bounds__(64 * kLuWaves) btd_factor_kernel(const int *nb
 // the reciprocals of U's diagonal, so that a division is a product and one correction step. Before, blocks were
 // staged in LDS by the wave that used them, interchanges were 53 shuffles of the vector one after the other and
 // divisions whole. Measured before and after (us): 24 systems of 30..61 blocks of 53 2,460 -> 296, 2,000 of 2..4 268 -> 91;
-// solutions are bitwise the same.
+// solutions are bitwise the same. The product with a correction is the rounded quotient where the diagonal is within
+// 2^-300 .. 2^300 and the quotient within 2^-600 .. 2^600 or zero; a block with anything else (a singular one, infinities, NaN) is
+// solved again with divisions, each row touched only by the columns that it has.
 template <int NC>
 __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1)))
 btd_solve_kernel(const int *nblocks, int bs, const double *factors, const long *voff, const double *lval, const long *loff,
@@ -249,7 +390,7 @@ btd_solve_kernel(const int *nblocks, int bs, const double *factors, const long *
     double t = act ? bi : 0.;
 #pragma unroll
     for (int c = 0; c < NC; ++c) t = fma(column(of, c, act), -lane_value(y, c), t);
-    y = t;
+    y = act ? t : 0.;  // (columns beyond the block are zero, and so are their entries: 0 times an infinity is none)
     if (act) X[(long)i * bs + lane] = y;
   };
   if (nb > 1) {
@@ -274,6 +415,7 @@ btd_solve_kernel(const int *nblocks, int bs, const double *factors, const long *
     double r = i == nb - 1 ? yi : fma(-s, xn, yi);
     r = act ? r : 0.;
     r = __shfl(r, from, 64);
+    const double r0 = r;
     int ln = lane;
     asm volatile("" : "+v"(ln));  // opaque: the comparisons below are not kept (and spilled) over the blocks
 #pragma unroll
@@ -284,6 +426,22 @@ btd_solve_kernel(const int *nblocks, int bs, const double *factors, const long *
       q = fma(fma(-u, q, r), v, q);
       r = ln == j ? q : r;
       r = fma(-column(of, j, ln < j), lane_value(q, j), r);
+    }
+    // not what divisions give, or entries that the substitutions would not have touched
+    if (__any(act && (extreme<300>(u) || (r != 0. && extreme<600>(r))))) {
+      const double *Di = D + i * nb2 + rl;
+      r = r0;
+#pragma unroll 1
+      for (int j = 0; j < bs; ++j) {
+        const double d = Di[j * bs], q = lane_value(r, j);
+        if (act && lane > j) r = fma(-d, q, r);
+      }
+#pragma unroll 1
+      for (int j = bs - 1; j >= 0; --j) {
+        if (lane == j) r /= u;
+        const double d = Di[j * bs], q = lane_value(r, j);
+        if (act && lane < j) r = fma(-d, q, r);
+      }
     }
     xn = r;
     if (act) X[(long)i * bs + lane] = r;

@@ -239,3 +239,128 @@ def test_lapack_solve_ends_on_a_one_block_system(bs, sizes):
     for s in range(len(sizes)):
         g = got[offsets[2][s]:offsets[2][s] + nb[s] * bs]
         assert np.max(np.abs(dense[s] @ g - rhs[s])) <= 1e3 * bs * 2.2e-16 * np.max(np.abs(rhs[s]))
+
+
+def _plain_lu(A):
+    """LAPACK's unblocked factors in place and the interchanges (0-based): only what lies beyond a pivot is touched"""
+    n, piv = len(A), []
+    for j in range(n):
+        a = np.where(np.isnan(A[j:, j]), -1., np.abs(A[j:, j]))
+        p = j + int(np.argmax(a))
+        piv.append(p)
+        A[[j, p]] = A[[p, j]]
+        if A[j, j] != 0.:
+            A[j + 1:, j] *= 1. / A[j, j]
+        A[j + 1:, j + 1:] -= A[j + 1:, j, None] * A[None, j, j + 1:]
+    return piv
+
+
+def _plain_solve(A, piv, X):
+    """X <- A^{-1} X in place with these factors, one division an entry"""
+    for j, p in enumerate(piv):
+        X[[j, p]] = X[[p, j]]
+    for j in range(len(A)):
+        X[j + 1:] -= A[j + 1:, j, None] * X[None, j]
+    for j in reversed(range(len(A))):
+        X[j] /= A[j, j]
+        X[:j] -= A[:j, j, None] * X[None, j]
+
+
+def _plain_system(V, lo, up, b):
+    """factors, L blocks, pivots and solution of one system by the two above"""
+    D, L, P, n = [], [None], [], len(V)
+    for i in range(n):
+        A = V[i].copy()
+        if i > 0:
+            X = np.eye(len(A))
+            _plain_solve(D[-1], P[-1], X)
+            L.append(lo[i - 1][:, None] * X)
+            A -= L[-1] * up[i - 1][None, :]
+        P.append(_plain_lu(A))
+        D.append(A)
+    y = [b[0].copy()]
+    for i in range(1, n):
+        t = b[i].copy()
+        for c in range(len(t)):
+            t -= L[i][:, c] * y[-1][c]
+        y.append(t)
+    x = [None] * n
+    for i in reversed(range(n)):
+        r = (y[i] - up[i] * x[i + 1] if i + 1 < n else y[i].copy())[:, None]
+        _plain_solve(D[i], P[i], r)
+        x[i] = r[:, 0]
+    return D, L, P, x
+
+
+def _alike(a, b, tol):
+    """the same infinities and NaN, and finite entries within tol of the largest finite one"""
+    a, b = np.asarray(a), np.asarray(b)
+    f = np.isfinite(b)
+    ok = np.array_equal(a[~f], b[~f], equal_nan=True) and np.isfinite(a[f]).all()
+    return bool(ok and (not f.any() or np.max(np.abs(a[f] - b[f])) <= tol * np.max(np.abs(b[f]))))
+
+
+@pytest.mark.parametrize('kind', ['zero column', 'infinity', 'two infinities', 'tiny pivot', 'huge pivot', 'infinite rhs'])
+@pytest.mark.parametrize('bs', [2, 9, 53, 64])
+def test_lapack_format_of_singular_and_extreme_blocks(bs, kind):
+    """Singular blocks, infinities and pivots at the ends of the range, as the first, a middle, the last and the only block of a
+    system, give what LAPACK's order of operations gives: the same infinities and NaN, and all else to rounding; ordinary systems
+    beside them are what they are. Tolerance: 1,000 N eps, the blocks' growth and condition being below 10 except in the odd entry,
+    times 100 for the chain."""
+    import torch
+    from spitfire_amd import _native
+    rng = np.random.default_rng(bs)
+    parts = []
+    for n, at in ((1, 0), (4, 0), (4, 1), (3, 2), (2, -1), (1, -1)):
+        V = rng.uniform(0.5, 1., (n, bs, bs)) * rng.choice([-1., 1.], (n, bs, bs)) + (4. + 2. * bs) * np.eye(bs)
+        lo, up = rng.uniform(0.05, 0.1, (2, n - 1, bs))
+        b = rng.uniform(0.5, 1., (n, bs))
+        k = bs - 1 if kind == 'tiny pivot' else bs // 2  # (zeros below it times its reciprocal would be NaN)
+        if at >= 0:
+            if kind == 'zero column':
+                V[at][:, k] = 0.
+                if at > 0:
+                    lo[at - 1][:] = 0.
+            elif kind == 'infinity':
+                V[at][k, bs - 1] = np.inf
+            elif kind == 'two infinities':
+                V[at][0, bs - 1], V[at][bs - 1, k] = np.inf, -np.inf
+            elif kind == 'infinite rhs':
+                b[at][k] = np.inf
+            else:
+                V[at][k], V[at][:, k] = 0., 0.
+                V[at][k, k] = 1e-310 if kind == 'tiny pivot' else 1.7e308
+                b[at][k] = 1e-310 if kind == 'tiny pivot' else 1e300
+                if at > 0:
+                    lo[at - 1][k] = up[at - 1][k] = 0.
+                if at + 1 < n:
+                    lo[at][k] = up[at][k] = 0.
+        parts.append((V, lo, up, b))
+    sizes = np.array([len(q[0]) for q in parts])
+    values = [np.concatenate([V.transpose(0, 2, 1).ravel(), lo.ravel(), up.ravel()]) for V, lo, up, _ in parts]
+    dev = torch.device('cuda:0')
+    vo, do, xo = [np.cumsum(np.r_[0, a])[:-1].astype(np.int64) for a in ([v.size for v in values], sizes * bs * bs, sizes * bs)]
+    V, b = torch.tensor(np.concatenate(values), device=dev), torch.tensor(np.concatenate([q[3].ravel() for q in parts]), device=dev)
+    n, vt, dt, xt = (torch.tensor(a, device=dev) for a in (sizes.astype(np.int32), vo, do, xo))
+    L = torch.zeros(int((sizes * bs * bs).sum()), device=dev, dtype=torch.float64)
+    P = torch.zeros(int((sizes * bs).sum()), device=dev, dtype=torch.int32)
+    x = torch.zeros_like(b)
+    st = torch.cuda.current_stream().cuda_stream
+    lib = _native.lib()
+    _native.check(lib.gf_batch_btddod_full_factorize(len(sizes), n.data_ptr(), bs, V.data_ptr(), vt.data_ptr(), L.data_ptr(),
+                                                     dt.data_ptr(), P.data_ptr(), xt.data_ptr(), st))
+    _native.check(lib.gf_batch_btddod_full_solve(len(sizes), n.data_ptr(), bs, V.data_ptr(), vt.data_ptr(), L.data_ptr(),
+                                                 dt.data_ptr(), P.data_ptr(), xt.data_ptr(), b.data_ptr(), x.data_ptr(),
+                                                 xt.data_ptr(), st))
+    v, l, p, g = (t.cpu().numpy() for t in (V, L, P, x))
+    tol = 1e5 * bs * 2.2e-16
+    with np.errstate(all='ignore'):
+        for s, part in enumerate(parts):
+            D, Lb, piv, xs = _plain_system(*part)
+            for i in range(sizes[s]):
+                at = do[s] + i * bs * bs
+                assert _alike(v[vo[s] + i * bs * bs:vo[s] + (i + 1) * bs * bs].reshape(bs, bs).T, D[i], tol), (s, i)
+                assert np.array_equal(p[xo[s] + i * bs:xo[s] + (i + 1) * bs] - 1, piv[i]), (s, i)
+                if i > 0:
+                    assert _alike(l[at:at + bs * bs].reshape(bs, bs).T, Lb[i], tol), (s, i)
+                assert _alike(g[xo[s] + i * bs:xo[s] + (i + 1) * bs], xs[i], tol), (s, i)
