@@ -378,10 +378,12 @@ struct Window {
 // update, which holds the next panel, is waited for: the others and the store follow while that panel is factored.
 template <typename T, int NT>
 __global__ void __launch_bounds__(128 * (NT + 1)) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 6 : NT == 2 ? 5 : NT == 3 ? 4 : 2)))
-twist_factor_kernel(int nsys, const int *nblocks, int n, const double *values, const long *voff, T *dinv, const long *doff) {
+twist_factor_kernel(int nsys, const int *nblocks, int n, const double *values, const long *voff, T *dinv, const long *doff,
+                    int least) {
   using S = ChainLds<T, NT>;
   extern __shared__ double v_raw[];
   __shared__ S lds[2];
+  if (nblocks[blockIdx.x] < least) return;  // (systems of fewer blocks are another kernel's)
   // Two one-block systems share a workgroup, the second (256 further on, so that the workgroups that are left without
   // work are spread evenly over the XCDs and compute units) in the bottom chain's place.
   const int other = blockIdx.x ^ 256;
@@ -546,14 +548,15 @@ twist_factor_kernel(int nsys, const int *nblocks, int n, const double *values, c
 
 template <typename T, int NT>
 int launch_nt(int nsys, const int *nblocks, int bs, const double *values, const long *voff, T *dinv,
-              const long *doff, hipStream_t st) {
+              const long *doff, int least, hipStream_t st) {
   auto kern = twist_factor_kernel<T, NT>;
   using S = ChainLds<T, NT>;
   const size_t lds = sizeof(double) * ((2 * S::v_words(bs) + 1) & ~1) + 2 * sizeof(T) * S::m_words((bs + 7) & ~7);
   if (lds + 2 * sizeof(S) > 65536 &&
       hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return fail(GF_ERR_UNSUPPORTED, "block too large for LDS");
-  hipLaunchKernelGGL(kern, dim3(nsys), dim3(128 * (NT + 1)), lds, st, nsys, nblocks, bs, values, voff, dinv, doff);
+  hipLaunchKernelGGL(kern, dim3(nsys), dim3(128 * (NT + 1)), lds, st, nsys, nblocks, bs, values, voff, dinv, doff,
+                     least);
   return hipGetLastError() == hipSuccess ? GF_OK : fail(GF_ERR_HIP, "btd inverse factor launch failed");
 }
 
@@ -570,11 +573,21 @@ int launch_btd_inv_factor(int nsys, const int *nblocks, int bs, const double *va
   // systems or larger blocks the kernel above wins (1,024 chains of 13: 289 against 491 us).
   if (bs <= kSmallFactor && nsys >= 1536)
     return launch_btd_inv_factor_small<T>(nsys, nblocks, bs, values, voff, dinv, doff, st);
+  // Blocks of 17..22 (FP32 28) in such batches: the same for the one-block systems among them, in a launch of its own, since how
+  // many there are is on the device. Single blocks of 18 / 20 / 22 / 24, 4,000 of them, without and with it: 41 / 41 / 43 / 43
+  // and 29 / 33 / 38 / 43 us FP64, of 18 / 20 / 24 / 28 34 / 34 / 36 / 47 and 21 / 24 / 31 / 39 us FP32; 1,536 of 20 21 and 19,
+  // 17 and 16 us. Batches of chains lose the launch, 2 us (1,536 chains of 2..7 blocks of 20: 91 and 94 us).
+  int least = 1;
+  if (bs >= kSingleFrom && bs <= kSingleTo<T> && nsys >= 1536) {
+    const int rc = launch_btd_inv_factor_single<T>(nsys, nblocks, bs, values, voff, dinv, doff, st);
+    if (rc != GF_OK) return rc;
+    least = 2;
+  }
   switch ((bs + 15) / 16) {
-    case 1: return launch_nt<T, 1>(nsys, nblocks, bs, values, voff, dinv, doff, st);
-    case 2: return launch_nt<T, 2>(nsys, nblocks, bs, values, voff, dinv, doff, st);
-    case 3: return launch_nt<T, 3>(nsys, nblocks, bs, values, voff, dinv, doff, st);
-    default: return launch_nt<T, 4>(nsys, nblocks, bs, values, voff, dinv, doff, st);
+    case 1: return launch_nt<T, 1>(nsys, nblocks, bs, values, voff, dinv, doff, least, st);
+    case 2: return launch_nt<T, 2>(nsys, nblocks, bs, values, voff, dinv, doff, least, st);
+    case 3: return launch_nt<T, 3>(nsys, nblocks, bs, values, voff, dinv, doff, least, st);
+    default: return launch_nt<T, 4>(nsys, nblocks, bs, values, voff, dinv, doff, least, st);
   }
 }
 

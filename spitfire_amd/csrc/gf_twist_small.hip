@@ -1,7 +1,8 @@
 // Twisted block factorisation (gf_twist.hip) for many systems of small blocks (1..11 unknowns): one wave per chain, the
 // block in the wave's registers, no barriers inside an inverse. The MFMA kernel pads a block to panels of eight and
 // tiles of sixteen and keeps several waves per chain; once the systems alone fill the chip, small blocks are faster
-// without either (launch_btd_inv_factor).
+// without either (launch_btd_inv_factor). The same for the one-block systems of batches of somewhat larger blocks, which
+// are padded by up to half (17 of 32).
 #include "gf_internal.h"
 #include "gf_wave.h"
 #include "../../include/griffon_amd.h"
@@ -158,10 +159,32 @@ __global__ void __launch_bounds__(128) small_factor_kernel(const int *nblocks, c
   }
 }
 
+// The one-block systems of a batch, one wave each; systems of several blocks are left alone. Four waves per workgroup, so that
+// 1,024 systems are a wave for every SIMD (workgroups of one or two waves double up on some: 1,024 blocks of 20 11.9 -> 16.7 us).
+template <typename T, int N>
+__global__ void __launch_bounds__(256) single_factor_kernel(int nsys, const int *nblocks, const double *values,
+                                                            const long *voff, T *dinv, const long *doff) {
+  const int sys = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  if (sys >= nsys || nblocks[sys] != 1) return;
+  const int lane = threadIdx.x & 63;
+  T x[N];
+  int rowid, colid;
+  reg_load_block<T, N>(x, values + voff[sys], rowid, colid, lane);
+  reg_gj_inverse<T, N>(x, rowid, colid, lane);
+  reg_store_block<T, N>(x, dinv + doff[sys], rowid, colid, lane);
+}
+
 template <typename T, int N>
 void launch_small(int nsys, const int *nblocks, const double *values, const long *voff, T *dinv, const long *doff,
                   hipStream_t st) {
   hipLaunchKernelGGL((small_factor_kernel<T, N>), dim3(nsys), dim3(128), 0, st, nblocks, values, voff, dinv, doff);
+}
+
+template <typename T, int N>
+void launch_single(int nsys, const int *nblocks, const double *values, const long *voff, T *dinv, const long *doff,
+                   hipStream_t st) {
+  hipLaunchKernelGGL((single_factor_kernel<T, N>), dim3((nsys + 3) / 4), dim3(256), 0, st, nsys, nblocks, values, voff,
+                     dinv, doff);
 }
 
 template <typename T>
@@ -173,7 +196,26 @@ SmallFn<T> small_fn(int bs, std::integer_sequence<int, I...>) {
   return tab[bs - 1];
 }
 
+template <typename T, int... I>
+SmallFn<T> single_fn(int bs, std::integer_sequence<int, I...>) {
+  constexpr SmallFn<T> tab[] = {&launch_single<T, I + kSingleFrom>...};
+  return tab[bs - kSingleFrom];
+}
+
 }  // namespace
+
+template <typename T>
+int launch_btd_inv_factor_single(int nsys, const int *nblocks, int bs, const double *values, const long *voff, T *dinv,
+                                 const long *doff, hipStream_t st) {
+  single_fn<T>(bs, std::make_integer_sequence<int, kSingleTo<T> - kSingleFrom + 1>{})(nsys, nblocks, values, voff, dinv, doff,
+                                                                                    st);
+  return hipGetLastError() == hipSuccess ? GF_OK : fail(GF_ERR_HIP, "btd inverse factor launch failed");
+}
+
+template int launch_btd_inv_factor_single<double>(int, const int *, int, const double *, const long *, double *,
+                                                  const long *, hipStream_t);
+template int launch_btd_inv_factor_single<float>(int, const int *, int, const double *, const long *, float *,
+                                                 const long *, hipStream_t);
 
 template <typename T>
 int launch_btd_inv_factor_small(int nsys, const int *nblocks, int bs, const double *values, const long *voff, T *dinv,

@@ -364,3 +364,22 @@ def test_lapack_format_of_singular_and_extreme_blocks(bs, kind):
                 if i > 0:
                     assert _alike(l[at:at + bs * bs].reshape(bs, bs).T, Lb[i], tol), (s, i)
                 assert _alike(g[xo[s] + i * bs:xo[s] + (i + 1) * bs], xs[i], tol), (s, i)
+
+
+@pytest.mark.parametrize('precision', [64, 32])
+@pytest.mark.parametrize('bs', [16, 17, 20, 22, 23, 28, 29])
+def test_one_block_systems_of_a_large_batch_are_bitwise_the_same(bs, precision):
+    """In a large batch the one-block systems of these sizes have a kernel of their own; the inverses are those of a small batch,
+    where they have not, entry by entry, and so are the longer systems' beside them. Tolerance: none."""
+    rng = np.random.default_rng(bs)
+    sizes = [1, 1, 3, 1, 2, 1, 1]
+    values = []
+    for s, n in enumerate(sizes):
+        V = rng.standard_normal(n * bs * bs) if s % 2 else rng.integers(-2, 3, n * bs * bs).astype(float)
+        values.append(np.concatenate([V, rng.standard_normal(2 * (n - 1) * bs)]))
+    few = _factor(sizes, bs, values, precision)
+    many = _factor(sizes * 220 + [1], bs, values * 220 + values[:1], precision)  # 1,541 systems: not whole workgroups
+    for s in range(len(sizes)):
+        for k in (0, 1, 219):
+            assert np.array_equal(few[s], many[s + k * len(sizes)], equal_nan=True)
+    assert np.array_equal(few[0], many[-1], equal_nan=True)
