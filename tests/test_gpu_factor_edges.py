@@ -1,4 +1,8 @@
 """The batched inverse factor at the edges of its tiles, panels and workgroup pairs (GPU)."""
+import ctypes
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -383,3 +387,38 @@ def test_one_block_systems_of_a_large_batch_are_bitwise_the_same(bs, precision):
         for k in (0, 1, 219):
             assert np.array_equal(few[s], many[s + k * len(sizes)], equal_nan=True)
     assert np.array_equal(few[0], many[-1], equal_nan=True)
+
+
+@pytest.fixture(scope='module')
+def host_factor(tmp_path_factory):
+    """inverse factors of one system, eliminated pivot by pivot on the host (tests/native/gauss_jordan_host.cpp)"""
+    so = str(tmp_path_factory.mktemp('gauss_jordan') / 'libgj.so')
+    subprocess.run(['g++', '-O2', '-std=c++17', '-ffp-contract=off', '-mfma', '-shared', '-fPIC', '-o', so,
+                    os.path.join(os.path.dirname(os.path.abspath(__file__)), 'native', 'gauss_jordan_host.cpp')], check=True)
+    lib = ctypes.CDLL(so)
+
+    def factor(n, bs, values, precision):
+        out = np.empty((n, bs, bs), dtype=np.float64 if precision == 64 else np.float32)
+        v = np.ascontiguousarray(values)
+        getattr(lib, 'inverse_factor_f%d' % precision)(n, bs, v.ctypes.data_as(ctypes.c_void_p),
+                                                       out.ctypes.data_as(ctypes.c_void_p))
+        return out.transpose(0, 2, 1).astype(np.float64)
+    return factor
+
+
+@pytest.mark.parametrize('precision', [64, 32])
+@pytest.mark.parametrize('bs', [5, 8, 12, 16, 17, 31, 32, 33, 48, 49, 53, 57, 64])
+def test_inverse_factor_is_bitwise_the_elimination_pivot_by_pivot(bs, precision, host_factor):
+    """Whatever the panels and tiles: blocks of one to four tiles, random ones and integers whose pivots tie, alone, in chains that
+    permute a permuted block's rows and columns, and one-block systems that share a workgroup (the batch of 300, where 256
+    further on there is another one) against an independent elimination on the host. Tolerance: none."""
+    rng = np.random.default_rng(100 + bs)
+    for sizes in ([1, 2, 3, 4, 7, 1, 2], [1] * 300):
+        values = []
+        for s, n in enumerate(sizes):
+            V = rng.standard_normal(n * bs * bs) if s % 2 else rng.integers(-3, 4, n * bs * bs).astype(float)
+            values.append(np.concatenate([V, rng.standard_normal(2 * (n - 1) * bs)]))
+        got = _factor(sizes, bs, values, precision)
+        for s in list(range(7)) + ([255, 256, 257, 299] if len(sizes) > 7 else []):
+            ref = host_factor(sizes[s], bs, values[s], precision)
+            assert np.isfinite(ref).all() and np.array_equal(got[s], ref), (s, sizes[s])
