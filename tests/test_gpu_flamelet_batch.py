@@ -472,3 +472,36 @@ def test_time_step_matrix_of_a_fresh_batch(precision, mech_c1_data):
         _native.check(lib.gf_flamelet_batch_transient_solve(fb._h, _native.iptr(flags), r.data_ptr(), out.data_ptr()))
         got.append(out.cpu().numpy())
     assert np.isfinite(got[1]).all() and np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize('precision', [64, 32])
+@pytest.mark.parametrize('ns', [13, 14, 16, 52, 53, 59])
+def test_solve_with_a_compute_unit_per_chain_at_its_sizes(ns, precision):
+    """The solve of few long flamelets (up to 128, 40 points and more on average) against the one of many, for block sizes with
+    every remainder of four columns and flamelets of 2 and 3 interior points beside long ones, the right-hand side apart from and in
+    place of the solution. Tolerance: none (the same sums in the same order)."""
+    import torch
+    from spitfire_amd import _native, synthetic
+    from spitfire_amd.flamelet import FlameletBatch
+    from spitfire_amd.mechanism import ChemicalMechanismSpec
+    m = ChemicalMechanismSpec(synthetic.make_mechanism(ns, 2 * ns, seed=0))
+    npts = [120, 101, 62, 4, 5]
+    lib, dev = _native.lib(), torch.device('cuda:0')
+    rng = np.random.default_rng(ns)
+    few = np.concatenate([rng.standard_normal((n - 2) * ns) for n in npts])
+    ref = None
+    for copies in (26, 1):  # 130 flamelets, and five
+        B = len(npts) * copies
+        fb = FlameletBatch(_flamelets(m, [10.] * B, npts * copies))
+        flags, pre = np.ones(B, dtype=np.int32), np.full(B, 1e-7)
+        x, r = torch.tensor(fb._x0, device=dev), torch.tensor(np.tile(few, copies), device=dev)
+        apart = torch.full_like(r, 7.)
+        torch.cuda.synchronize()
+        _native.check(lib.gf_flamelet_batch_transient_setup(fb._h, _native.iptr(flags), x.data_ptr(), _native.dptr(pre),
+                                                            precision))
+        _native.check(lib.gf_flamelet_batch_transient_solve(fb._h, _native.iptr(flags), r.data_ptr(), apart.data_ptr()))
+        _native.check(lib.gf_flamelet_batch_transient_solve(fb._h, _native.iptr(flags), r.data_ptr(), r.data_ptr()))
+        assert torch.equal(apart, r)
+        got = r.cpu().numpy().reshape(copies, -1)
+        ref = got[0] if ref is None else ref
+        assert np.isfinite(ref).all() and (got == ref).all()
