@@ -284,9 +284,7 @@ constexpr int kSmallFactor = 11;  // largest block of the one-wave-per-chain fac
 template <typename T>
 int launch_btd_inv_factor_small(int nsys, const int *nblocks, int bs, const double *values, const long *voff, T *dinv,
                                 const long *doff, hipStream_t st);
-constexpr int kSingleFrom = 17;  // blocks whose one-block systems it takes out of large batches
-template <typename T>
-constexpr int kSingleTo = sizeof(T) == 8 ? 22 : 28;
+constexpr int kSingleFrom = 17;  // smallest block of its kernel for the one-block systems of large batches
 template <typename T>
 int launch_btd_inv_factor_single(int nsys, const int *nblocks, int bs, const double *values, const long *voff, T *dinv,
                                  const long *doff, hipStream_t st);

@@ -43,6 +43,8 @@
 #include "gf_wave.h"
 #include "../../include/griffon_amd.h"
 
+#include <climits>
+
 namespace gfa {
 
 namespace {
@@ -560,6 +562,26 @@ int launch_nt(int nsys, const int *nblocks, int bs, const double *values, const 
   return hipGetLastError() == hipSuccess ? GF_OK : fail(GF_ERR_HIP, "btd inverse factor launch failed");
 }
 
+// From how many systems on the one-block systems of a batch have a launch of their own, one wave each, ahead of the panels' (how
+// many there are is known on the device only; panels take the rest). A wave takes time with the block's size, panels with the
+// tiles that it is padded to, and of these fewer fit a compute unit with each tile. Single blocks, panels and one wave (us):
+//                     FP64 17         20         27         32         33         48         53         64
+//   1,536 systems   19 -> 16   21 -> 19   26 -> 29   27 -> 38   44 -> 39   68 -> 73   74 -> 87  89 -> 117
+//   2,048 systems   22 -> 16   23 -> 19   29 -> 29   30 -> 40   52 -> 40   90 -> 76   97 -> 89 117 -> 120
+//   4,000 systems   39 -> 26   41 -> 33   53 -> 51   56 -> 67   93 -> 70 174 -> 131 186 -> 155 226 -> 220
+//                     FP32 17         20         28         32         33         48         53         64
+//   1,280 systems   15 -> 12   16 -> 14   20 -> 21   20 -> 27   28 -> 26   40 -> 47   60 -> 56   68 -> 70
+//   1,536 systems   17 -> 12   17 -> 14   22 -> 21   22 -> 27   34 -> 26   49 -> 48   64 -> 58   73 -> 72
+//   4,000 systems   33 -> 19   34 -> 23   48 -> 39   52 -> 50   76 -> 49  100 -> 85 168 -> 102 189 -> 131
+// Batches of chains lose the launch, 2 us (1,536 chains of 2..7 blocks of 20: 91 -> 94 us).
+template <typename T>
+int many_singles(int n) {
+  if (sizeof(T) == 4) return n <= 22 ? 1025 : n >= 29 && n <= 32 ? 4000 : 1536;
+  if (n <= 20) return 1280;
+  if (n >= 28 && n <= 32) return INT_MAX;
+  return n >= 23 && n <= 27 ? 3000 : n <= 38 ? 1536 : 1537;  // (three rounds of panels at one workgroup per compute unit)
+}
+
 }  // namespace
 
 template <typename T>
@@ -570,15 +592,13 @@ int launch_btd_inv_factor(int nsys, const int *nblocks, int bs, const double *va
   // Blocks below 12 in batches of at least six systems per compute unit: one wave per chain without barriers is faster
   // there when the systems are single blocks (4,000 blocks of 10: 12 against 20 us FP64, 9 against 16 us FP32) and
   // about even on chains (3,000 chains of 30-99 blocks of 6: 303 against 347 us, of 10: 702 against 640 us); with fewer
-  // systems or larger blocks the kernel above wins (1,024 chains of 13: 289 against 491 us).
-  if (bs <= kSmallFactor && nsys >= 1536)
+  // systems or larger blocks the kernel above wins (1,024 chains of 13: 289 against 491 us). Blocks of up to 4 would be padding
+  // for the most part: one wave whatever the batch (one chain of 126 blocks of 1 / 4 unknowns 30 / 97 against 90 / 117 us FP64, 28 /
+  // 85 against 80 / 103 us FP32, 300 chains of 40..99 of 4 92 against 100 us; of 5 120 against 126 and 115 against 108 us).
+  if (bs <= 4 || (bs <= kSmallFactor && nsys >= 1536))
     return launch_btd_inv_factor_small<T>(nsys, nblocks, bs, values, voff, dinv, doff, st);
-  // Blocks of 17..22 (FP32 28) in such batches: the same for the one-block systems among them, in a launch of its own, since how
-  // many there are is on the device. Single blocks of 18 / 20 / 22 / 24, 4,000 of them, without and with it: 41 / 41 / 43 / 43
-  // and 29 / 33 / 38 / 43 us FP64, of 18 / 20 / 24 / 28 34 / 34 / 36 / 47 and 21 / 24 / 31 / 39 us FP32; 1,536 of 20 21 and 19,
-  // 17 and 16 us. Batches of chains lose the launch, 2 us (1,536 chains of 2..7 blocks of 20: 91 and 94 us).
   int least = 1;
-  if (bs >= kSingleFrom && bs <= kSingleTo<T> && nsys >= 1536) {
+  if (bs >= kSingleFrom && nsys >= many_singles<T>(bs)) {
     const int rc = launch_btd_inv_factor_single<T>(nsys, nblocks, bs, values, voff, dinv, doff, st);
     if (rc != GF_OK) return rc;
     least = 2;

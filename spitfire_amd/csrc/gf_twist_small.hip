@@ -1,8 +1,8 @@
 // Twisted block factorisation (gf_twist.hip) for many systems of small blocks (1..11 unknowns): one wave per chain, the
 // block in the wave's registers, no barriers inside an inverse. The MFMA kernel pads a block to panels of eight and
 // tiles of sixteen and keeps several waves per chain; once the systems alone fill the chip, small blocks are faster
-// without either (launch_btd_inv_factor). The same for the one-block systems of batches of somewhat larger blocks, which
-// are padded by up to half (17 of 32).
+// without either (launch_btd_inv_factor). The same for the one-block systems of large batches of larger blocks: nothing is
+// padded, and none of a chain's LDS is held for a block that has no neighbours.
 #include "gf_internal.h"
 #include "gf_wave.h"
 #include "../../include/griffon_amd.h"
@@ -207,8 +207,7 @@ SmallFn<T> single_fn(int bs, std::integer_sequence<int, I...>) {
 template <typename T>
 int launch_btd_inv_factor_single(int nsys, const int *nblocks, int bs, const double *values, const long *voff, T *dinv,
                                  const long *doff, hipStream_t st) {
-  single_fn<T>(bs, std::make_integer_sequence<int, kSingleTo<T> - kSingleFrom + 1>{})(nsys, nblocks, values, voff, dinv, doff,
-                                                                                    st);
+  single_fn<T>(bs, std::make_integer_sequence<int, 64 - kSingleFrom + 1>{})(nsys, nblocks, values, voff, dinv, doff, st);
   return hipGetLastError() == hipSuccess ? GF_OK : fail(GF_ERR_HIP, "btd inverse factor launch failed");
 }
 
