@@ -615,6 +615,125 @@ __global__ void __launch_bounds__(512) btd_twist_solve_kernel(const int *nblocks
   }
 }
 
+// The same solve with one wave per chain, for small blocks and for many systems: a wave has all columns of a block, so a product
+// needs no exchange, and the chains of a system meet at the middle block only. What bounds it is a product's chain of broadcasts
+// and multiply-adds where systems are few, and the reads of the inverses where they are many; loads are issued two products
+// ahead (one: 300 chains of 10..40 blocks of 10 24 us instead of 21; three take too many registers). Eight waves per
+// system and this (us; before both, two waves per system that waited for their loads: third figure), chains of 10..40 blocks:
+//   systems            FP64 4               10               20               32              40
+//       1 of 60   26 / 19 / 31     32 / 24 / 56     37 / 37 / 64     50 / 54 / 83   59 / 65 / 109
+//     300         24 / 16 / 24     35 / 21 / 42     42 / 35 / 57     58 / 51 / 82   69 / 61 / 113
+//   1,000         40 / 20 / 26     65 / 34 / 59     77 / 56 / 81   106 / 90 / 106 158 / 152 / 181
+//   4,000       114 / 56 / 65   189 / 100 / 148  269 / 222 / 247  404 / 397 / 440 548 / 553 / 646
+//   systems            FP32 4               10               20               32              40
+//       1 of 60   26 / 19 / 30     30 / 25 / 52     32 / 34 / 61     36 / 42 / 80   42 / 50 / 105
+//     300         24 / 16 / 24     28 / 21 / 40     29 / 28 / 48     36 / 36 / 73   44 / 48 / 104
+//   1,000         37 / 18 / 25     47 / 24 / 44     49 / 36 / 68     64 / 44 / 84   78 / 61 / 119
+//   4,000        102 / 38 / 48    140 / 65 / 112   137 / 83 / 135  207 / 171 / 222 260 / 265 / 344
+// (48: 4,000 chains 695 / 769 us FP64, 332 / 361 us FP32.) Bitwise the same.
+constexpr int kWaveSolve = 40;  // its largest block
+template <typename T>
+constexpr int kWaveSolveAlways = sizeof(T) == 8 ? 20 : 16;  // the largest that it takes whatever the number of systems
+
+template <typename T, int N>
+__global__ void __launch_bounds__(128) btd_wave_solve_kernel(const int *nblocks, const double *values, const long *voff,
+                                                             const T *dinv, const long *doff, const double *rhs, double *x,
+                                                             const long *xoff) {
+  __shared__ double part[2][64];
+  const int lane = threadIdx.x & 63;
+  const int chain = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool top = chain == 0;
+  const int sys = blockIdx.x;
+  const int nb = __builtin_amdgcn_readfirstlane(nblocks[sys]);
+  if (!top && nb == 1) return;
+  const bool act = lane < N;
+  const int rl = act ? lane : 0;
+  const int m = (nb - 1) / 2;
+  const double *b = rhs + xoff[sys];
+  double *X = x + xoff[sys];
+  const double *sub = values + voff[sys] + (long)nb * (N * N);
+  const double *sup = sub + (long)(nb - 1) * N;
+  const T *DI = dinv + doff[sys] + rl;
+  struct Ahead {
+    T d[N];
+    double a, c;
+  };
+  double v;
+  auto columns = [&](Ahead &B, int i) {
+    const T *D = DI + (long)i * (N * N);
+#pragma unroll
+    for (int k = 0; k < N; ++k) B.d[k] = D[k * N];
+  };
+  auto multiply = [&](const Ahead &B) {
+    constexpr int K4 = N / 4 * 4;
+    double p[4] = {0., 0., 0., 0.};
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const int j = k < K4 ? k & 3 : 0;
+      p[j] = fma((double)B.d[k], lane_value(v, k), p[j]);
+    }
+    return (p[0] + p[1]) + (p[2] + p[3]);
+  };
+  if (nb == 1) {
+    Ahead B;
+    v = b[rl];
+    columns(B, 0);
+    v = multiply(B);
+    if (act) X[lane] = v;
+    return;
+  }
+  // (products, places and loads as in the kernel above)
+  const int L = nb - 1 - m;
+  const int len = top ? m : L, off = L - len;
+  const int first = top ? 0 : nb - 1, dir = top ? 1 : -1;
+  auto block = [&](int s) { return first + dir * max(len - abs(len - s), 0); };
+  auto at = [&](int i) { return (unsigned)(i * N + rl); };
+  const double bm = b[at(m)], ct = m > 0 ? sub[at(m - 1)] : 0., cb = sup[at(m)];
+  double last = 0.;
+  v = b[at(block(0))];
+  if (len > 0 && act) X[at(block(0))] = v;
+  auto operands = [&](Ahead &B, int s) {
+    const int i = block(s), j = block(s + 1);
+    columns(B, i);
+    B.c = (top == (s < len) ? sub : sup)[at(min(min(i, j), nb - 2))];
+  };
+  auto addend = [&](Ahead &B, int s) { B.a = (s < len ? b : X)[at(block(s + 1))]; };
+  constexpr int A = 2;
+  Ahead buf[A];
+#pragma unroll
+  for (int k = 0; k < A; ++k) {
+    operands(buf[k], max(k - off, 0));
+    addend(buf[k], max(k - off, 0));
+  }
+  auto product = [&](Ahead &B, int g) {
+    const int s = g - off;
+    const double mv = multiply(B);
+    const double a = s == len ? last : B.a, c = B.c;
+    asm volatile("" ::"v"(B.a));
+    operands(B, s + A);
+    if (g == L - 1) {
+#pragma clang fp contract(off)
+      part[chain][lane] = mv;
+      __syncthreads();
+      const double tt = m > 0 ? ct * part[0][lane] : 0., tb = cb * part[1][lane];
+      last = v;
+      v = bm - tt - tb;
+    } else if ((unsigned)s <= (unsigned)(2 * len)) {
+      const bool in = s < len;
+      v = fma(-c, mv, a);
+      if (act) X[at(block(in ? s + 1 : s))] = in ? v : mv;
+    }
+    addend(B, s + A);
+  };
+  for (int g = 0; g <= 2 * L; g += A) {
+#pragma unroll
+    for (int k = 0; k < A; ++k) {
+      if (g + k > 2 * L) break;
+      product(buf[k], g + k);
+    }
+  }
+}
+
 // The same solve with the two chains of a system on two compute units, for few systems of long chains: inwards and outwards one
 // workgroup of four waves per chain (blockIdx.x = 2 system + chain), in between the middle block. Both chains of a system
 // on one compute unit are bound by its cache fills (45 KB a product at 53); three launches cost about 8 us more.
@@ -722,7 +841,12 @@ using InvSolve = void (*)(const int *, const double *, const long *, const T *, 
                           const long *);
 template <typename T, int... I>
 InvSolve<T> inv_solve_kernel(int bs, std::integer_sequence<int, I...>) {
-  constexpr InvSolve<T> tab[] = {&btd_twist_solve_kernel<T, I + 1>...};
+  constexpr InvSolve<T> tab[] = {&btd_twist_solve_kernel<T, kWaveSolveAlways<T> + I + 1>...};
+  return tab[bs - kWaveSolveAlways<T> - 1];
+}
+template <typename T, int... I>
+InvSolve<T> wave_solve_kernel(int bs, std::integer_sequence<int, I...>) {
+  constexpr InvSolve<T> tab[] = {&btd_wave_solve_kernel<T, I + 1>...};
   return tab[bs - 1];
 }
 
@@ -793,9 +917,12 @@ int launch_btd_inv_solve(int nsys, const int *nblocks, int bs, const double *val
     hipLaunchKernelGGL(middle_solve_kernel<T>(bs, sizes), dim3(nsys), dim3(512), 0, st, nblocks, values, voff, dinv, doff,
                        rhs, x, xoff);
     hipLaunchKernelGGL(chain, dim3(2 * nsys), dim3(256), 0, st, nblocks, values, voff, dinv, doff, rhs, x, xoff, 0);
+  } else if (bs <= kWaveSolveAlways<T> || (bs <= kWaveSolve && nsys >= (sizeof(T) == 8 ? 300 : 600))) {
+    hipLaunchKernelGGL(wave_solve_kernel<T>(bs, std::make_integer_sequence<int, kWaveSolve>{}), dim3(nsys), dim3(128), 0, st,
+                       nblocks, values, voff, dinv, doff, rhs, x, xoff);
   } else {
-    hipLaunchKernelGGL(inv_solve_kernel<T>(bs, sizes), dim3(nsys), dim3(512), 0, st, nblocks, values, voff, dinv, doff,
-                       rhs, x, xoff);
+    const auto kern = inv_solve_kernel<T>(bs, std::make_integer_sequence<int, 64 - kWaveSolveAlways<T>>{});
+    hipLaunchKernelGGL(kern, dim3(nsys), dim3(512), 0, st, nblocks, values, voff, dinv, doff, rhs, x, xoff);
   }
   if (hipGetLastError() != hipSuccess) return fail(GF_ERR_HIP, "btd inverse solve launch failed");
   return GF_OK;

@@ -422,3 +422,36 @@ def test_inverse_factor_is_bitwise_the_elimination_pivot_by_pivot(bs, precision,
         for s in list(range(7)) + ([255, 256, 257, 299] if len(sizes) > 7 else []):
             ref = host_factor(sizes[s], bs, values[s], precision)
             assert np.isfinite(ref).all() and np.array_equal(got[s], ref), (s, sizes[s])
+
+
+@pytest.mark.parametrize('precision', [64, 32])
+@pytest.mark.parametrize('bs', [17, 20, 21, 24, 31, 39, 40, 41])
+def test_inverse_solve_of_few_and_many_systems_is_bitwise_the_same(bs, precision):
+    """Few systems share each chain among four waves, many have a wave per chain (up to 40 unknowns): the same sums in the same order,
+    for every remainder of four columns, chains from one block to some more than the loads in flight, the right-hand side apart
+    from and in place of the solution. Tolerance: none."""
+    import torch
+    from spitfire_amd import _native
+    rng = np.random.default_rng(bs)
+    sizes = [1, 2, 3, 4, 5, 6, 9, 12]
+    values = [rng.standard_normal(n * bs * bs + 2 * (n - 1) * bs) for n in sizes]
+    inverses = [0.1 * rng.standard_normal(n * bs * bs) for n in sizes]
+    rhs = [rng.standard_normal(n * bs) for n in sizes]
+    dev, lib = torch.device('cuda:0'), _native.lib()
+    st = torch.cuda.current_stream().cuda_stream
+    got = []
+    for copies in (1, 80):
+        nb = np.asarray(sizes * copies)
+        vo, do, xo = [torch.tensor(np.cumsum(np.r_[0, a])[:-1].astype(np.int64), device=dev)
+                      for a in (nb * bs * bs + 2 * (nb - 1) * bs, nb * bs * bs, nb * bs)]
+        V, D, b = (torch.tensor(np.tile(np.concatenate(a), copies), device=dev) for a in (values, inverses, rhs))
+        D = D.to(torch.float64 if precision == 64 else torch.float32)
+        n, x = torch.tensor(nb.astype(np.int32), device=dev), torch.full_like(b, 7.)
+        in_place = b.clone()
+        for r, out in ((b, x), (in_place, in_place)):
+            _native.check(lib.gf_batch_btddod_inverse_solve(nb.size, n.data_ptr(), bs, V.data_ptr(), vo.data_ptr(),
+                                                            D.data_ptr(), do.data_ptr(), precision, r.data_ptr(),
+                                                            out.data_ptr(), xo.data_ptr(), st))
+        assert torch.equal(x, in_place)
+        got.append(x.cpu().numpy().reshape(copies, -1))
+    assert np.isfinite(got[0]).all() and (got[1] == got[0]).all()
