@@ -22,9 +22,11 @@
 //       (rho,T,Y)->(T,Y) transform at constant pressure); the temperature row is the enthalpy-weighted
 //       wave sum of the column; each column of each state is one contiguous 53-double store.
 //
-// What bounds it is latency, with few wavefronts: the Jacobian kernel's state (28 KB of LDS a state, 250 registers) leaves room
+// What bounds it is latency, with few wavefronts: the Jacobian kernel's state (28 KB of LDS a state, 256 registers) leaves room
 // for eight waves per compute unit, the rates' registers for twelve (held to 168: at 186 they were eight and
-// 100,003 states took 1,033 us instead of 803). The states of a group are interleaved in LDS, so that neighbouring lanes read
+// 100,003 states took 1,033 us instead of 803). The Jacobian's are held to 256: with six more, small mechanisms, whose LDS has
+// room for two workgroups of 256 threads, had one of them (4,000 states of 10 species 73 us instead of 56). The states of
+// a group are interleaved in LDS, so that neighbouring lanes read
 // neighbouring words, and a reaction's record is read whole, its short lists unrolled with factors of one beyond their
 // ends: field by field, with loops of one to four trips around dependent loads, P1 took 41,000 cycles for a group
 // of four states with derivatives and now takes 32,000. 53 species, 325 reactions, before and after (us): RHS of 512 / 7,600 /
@@ -147,7 +149,7 @@ __device__ __forceinline__ double troe_fcent(const DevRxn &R, double T, double i
 }
 
 template <int S, int THREADS, bool JAC>
-__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(JAC ? 1 : 3))) chem_kernel(MechView mv, ChemArgs a, long groups_per_wg) {
+__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(JAC ? 2 : 3))) chem_kernel(MechView mv, ChemArgs a, long groups_per_wg) {
   static_assert(S >= 1 && S <= 4, "the temperature-row sums take at most four states at once");
   extern __shared__ double lds[];
   const int ns = mv.ns, nr = mv.nr, nm = ns - 1;
