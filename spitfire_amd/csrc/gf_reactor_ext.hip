@@ -6,10 +6,10 @@
 //   - the isochoric reactor in (rho, T, Y) with the same options (isochoric_reactor_kernels.cpp:18-333);
 // from the chemistry kernel's per-state production rates, raw option-0/1 sensitivities (ns+1)^2, mixture scalars
 // {rho, cp, dcp/dT, M} and species cp and h. One workgroup per state. The sensitivities are staged in LDS with coalesced
-// loads; the energy row's inner products run serially in the reference's summation order, thread t for columns t,
-// t+256, ...; the species rows are elementwise in the order of the output. (One wave per state, each lane reading
-// and writing its columns in memory, was bound by uncoalesced access: 1,200 isochoric states of 53 species
-// 73 us, the whole call with rates and sensitivities 268; now 114, this kernel and the sensitivities' gather from LDS.)
+// loads; the energy row's inner products run serially in the reference's summation order, a thread per column; the
+// species rows are elementwise in the order of the output. (One wave per state, each lane reading and writing its columns
+// in memory, was bound by uncoalesced access: 1,200 isochoric states of 53 species 73 us, the whole call with rates and
+// sensitivities 268; now 105, this kernel and the sensitivities' gather from LDS.)
 //
 // thermo_getters_kernel evaluates the getters of griffon.pyx:684-758 for one (T, y): mixture molecular weight, mole
 // fractions, ideal-gas density and pressure, cp/cv/h/e of the mixture and of the species, and dcp/dT of the species
@@ -35,13 +35,24 @@ __device__ inline double dotp(int n, const double *a, const double *b) {
 
 constexpr int kExtThreads = 256;
 
+// Threads of a state: a Jacobian's elementwise parts use 256, but not of a small mechanism, and a right-hand side has
+// little to do beyond its serial sums. Whole calls with 64 / 128 / 256 threads, 20,000 isochoric states (us):
+//   species            10                24                30                   53
+//   Jacobian     310 / 320 / 343   453 / 448 / 474   658 / 632 / 657   1,458 / 1,227 / 1,111
+//   RHS           97 / 102 / 114   146 / 151 / 165   150 / 156 / 170       200 / 203 / 218
+// 1,200 states of 53: 121 / 110 / 105 and 26.3 / 25.5 / 25.7.
+int ext_threads(int ns, bool jac) {
+  if (jac) return ns <= 24 ? 128 : kExtThreads;
+  return ns <= 32 ? 64 : 128;
+}
+
 template <bool ISOCHORIC>
 __global__ void __launch_bounds__(kExtThreads) reactor_ext_kernel(MechView mv, ReactorExtIO a) {
   const int ns = mv.ns, nm = ns - 1;
   const int np = ns + 1;                   // columns of the primitive Jacobian (rho, T, Y_0..Y_{ns-2})
   const int n = ISOCHORIC ? ns + 1 : ns;   // equations
   const long s = blockIdx.x;
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, NT = blockDim.x;
   __shared__ double y[NS_MAX], ue[NS_MAX], cvi[NS_MAX], w[NS_MAX], uin[NS_MAX], yin[NS_MAX], extra[8], er[NS_MAX + 1];
   extern __shared__ double sl[];  // with a Jacobian: sensitivities, column-major with stride ld (odd: spreads the banks)
   const int ld = np | 1;
@@ -54,7 +65,7 @@ __global__ void __launch_bounds__(kExtThreads) reactor_ext_kernel(MechView mv, R
   const double Ru = mv.Ru;
   if (a.jac) {
     const double *ws = a.sens + s * (long)np * np;
-    for (int e = t; e < np * np; e += kExtThreads) sl[e / np * ld + e % np] = ws[e];
+    for (int e = t; e < np * np; e += NT) sl[e / np * ld + e % np] = ws[e];
   }
   if (t < nm) y[t] = ystate[t];
   if (t < ns) {
@@ -73,7 +84,7 @@ __global__ void __launch_bounds__(kExtThreads) reactor_ext_kernel(MechView mv, R
     }
   }
   __syncthreads();
-  if (t == 64) {  // y_{ns-1} = 1 - sum of the others, in extract_y's order (combustion_kernels.h:526-530)
+  if (t == (NT > 64 ? 64 : 0)) {  // y_{ns-1} = 1 - sum of the others, in extract_y's order (combustion_kernels.h:526-530)
     double last = 1.;
     for (int j = 0; j < nm; ++j) last -= y[j];
     y[nm] = last;
@@ -111,7 +122,7 @@ __global__ void __launch_bounds__(kExtThreads) reactor_ext_kernel(MechView mv, R
   if (a.rhs) {
     double *out = a.rhs + s * n;
     const int e0 = ISOCHORIC ? 1 : 0;  // energy equation index
-    for (int i = t; i < n; i += kExtThreads) {
+    for (int i = t; i < n; i += NT) {
       double v;
       if (ISOCHORIC && i == 0) {
         v = 0. + (a.open ? m_rho : 0.);
@@ -143,7 +154,7 @@ __global__ void __launch_bounds__(kExtThreads) reactor_ext_kernel(MechView mv, R
 
   if (!ISOCHORIC) {
     // primitive Jacobian n x (n+1) column-major (isobaric_reactor_kernels.cpp:58-168), then the transform
-    for (int c = t; c < np; c += kExtThreads) {
+    for (int c = t; c < np; c += NT) {
       const double *wc = sl + c * ld;
       double v;
       if (c == 0) {
@@ -162,12 +173,12 @@ __global__ void __launch_bounds__(kExtThreads) reactor_ext_kernel(MechView mv, R
       }
       pj[c * ns] = a.heat == 1 ? 0. : v;
     }
-    for (int e = t; e < np * nm; e += kExtThreads) pj[e / nm * ns + 1 + e % nm] = species(e / nm, e % nm);
+    for (int e = t; e < np * nm; e += NT) pj[e / nm * ns + 1 + e % nm] = species(e / nm, e % nm);
     __syncthreads();
     // (rho, T, Y) -> (T, Y) at constant pressure (isobaric_reactor_kernels.cpp:319-343)
     double *J = a.jac + s * (long)ns * ns;
     const double roT = rho / T, nrm = -rho * mmw;
-    for (int e = t; e < ns * ns; e += kExtThreads) {
+    for (int e = t; e < ns * ns; e += NT) {
       const int c = e / ns, i = e - c * ns;
       J[e] = (c == 0) ? pj[ns + i] - roT * pj[i] : pj[(1 + c) * ns + i] + nrm * mv.dinvm[c - 1] * pj[i];
     }
@@ -175,7 +186,7 @@ __global__ void __launch_bounds__(kExtThreads) reactor_ext_kernel(MechView mv, R
   }
 
   // isochoric: (ns+1) x (ns+1) column-major in (rho, T, Y) (isochoric_reactor_kernels.cpp:60-333)
-  for (int c = t; c < np; c += kExtThreads) {
+  for (int c = t; c < np; c += NT) {
     const double *wc = sl + c * ld;
     double v;
     if (c == 0) {
@@ -196,7 +207,7 @@ __global__ void __launch_bounds__(kExtThreads) reactor_ext_kernel(MechView mv, R
   }
   __syncthreads();
   double *J = a.jac + s * (long)np * np;
-  for (int e = t; e < np * np; e += kExtThreads) {
+  for (int e = t; e < np * np; e += NT) {
     const int c = e / np, i = e - c * np;
     J[e] = i == 0 ? (c == 0 && a.open ? -it : 0.) : i == 1 ? er[c] : species(c, i - 2);
   }
@@ -275,7 +286,7 @@ int launch_reactor_ext(const gf_mech *m, const ReactorExtIO &a, hipStream_t st) 
   auto kern = a.isochoric ? reactor_ext_kernel<true> : reactor_ext_kernel<false>;
   if (lds > 60000 && hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return fail(GF_ERR_UNSUPPORTED, "mechanism needs more LDS per workgroup than the device allows");
-  hipLaunchKernelGGL(kern, dim3((unsigned)a.n), dim3(kExtThreads), lds, st, m->view, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)a.n), dim3(ext_threads(m->view.ns, a.jac)), lds, st, m->view, a);
   if (hipGetLastError() != hipSuccess) return fail(GF_ERR_HIP, "reactor kernel launch failed");
   return GF_OK;
 }
