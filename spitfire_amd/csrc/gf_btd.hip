@@ -42,6 +42,12 @@ __device__ __forceinline__ bool extreme(double f) {
   return e - ((unsigned)(1023 - range) << 20) > ((unsigned)(2 * range) << 20);
 }
 
+// x / u with id the rounded 1 / u: the rounded quotient, unless out of range
+__device__ __forceinline__ double quotient(double x, double u, double id) {
+  const double q = x * id;
+  return fma(fma(-u, q, x), id, q);
+}
+
 // A block in LDS, [column][row], factored by a workgroup step by step as LAPACK's dgetf2 does: nothing but the rows and columns
 // beyond a pivot is touched, so an infinity goes no further than there, and a pivot of zero leaves its column as it is.
 __device__ void plain_lu(double (*A)[64], int *piv, int bs, int t) {
@@ -145,12 +151,14 @@ __device__ void plain_inverse(const double (*A)[64], const int *piv, int bs, int
 // What bounds it is the chain of pivots, blocks after blocks: the wave with column j searches it, publishes the
 // multipliers in LDS, and one barrier later all waves update their columns. The next column's owner does that column first
 // and searches it before its other ones. The back substitution of the inverse needs no barrier: every wave has the
-// columns of U that it wants from LDS, scaled by the reciprocal pivots (so the inverse's rows are scaled once at the end,
-// instead of a division for every entry). The next block's values are loaded while a block is factored. Before, a block in
-// LDS took four barriers a pivot, two more and a division for the substitutions. About 1,000 cycles a pivot now: the two LDS words, the update,
-// search and reciprocal of one column and the way back, one after the other. Measured before and after (us): one
-// system of 60 blocks of 53 10,450 -> 2,260, 24 of 30..61 9,960 -> 2,160, 2,000 of 2..4 1,840 -> 690; 24 of 24x24 blocks
-// 2,850 -> 805, of 10x10 1,050 -> 346. Putting a searching wave's other columns off behind the next barrier gained nothing.
+// columns of U that it wants from LDS, divided by their pivots, so the inverse's rows are divided once at the end instead of
+// every entry in its turn. (Errors of L blocks against long double, 60 systems of three diagonally dominant blocks: of 12 / 24 /
+// 37 / 53 unknowns 0.99 / 0.99 / 1.00 / 1.00 of those with a division for every entry; with products with rounded
+// reciprocals 1.06 / 1.00 / 1.01 / 1.01.) The next block's values are loaded while a block is factored. Before, a block in
+// LDS took four barriers a pivot, two more and a division for the substitutions. About 1,000 cycles a pivot now: the two LDS
+// words, the update, search and reciprocal of one column and the way back, one after the other. Measured before and after
+// (us): one system of 60 blocks of 53 10,140 -> 2,290, 24 of 30..60 9,620 -> 2,180, 1,500 of 2..11 4,070 -> 1,400; 24 of 24x24
+// blocks 2,600 -> 790, of 10x10 920 -> 330. Putting a searching wave's other columns off behind the next barrier gained nothing.
 // Finished rows are updated along with the others, with a multiplier of zero, and U is scaled by reciprocals: where a block has
 // infinities, NaN or a pivot outside 2^-300 .. 2^300 (a singular one among them), that is not what LAPACK's order of operations
 // gives. Such a block is found when it is done, before it is stored; from there on the system is factored in LDS by plain_lu and
@@ -160,7 +168,8 @@ __global__ void __launch_bounds__(64 * kLuWaves) __attribute__((amdgpu_waves_per
 btd_factor_kernel(const int *nblocks, int bs, double *values, const long *voff, double *lout, const long *loff, int *piv,
                   const long *poff) {
   __shared__ double A[8 * C][64], gb[2][64];  // columns of U for the substitution, [column][lane]; what a step publishes, by
-  __shared__ int pb[2];                       // parity of the step
+  __shared__ double diagonal[64];             // parity of the step; of U, by lane
+  __shared__ int pb[2];
   __shared__ int odd[2], plain_piv[64];       // by parity of the block: whether it has to be factored plainly
   const int sys = blockIdx.x;
   const int lane = threadIdx.x & 63;
@@ -277,15 +286,18 @@ btd_factor_kernel(const int *nblocks, int bs, double *values, const long *voff, 
     // the loop take more than the 80 registers of three workgroups per compute unit: 1,500 chains of 2..11 of 53 1,410 -> 1,510 us.)
     if (C == 7 || i + 1 < nb) eliminate(std::true_type{});
     else eliminate(std::false_type{});
-    double za = 0., zx = 0.;  // NaN where an entry is not finite
+    double za = 0., zx = 0., own = 0.;  // NaN where an entry is not finite; the diagonal of U if this wave has it
 #pragma unroll
     for (int k = 0; k < C; ++k) {
       za = fma(a[k], 0., za);
       zx = fma(x[k], 0., zx);
       // (the reciprocal is its row's; rows at and below the diagonal have no part in the substitution)
-      const double id = lane_value(idl, __builtin_amdgcn_readlane(row_of, 8 * k + w));
-      A[8 * k + w][lane] = cur < 8 * k + w ? a[k] * id : 0.;
+      const int r = __builtin_amdgcn_readlane(row_of, 8 * k + w);
+      const double q = quotient(a[k], lane_value(a[k], r), lane_value(idl, r));
+      A[8 * k + w][lane] = cur < 8 * k + w ? q : 0.;
+      own = cur == 8 * k + w ? a[k] : own;
     }
+    if (act && (cur & 7) == w) diagonal[lane] = own;
     if (__any((act && extreme<300>(idl)) || za + zx != 0.)) odd[i & 1] = 1;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(odd[i & 1])) {
@@ -305,11 +317,11 @@ btd_factor_kernel(const int *nblocks, int bs, double *values, const long *voff, 
 #pragma unroll
       for (int c = 0; c < C; ++c) update(x[c]);
     }
-    const double subr = __shfl(subv, cur, 64);
+    const double subr = __shfl(subv, cur, 64), u = diagonal[lane];
 #pragma unroll
     for (int k = 0; k < C; ++k) {
       const int c = 8 * k + w;
-      const double lx = x[k] * idl * subr;
+      const double lx = quotient(x[k], u, idl) * subr;
       if (act && c < bs) L[(i + 1) * nb2 + c * bs + cur] = lx;
       const double up = lane_value(supv, min(c, 63));
       a[k] = act && c < bs ? fma(-up, lx, __shfl(v[k], cur, 64)) : 0.;
@@ -431,8 +443,7 @@ btd_solve_kernel(const int *nblocks, int bs, const double *factors, const long *
     for (int j = 0; j < NC; ++j) r = fma(-column(of, j, ln > j), lane_value(r, j), r);
 #pragma unroll
     for (int j = NC - 1; j >= 0; --j) {
-      double q = r * v;
-      q = fma(fma(-u, q, r), v, q);
+      const double q = quotient(r, u, v);
       r = ln == j ? q : r;
       r = fma(-column(of, j, ln < j), lane_value(q, j), r);
     }

@@ -25,7 +25,7 @@
 // What bounds it is latency, with few wavefronts: the Jacobian kernel's state (28 KB of LDS a state, 256 registers) leaves room
 // for eight waves per compute unit, the rates' registers for twelve (held to 168: at 186 they were eight and
 // 100,003 states took 1,033 us instead of 803). The Jacobian's are held to 256: with six more, small mechanisms, whose LDS has
-// room for two workgroups of 256 threads, had one of them (4,000 states of 10 species 73 us instead of 56). The states of
+// room for two workgroups of 256 threads, had one of them (4,000 states of 10 species 73 us instead of 48). The states of
 // a group are interleaved in LDS, so that neighbouring lanes read
 // neighbouring words, and a reaction's record is read whole, its short lists unrolled with factors of one beyond their
 // ends: field by field, with loops of one to four trips around dependent loads, P1 took 41,000 cycles for a group

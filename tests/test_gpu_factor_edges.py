@@ -455,3 +455,31 @@ def test_inverse_solve_of_few_and_many_systems_is_bitwise_the_same(bs, precision
         assert torch.equal(x, in_place)
         got.append(x.cpu().numpy().reshape(copies, -1))
     assert np.isfinite(got[0]).all() and (got[1] == got[0]).all()
+
+
+def test_lapack_l_blocks_have_one_rounding_an_operation():
+    """L_1 = diag(sub) D_0^{-1} of upper triangular 2x2 blocks: 1/u and a product on the diagonal, two divisions and a product off it,
+    and no further roundings (reciprocals in place of divisions would have two more). Tolerance: two and three half units in
+    the last place against long double, and their squares."""
+    import torch
+    from spitfire_amd import _native
+    n = 4000
+    rng = np.random.default_rng(4)
+    u0, u1, r, s0, s1 = rng.uniform(1., 2., (5, n)) * 2. ** rng.integers(-3, 4, (5, n))
+    zero, one = np.zeros(n), np.ones(n)
+    dev = torch.device('cuda:0')
+    # blocks column by column, then the sub- and super-diagonals
+    V = torch.tensor(np.stack([u0, zero, r, u1, one, zero, zero, one, s0, s1, zero, zero], axis=1).ravel(), device=dev)
+    nb = torch.full((n,), 2, dtype=torch.int32, device=dev)
+    vo, lo, po = (torch.arange(n, dtype=torch.int64, device=dev) * k for k in (12, 8, 4))
+    L = torch.zeros(8 * n, dtype=torch.float64, device=dev)
+    P = torch.zeros(4 * n, dtype=torch.int32, device=dev)
+    _native.check(_native.lib().gf_batch_btddod_full_factorize(n, nb.data_ptr(), 2, V.data_ptr(), vo.data_ptr(), L.data_ptr(),
+                                                               lo.data_ptr(), P.data_ptr(), po.data_ptr(),
+                                                               torch.cuda.current_stream().cuda_stream))
+    l = L.cpu().numpy().reshape(n, 2, 2, 2)[:, 1].transpose(0, 2, 1).astype(np.longdouble)
+    u0, u1, r, s0, s1 = (a.astype(np.longdouble) for a in (u0, u1, r, s0, s1))
+    half = 2. ** -53 * (1. + 1e-6)
+    assert (l[:, 1, 0] == 0).all()
+    for got, ref, k in ((l[:, 0, 0], s0 / u0, 2), (l[:, 1, 1], s1 / u1, 2), (l[:, 0, 1], -s0 * r / u1 / u0, 3)):
+        assert np.max(np.abs((got - ref) / ref)) <= k * half
