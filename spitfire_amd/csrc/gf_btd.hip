@@ -1,22 +1,19 @@
-// Batched block-tridiagonal factor/solve with diagonal off-diagonal blocks (griffon's BTDDOD format), with
-// FP64 factors (in place, as the reference) or FP32 factors in separate arrays (the mixed-precision path of
-// the flamelet solvers: FP32 block LU, FP64 right-hand sides, solutions and residuals).
+// Batched block-tridiagonal factor/solve with diagonal off-diagonal blocks (griffon's BTDDOD format), in two forms.
 //
-// Algorithm restated from btddod_matrix_kernels.cpp:19-119 (block Thomas):
+// As the reference has it, restated from btddod_matrix_kernels.cpp:19-119 (block Thomas):
 //   D_0 = LU(D_0);  for i >= 1:  L_i = diag(sub_{i-1}) D_{i-1}^{-1},  D_i -= L_i diag(sup_{i-1}),  D_i = LU(D_i)
 //   forward  y_0 = b_0,  y_i = b_i - L_i y_{i-1};   backward  x_{n-1} = D^{-1} y,  x_i = D_i^{-1}(y_i - sup_i * x_{i+1})
 // with LAPACK dgetrf/dgetrs semantics for each dense block (partial pivoting, first maximum, 1-based pivots,
-// factors stored in place in the values array, column-major blocks).
+// factors stored in place in the values array, column-major blocks, FP64). btd_factor_kernel: one workgroup of eight waves per
+// system, a block and its inverse in registers, lane = row. btd_solve_kernel: a wave that runs the chain and one that prepares the
+// next block. Blocks that are singular or hold infinities or NaN go through a plain form of the same operations.
 //
-// Factorization: one workgroup per system, the factored diagonal block and the L block live in LDS
-// (2 x bs^2 values); right-looking LU with a wave-reduced pivot search; D^{-1} by column-parallel
-// forward/back substitution on the identity. Solve: one wave per system, lane = row, each block staged in LDS
-// by one coalesced load, register-resident vectors, shuffles broadcast the pivot/substitution values.
-//
-// The batched flamelet solver uses a throughput form of the same recurrence (btd_inv_*): each chain is
+// The batched flamelet and reactor solvers use a throughput form of the same recurrence: each chain is
 // eliminated from both ends at once (twisted factorisation, halving the serial chain), every Schur-updated
-// diagonal block is inverted by blocked Gauss-Jordan elimination with partial pivoting on the matrix cores (gf_twist.hip)
-// and stored as its inverse, so no L blocks are stored and both sweeps of a solve are matrix-vector products.
+// diagonal block is inverted by Gauss-Jordan elimination with partial pivoting (gf_twist.hip on the matrix cores,
+// gf_twist_small.hip one wave per chain) and stored as its inverse, in FP64 or FP32, so no L blocks are stored and both sweeps of a
+// solve are matrix-vector products. Their solves: btd_twist_solve_kernel, four waves per chain; btd_wave_solve_kernel, one;
+// btd_chain_solve_kernel and btd_middle_solve_kernel, a compute unit per chain. All three give bitwise the same.
 #include "gf_btd_index.h"
 #include "gf_internal.h"
 #include "gf_wave.h"

@@ -84,10 +84,12 @@ __device__ __forceinline__ int pivot_of(unsigned scanned, unsigned key, T f, uns
   return __builtin_ctzll(hit);
 }
 
-// One chain's LDS. Rows and columns are padded to Np = 8 ceil(N / 8) by an identity, so that every panel is full: the
-// padding's pivots are its own ones. Two more arrays are in dynamic LDS: M, the block before each panel's update, a row as
-// [lane group][tile][register] (the pivot rows are read from it), and V, the values of the chain's next block, column-major
-// with one row and one column of zeros, which stand for the padding.
+// One chain's LDS. Panels and tiles are whole ones: pivots go up to Np = 8 ceil(N / 8), rows and columns to 16 NT. What the rows
+// and columns beyond the block hold is arbitrary (V has no entries for them: a row beyond reads the next column's, a column
+// beyond words that nothing has written), and never gets into the block: rows beyond are not searched and are never pivots, the
+// steps beyond N have multipliers and pivot rows of zero, and an MFMA's output depends on its own row and column only.
+// Two more arrays are in dynamic LDS: M, the block before each panel's update, a row as
+// [lane group][tile][register] (the pivot rows are read from it), and V, the values of the chain's next block, column-major.
 template <typename T, int NT>
 struct ChainLds {
   static constexpr int R = 16 * NT;
@@ -101,7 +103,7 @@ struct ChainLds {
   double rs[R];            // its row scales
   T sig[R];                // scale of each row: the reciprocal of its pivot
   alignas(16) int prow[R];  // pivot row of each column
-  int rowid[R];            // the row and the column of the inverse that a row and a column hold, N for padding
+  int rowid[R];            // the row and the column of the inverse that a row and a column hold, N for those beyond it
   alignas(16) int colid[4][CS + 2];
   static __host__ __device__ constexpr int m_words(int np) { return (np + 1) * MS; }  // a row more, for those beyond
   static __host__ __device__ constexpr int v_words(int n) { return (n + 1) * n + 1; }
@@ -113,7 +115,7 @@ struct ChainLds {
 // search of the next pivot is a chain of dependent lane shifts, so a step updates the next pivot's column first
 // and then does one lane shift, one step of the next reciprocal and one of the other columns at a time, in an
 // order that the compiler's scheduler (which otherwise runs the chains one after the other) has to keep.
-// The padding is not pivoted. Returns the pivot column of the lane's row.
+// Columns beyond the block (left <= j) are not pivoted. Returns the pivot column of the lane's row.
 template <bool PART, typename T>
 __device__ __forceinline__ void panel_pivots(T (&f)[8], T (&g)[8], unsigned &mask, T &sig, int &rj, int left, int lane) {
   unsigned key = key_of(f[0], mask), most = key;

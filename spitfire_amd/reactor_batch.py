@@ -6,8 +6,8 @@ methods.py:441-612; frozen-Jacobian Newton, nonlinear.py:185-268, tolerance 1e-1
 PI control, stepcontrol.py:50-117; a Jacobian setup every step; negative entries clipped after every step),
 run for all reactors in lock step. Each reactor keeps its own time, step size, Newton convergence and clipping.
 The chemistry (RHS, Jacobian) runs in the batched HIP kernel; every dt*gamma*J - I is inverted by the batched
-register-resident Gauss-Jordan kernel (partial pivoting, one block per system) and each Newton solve is a
-matrix-vector product with that inverse.
+Gauss-Jordan elimination of the block-tridiagonal inverse form (partial pivoting, one block per system) and each Newton
+solve is a matrix-vector product with that inverse.
 
 Loss: L = integral over [0, t_end] of qdot = -sum_k h_k w_k (= rho cp dT/dt for a closed adiabatic isobaric
 reactor, isobaric_reactor_kernels.cpp:23), discretised by the Runge-Kutta weights of each step, i.e. as an
@@ -34,9 +34,9 @@ from .time_integration import KennedyCarpenterS6P4Q3, SimpleNewtonSolver
 
 
 class _BatchedLU:
-    """Solves with R independent ns x ns column-major blocks: each block inverted once per factor() by the
-    blocked Gauss-Jordan kernel with partial pivoting (the one-block case of the batched block-tridiagonal inverse
-    form), each solve one matrix-vector product with the stored FP64 inverse."""
+    """Solves with R independent ns x ns column-major blocks: each block inverted once per factor() by Gauss-Jordan
+    elimination with partial pivoting (the one-block case of the batched block-tridiagonal inverse form), each solve one
+    matrix-vector product with the stored FP64 inverse."""
 
     def __init__(self, R, ns, device):
         import torch
