@@ -357,7 +357,7 @@ btd_factor_kernel(const int *nblocks, int bs, double *values, const long *voff, 
 // 2^-300 .. 2^300 and the quotient within 2^-600 .. 2^600 or zero; a block with anything else (a singular one, infinities, NaN) is
 // solved again with divisions, each row touched only by the columns that it has.
 // One wave per SIMD is enough for a chain, but not the most: small blocks need few registers, and batches of many small systems
-// want the other waves (4,000 single blocks of 10 / 20 10 / 15 us, with one wave 20 / 25, 1,500 chains of 2..11 of 10 33 and 49).
+// want the other waves (4,000 single blocks of 10 / 20 11 / 16 us, with one wave 20 / 25, 1,500 chains of 2..11 of 10 33 and 49).
 template <int NC>
 __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1)))
 btd_solve_kernel(const int *nblocks, int bs, const double *factors, const long *voff, const double *lval, const long *loff,

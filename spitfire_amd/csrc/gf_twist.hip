@@ -36,7 +36,7 @@
 //   256 chains of 62..254       4,807 -> 2,386   3,547 -> 1,818
 //   512 chains                  6,455 -> 4,580   4,546 -> 3,520
 //   1,024 chains               11,555 -> 8,046   8,106 -> 6,184
-//   1,024 / 4,000 blocks       53 / 238 -> 50 / 199   45 / 155 -> 42 / 173
+//   1,024 single blocks            53 ->    50      45 ->    42  (more of them: many_singles)
 // (The panel's multipliers instead of the u_j, H = -A_rK A_PK^{-1}, save the substitution, 1,026 us for the chain, but round
 // differently.)
 #include "gf_internal.h"
